@@ -37,6 +37,8 @@ EXPORTED_SYMBOLS = (
     "arctic_sum_lstm_embedded",
     "arctic_gather_rows",
     "arctic_argmax_clamp",
+    "arctic_argmax_clamp_split",
+    "arctic_argmax_workspace_bytes",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -114,6 +116,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.arctic_gather_rows.restype = i32
     lib.arctic_argmax_clamp.argtypes = [vp, vp, i64, i32, i64, i64, i32, vp]
     lib.arctic_argmax_clamp.restype = i32
+    lib.arctic_argmax_clamp_split.argtypes = [vp, vp, i64, i32, i64, i64, i32, vp, i64, vp]
+    lib.arctic_argmax_clamp_split.restype = i32
+    lib.arctic_argmax_workspace_bytes.argtypes = [i64, i32, i32]
+    lib.arctic_argmax_workspace_bytes.restype = i64
 
 
 def load() -> ctypes.CDLL:

@@ -5,14 +5,16 @@
 // (arctic_inference/vllm/spec_dec/arctic_speculator.py:846-848, 862), with torch's rules for the winner:
 // the largest value, the lowest index among equal values, and a NaN beats every number (the first NaN wins).
 //
-// One workgroup per row; a lane walks 16-byte chunks of the row with streaming loads and keeps its own
-// (value, index) winner; winners are merged inside the wave with lane exchanges and across the waves
-// through LDS.
+// A workgroup walks a row, or a segment of one, in 16-byte chunks with streaming loads; every lane keeps its own
+// (value, index) winner; winners are merged inside the wave with lane exchanges, across the waves through LDS and,
+// where a row is split over several workgroups, across those through a workspace (merge_segments below).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
+#include <random>
 
 #include "common.hpp"
 
@@ -33,30 +35,32 @@ __device__ __forceinline__ uint64_t winner_key(float value, int index) {
 }
 __device__ __forceinline__ int winner_index(uint64_t key) { return key ? (int)~(uint32_t)key : -1; }
 
-// The wave's winner in every lane.  Inside each row of 16 lanes the candidates meet through DPP lane exchanges
-// (vector-ALU moves, no LDS round trip): partners at distance 1 and 2 inside a quad, then the mirrored half and the
-// mirrored row, after which all 16 lanes of a row agree; the four row winners are read with v_readlane.
-template <int kCtrl>
-__device__ __forceinline__ uint64_t meet(uint64_t k) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)k, kCtrl, 0xf, 0xf, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(k >> 32), kCtrl, 0xf, 0xf, true);
-  const uint64_t other = ((uint64_t)hi << 32) | lo;
-  return other > k ? other : k;
+// The wave's winner in every lane, in two 32-bit passes: the largest upper half, then the largest lower half among the
+// candidates that have it.  A step of a pass is one v_max_u32 with a DPP operand (the 64-bit maximum it stands for
+// takes two moves, a compare and two selects): partners at distance 1 and 2 inside a quad, then the mirrored half and
+// the mirrored row of 16 lanes, then the row in front and the two rows in front broadcast into the next ones, which
+// leaves the wave's maximum in lane 63.  kRows = 1: only lanes 0 ... 15 hold candidates.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t max_dpp(uint32_t v) {
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRowMask, 0xf, kRowMask == 0xf));
 }
-
+template <int kRows>
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max_dpp<0xB1, 0xf>(v);    // quad_perm [1,0,3,2]
+  v = max_dpp<0x4E, 0xf>(v);    // quad_perm [2,3,0,1]
+  v = max_dpp<0x141, 0xf>(v);   // row_half_mirror
+  v = max_dpp<0x140, 0xf>(v);   // row_mirror
+  if constexpr (kRows == 1) return (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+  v = max_dpp<0x142, 0xa>(v);   // row_bcast15 into rows 1 and 3
+  v = max_dpp<0x143, 0xc>(v);   // row_bcast31 into rows 2 and 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+template <int kRows = 4>
 __device__ __forceinline__ uint64_t wave_winner(uint64_t k) {
-  k = meet<0xB1>(k);   // quad_perm [1,0,3,2]
-  k = meet<0x4E>(k);   // quad_perm [2,3,0,1]
-  k = meet<0x141>(k);  // row_half_mirror
-  k = meet<0x140>(k);  // row_mirror
-  uint64_t r = 0;
-#pragma unroll
-  for (int lane = 0; lane < 64; lane += 16) {
-    const uint64_t row = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(k >> 32), lane) << 32) |
-                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, lane);
-    r = row > r ? row : r;
-  }
-  return r;
+  const uint32_t value = (uint32_t)(k >> 32);
+  const uint32_t top = wave_max<kRows>(value);
+  const uint32_t index = wave_max<kRows>(value == top ? (uint32_t)k : 0u);
+  return ((uint64_t)top << 32) | index;
 }
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -110,11 +114,10 @@ struct HalfElem {
 // asked for batch k before any wave asks for batch k + 1 (a CU serves its oldest wave first: without the barrier the
 // oldest wave runs through all its batches before the youngest gets its first one in).
 // kHead: rows may start between two 16-byte boundaries (without it the host has checked that none does).
-template <typename Elem, bool kVec, int kUnroll = 4, bool kLockstep = false, bool kHead = false>
-__global__ __launch_bounds__(1024) void row_argmax_kernel(int64_t *__restrict__ out, const char *__restrict__ in,
-                                                          int64_t row_stride_bytes, int cols, int64_t max_index) {
+// Returns the winner of the `cols` elements at `row` as a key whose index counts from `first`, in every lane of wave 0.
+template <typename Elem, bool kVec, int kUnroll, bool kLockstep, bool kHead>
+__device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, int cols, int first) {
   __shared__ uint64_t wave_key[16];
-  const char *row = in + (int64_t)blockIdx.x * row_stride_bytes;
   // Per lane: the largest number seen, the chunk it was first seen in and that chunk's words (a strict ">" keeps the
   // earlier of equal values, the lane's chunk indices only grow); which of the chunk's elements it was is worked out
   // once, after the loop.  Apart from that the first NaN: a chunk's sum is NaN only if the chunk holds a NaN (or
@@ -216,30 +219,143 @@ __global__ __launch_bounds__(1024) void row_argmax_kernel(int64_t *__restrict__ 
     number(v, i);
     if (v != v) nan_at = min(nan_at, i);
   }
-  uint64_t w = nan_at != 0x7fffffff ? winner_key(__builtin_nanf(""), nan_at) : winner_key(best, best_at);
+  uint64_t w = nan_at != 0x7fffffff ? winner_key(__builtin_nanf(""), first + nan_at)
+                                    : winner_key(best, best_at < 0 ? -1 : first + best_at);
 
   w = wave_winner(w);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) wave_key[wave] = w;
   __syncthreads();
-  if (wave == 0) {
-    const int waves = blockDim.x >> 6;
-    uint64_t x = lane < waves ? wave_key[lane] : 0;
-    x = wave_winner(x);
-    if (lane == 0) {
-      const int found = winner_index(x);
-      int64_t idx = found < 0 ? 0 : found;
-      out[blockIdx.x] = idx > max_index ? max_index : idx;
-    }
+  if (wave > 0) return 0;
+  const int waves = blockDim.x >> 6;
+  return wave_winner<1>(lane < waves ? wave_key[lane] : 0);   // at most 16 waves
+}
+
+__device__ __forceinline__ void store_winner(int64_t *out, uint64_t key, int64_t max_index) {
+  const int found = winner_index(key);
+  const int64_t idx = found < 0 ? 0 : found;
+  *out = idx > max_index ? max_index : idx;
+}
+
+template <typename Elem, bool kVec, int kUnroll = 4, bool kLockstep = false, bool kHead = false>
+__global__ __launch_bounds__(1024) void row_argmax_kernel(int64_t *__restrict__ out, const char *__restrict__ in,
+                                                          int64_t row_stride_bytes, int cols, int64_t max_index) {
+  const uint64_t w =
+      find_winner<Elem, kVec, kUnroll, kLockstep, kHead>(in + (int64_t)blockIdx.x * row_stride_bytes, cols, 0);
+  if (threadIdx.x == 0) store_winner(out + blockIdx.x, w, max_index);
+}
+
+// ---- rows split over several workgroups ----------------------------------------------------------------------
+// One workgroup pulls at most about 50 GB/s out of HBM (what a CU keeps outstanding over the latency), 5 us for the
+// 256 KB of a row of 128256 16-bit logits, so a few rows leave the chip idle.  Here each row is cut into `parts`
+// segments of two to four chunks per lane.  Every workgroup leaves its segment's winner in the workspace and then reads
+// the winners of the whole row; a workgroup that finds all of them there merges them and stores the row's answer.
+//
+// The workspace is memory of the call's own with unknown contents: nothing has to be cleared beforehand and nothing is
+// shared between calls.  A winner counts as there when the word beside it is its seal, a bijection of the winner and of
+// a number that no other call has (64 bits from a generator seeded by the system), so what the memory held before
+// passes for a winner with a probability of 2^-64, and a half-written pair does not pass at all.  The workgroups that
+// answer break the row's seals, so that a graph that is replayed, with the same number, starts without any.
+//
+// Some workgroup always finds the row complete: every one waits until its own pair has been stored before it reads,
+// so the one whose pair is stored last sees all of them, unless another has answered already and broken the seals.
+// Several may answer; they store the same value.  No workgroup waits for another.  Stores and loads of the workspace
+// are agent-scope atomics, which go to the memory all XCDs see whatever their L2s hold, so the wait for the stores'
+// acknowledgement is all the order that is needed; a sequentially consistent fence in its place writes back and
+// invalidates the L2 once per workgroup, and those queue up (64 rows of 16 segments: 22.3 us instead of 7.0).
+struct Segment {
+  uint64_t key;
+  uint64_t seal;
+};
+static_assert(sizeof(Segment) == ARCTIC_ARGMAX_SEGMENT_BYTES, "the workspace holds one Segment per workgroup");
+
+__device__ __forceinline__ uint64_t seal_of(uint64_t key, uint64_t call) { return (key * 0x9E3779B97F4A7C15ull) ^ call; }
+__device__ __forceinline__ void share(uint64_t *p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t shared(const uint64_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// By wave 0 of the workgroup, `parts` at most 64.
+__device__ __forceinline__ void merge_segments(int64_t *out, Segment *row, int part, int parts, uint64_t key,
+                                               uint64_t call, int64_t max_index) {
+  const int lane = threadIdx.x;
+  if (lane == 0) {
+    share(&row[part].key, key);
+    share(&row[part].seal, seal_of(key, call));
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the pair is stored (comment above)
+  uint64_t theirs = 0;
+  bool there = true;
+  if (lane < parts) {
+    theirs = shared(&row[lane].key);
+    there = shared(&row[lane].seal) == seal_of(theirs, call);
+  }
+  if (!__all(there)) return;
+  const uint64_t w = wave_winner(theirs);
+  if (lane == 0) store_winner(out, w, max_index);
+  if (lane < parts) share(&row[lane].seal, ~seal_of(theirs, call));
+}
+
+constexpr int kSplitLanes = 512;
+
+template <typename Elem, bool kHead>
+__global__ __launch_bounds__(kSplitLanes) void row_argmax_split_kernel(int64_t *__restrict__ out,
+                                                                       const char *__restrict__ in,
+                                                                       int64_t row_stride_bytes, int cols,
+                                                                       int segment, int parts, uint64_t call,
+                                                                       int64_t max_index, Segment *workspace) {
+  const unsigned row = blockIdx.x / (unsigned)parts;
+  const int part = (int)(blockIdx.x - row * (unsigned)parts);
+  const int first = part * segment;
+  const char *at = in + (int64_t)row * row_stride_bytes + (int64_t)first * (16 / Elem::kPerChunk);
+  const uint64_t w = find_winner<Elem, true, 4, false, kHead>(at, min(segment, cols - first), first);
+  if (threadIdx.x < 64) merge_segments(out + row, workspace + (int64_t)row * parts, part, parts, w, call, max_index);
 }
 
 }  // namespace arctic
 
 using namespace arctic;
 
+// How many workgroups share a row (1: not split), and the elements of each one's segment.  The exchange costs about
+// a microsecond (store, acknowledgement, read), so a row is split when it is long and the rows are few enough that each
+// gets six workgroups or more out of about 512 (two per CU): us per call inside a graph, not split / split,
+//   rows x 128256 bf16:   1 row 6.2 / 3.9,  7 rows 6.7 / 4.4,  32 rows 7.6 / 5.3,  64 rows 7.9 / 6.5,  128 rows 8.6 / 8.7
+//   rows x 50257 bf16:    1 row 3.6 / 3.7,  7 rows 3.9 / 4.2,  64 rows 5.2 / 5.1;    7 rows x 262144: 11.6 / 4.8
+// which cross at about 8000 chunks of 16 bytes per row.  Segments shorter than 1024 chunks and more than 16 of them gain
+// nothing (7 rows x 128256: 32 parts 4.7 us); workgroups of 256 and 1024 lanes are 0.1-0.2 us slower.
+static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
+  constexpr int64_t kMinChunksPerRow = 10240, kMinChunksPerPart = 1024, kMostParts = 16, kFewestParts = 6, kWorkgroups = 512;
+  *segment = cols;
+  const int64_t chunks = dtype == ARCTIC_DTYPE_F32 ? cols / 4 : cols / 8;
+  if (rows <= 0 || chunks < kMinChunksPerRow) return 1;
+  const int64_t parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
+  if (parts < kFewestParts) return 1;
+  *segment = (int)((cols + parts - 1) / parts + 63) & ~63;   // whole 128-byte lines of an aligned row
+  return (cols + *segment - 1) / *segment;
+}
+
+extern "C" int64_t arctic_argmax_workspace_bytes(int64_t rows, int cols, int dtype) {
+  int segment;
+  const int parts = argmax_parts(rows, cols, dtype, &segment);
+  return parts > 1 ? rows * parts * (int64_t)sizeof(Segment) : 0;
+}
+
+// A number per call that no other call has: a 64-bit counter from a seed the system draws, spread by an odd factor.
+static uint64_t call_number() {
+  static std::atomic<uint64_t> next{((uint64_t)std::random_device{}() << 32) ^ std::random_device{}()};
+  return next.fetch_add(1, std::memory_order_relaxed) * 0xD1342543DE82EF95ull;
+}
+
 extern "C" int arctic_argmax_clamp(int64_t *out, const void *logits, int64_t rows, int cols, int64_t row_stride,
                                    int64_t max_index, int dtype, void *stream) {
+  return arctic_argmax_clamp_split(out, logits, rows, cols, row_stride, max_index, dtype, nullptr, 0, stream);
+}
+
+extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64_t rows, int cols, int64_t row_stride,
+                                         int64_t max_index, int dtype, void *workspace, int64_t workspace_bytes,
+                                         void *stream) {
   const char *fn = "argmax_clamp";
   if (dtype != ARCTIC_DTYPE_F32 && dtype != ARCTIC_DTYPE_F16 && dtype != ARCTIC_DTYPE_BF16)
     return fail(ARCTIC_ERR_UNSUPPORTED, "%s: logits must be fp32, fp16 or bf16", fn);
@@ -255,8 +371,31 @@ extern "C" int arctic_argmax_clamp(int64_t *out, const void *logits, int64_t row
   const bool vec = (uintptr_t)logits % es == 0;   // rows may start anywhere between two 16-byte boundaries
   const bool aligned_rows = (uintptr_t)logits % 16 == 0 && (stride_bytes % 16 == 0 || rows == 1);
   const int per_chunk = 16 / es;
-  int threads = (int)std::min<int64_t>(1024, std::max<int64_t>(64, ((cols / per_chunk / 4 + 63) / 64) * 64));
   hipStream_t s = (hipStream_t)stream;
+  int segment;
+  const int parts = argmax_parts(rows, cols, dtype, &segment);
+  if (vec && parts > 1 && workspace) {
+    if ((uintptr_t)workspace % 8 || workspace_bytes < rows * parts * (int64_t)sizeof(Segment))
+      return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: the workspace must be 8-byte aligned and hold %lld bytes", fn,
+                  (long long)(rows * parts * (int64_t)sizeof(Segment)));
+    const uint64_t call = call_number();
+#define ARCTIC_ARGMAX_SPLIT(ELEM, HEAD)                                                                            \
+  hipLaunchKernelGGL((row_argmax_split_kernel<ELEM, HEAD>), dim3((unsigned)(rows * parts)), dim3(kSplitLanes), 0, s, out, \
+                     (const char *)logits, stride_bytes, cols, segment, parts, call, max_index, (Segment *)workspace)
+    if (dtype == ARCTIC_DTYPE_F32) {
+      if (aligned_rows) ARCTIC_ARGMAX_SPLIT(F32Elem, false);
+      else ARCTIC_ARGMAX_SPLIT(F32Elem, true);
+    } else if (dtype == ARCTIC_DTYPE_BF16) {
+      if (aligned_rows) ARCTIC_ARGMAX_SPLIT(HalfElem<BF16>, false);
+      else ARCTIC_ARGMAX_SPLIT(HalfElem<BF16>, true);
+    } else {
+      if (aligned_rows) ARCTIC_ARGMAX_SPLIT(HalfElem<F16>, false);
+      else ARCTIC_ARGMAX_SPLIT(HalfElem<F16>, true);
+    }
+#undef ARCTIC_ARGMAX_SPLIT
+    return check_launch(fn);
+  }
+  int threads = (int)std::min<int64_t>(1024, std::max<int64_t>(64, ((cols / per_chunk / 4 + 63) / 64) * 64));
   const dim3 grid((unsigned)rows), block((unsigned)threads);
   // Launches of about one and a half to three workgroups per CU (the 256 CUs of this GPU; a decode batch of a few
   // hundred rows) keep their waves in step, a chunk at a time: the two workgroups of a CU then finish together with

@@ -398,6 +398,21 @@ int arctic_gather_rows(int num_tensors, const void *const *src, void *const *dst
 int arctic_argmax_clamp(int64_t *out, const void *logits, int64_t rows, int cols,
                         int64_t row_stride, int64_t max_index, int dtype, void *stream);
 
+/*
+ * The same with a workspace of the caller's, which lets a few long rows be split over several workgroups each.
+ *
+ *   workspace        device, 8-byte aligned, of at least arctic_argmax_workspace_bytes(rows, cols, dtype) bytes, which
+ *                    this call alone uses until its kernel has run; its contents do not matter and need not be
+ *                    cleared.  NULL: rows are not split (what arctic_argmax_clamp does).
+ *
+ * arctic_argmax_workspace_bytes returns 0 where splitting would not help; it makes no HIP call.
+ */
+#define ARCTIC_ARGMAX_SEGMENT_BYTES 16
+int64_t arctic_argmax_workspace_bytes(int64_t rows, int cols, int dtype);
+int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64_t rows, int cols,
+                              int64_t row_stride, int64_t max_index, int dtype, void *workspace,
+                              int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

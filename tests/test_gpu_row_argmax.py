@@ -141,3 +141,37 @@ def test_row_counts_around_the_in_step_kernel(ops, rows, dtype):
         got = ops.speculator_argmax(base.to(DEV)[:, :cols], cols)
         want = torch.argmax(base[:, :cols].float(), dim=-1)
         assert torch.equal(got.cpu(), want), f"{rows} x {cols} (+{pad}), {dtype}"
+
+
+@pytest.mark.parametrize("rows,cols,dtype,pad", [
+    (1, 81920, torch.bfloat16, 0), (1, 81919, torch.float16, 0),       # the shortest row that is split, and one below
+    (85, 128257, torch.float16, 0), (86, 128256, torch.bfloat16, 0),   # six workgroups per row, and no longer
+    (5, 131103, torch.bfloat16, 3), (3, 40960, torch.float32, 0), (2, 300001, torch.float32, 1)])
+def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
+    """Long rows of a small batch are cut into segments: ties, NaNs and infinities on both sides of the cuts, rows of one
+    value, and a captured graph whose inputs change between replays (the workspace keeps what the last replay left)."""
+    g = torch.Generator().manual_seed(cols)
+    levels = torch.tensor([-float("inf"), -2.0, -0.0, 0.0, 1.5, 3.0])
+    batches = []
+    for k in range(4):
+        x = levels[torch.randint(0, 4 if k == 1 else 6, (rows, cols + pad), generator=g)].to(dtype)
+        x[0] = -float("inf")
+        if k == 2:
+            for r in range(1, rows):
+                x[r, torch.randint(0, cols, (2,), generator=g)] = float("nan")
+        if k == 3 and rows > 1:
+            x[1] = -7.0
+            x[1, cols - 1] = -6.5
+        batches.append(x)
+    static = torch.empty(rows, cols + pad, dtype=dtype, device=DEV)[:, :cols]
+    static.copy_(batches[0][:, :cols])
+    assert torch.equal(ops.speculator_argmax(static, cols).cpu(), reference(batches[0][:, :cols], cols))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.speculator_argmax(static, cols - 1)
+    assert got.shape == (rows,) and got.is_contiguous()
+    for x in batches + batches[:2]:
+        static.copy_(x[:, :cols])
+        graph.replay()
+        assert torch.equal(got.cpu(), reference(x[:, :cols], cols - 1))
