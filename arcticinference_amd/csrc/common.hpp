@@ -112,16 +112,34 @@ __device__ __forceinline__ void store16_stream(void *p, const uint4 &v) {
   const u32x4 t = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(t, (ARCTIC_GLOBAL u32x4 *)p);
 }
-__device__ __forceinline__ void store16(void *p, const uint4 &v) {  // stays in the caches: read again soon
-  const u32x4 t = {v.x, v.y, v.z, v.w};
-  *(ARCTIC_GLOBAL u32x4 *)p = t;
-}
 __device__ __forceinline__ void store8_stream(void *p, const uint2 &v) {
   const u32x2 t = {v.x, v.y};
   __builtin_nontemporal_store(t, (ARCTIC_GLOBAL u32x2 *)p);
 }
 __device__ __forceinline__ void store4_stream(void *p, uint32_t v) {
   __builtin_nontemporal_store(v, (ARCTIC_GLOBAL uint32_t *)p);
+}
+
+// The same for addresses that are only element-aligned (rows of odd widths or pitches): still one 16-byte access per
+// lane, which the memory pipeline takes at any alignment; a wave's accesses then touch one 128-byte line more.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+template <bool kAnyAlignment>
+__device__ __forceinline__ uint4 load16(const void *p) {
+  if constexpr (!kAnyAlignment) return load16(p);
+  const u32x4 v = *(const ARCTIC_GLOBAL u32x4_any *)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <bool kAnyAlignment>
+__device__ __forceinline__ uint4 load16_stream(const void *p) {
+  if constexpr (!kAnyAlignment) return load16_stream(p);
+  const u32x4 v = __builtin_nontemporal_load((const ARCTIC_GLOBAL u32x4_any *)p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <bool kAnyAlignment>
+__device__ __forceinline__ void store16_stream(void *p, const uint4 &v) {
+  if constexpr (!kAnyAlignment) return store16_stream(p, v);
+  const u32x4_any t = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(t, (ARCTIC_GLOBAL u32x4_any *)p);
 }
 
 // A lane's unit of work on the speculator paths: eight consecutive 16-bit elements
@@ -131,10 +149,12 @@ struct Chunk {
   static constexpr int kBytes = 16;
   uint4 v;
   __device__ static __forceinline__ Chunk zero() { return Chunk{make_uint4(0, 0, 0, 0)}; }
-  __device__ static __forceinline__ Chunk load(const void *p) { return Chunk{load16(p)}; }
-  __device__ static __forceinline__ Chunk load_stream(const void *p) { return Chunk{load16_stream(p)}; }
-  __device__ __forceinline__ void store_stream(void *p) const { store16_stream(p, v); }
-  __device__ __forceinline__ void store(void *p) const { store16(p, v); }
+  template <bool kAnyAlignment = false>
+  __device__ static __forceinline__ Chunk load(const void *p) { return Chunk{load16<kAnyAlignment>(p)}; }
+  template <bool kAnyAlignment = false>
+  __device__ static __forceinline__ Chunk load_stream(const void *p) { return Chunk{load16_stream<kAnyAlignment>(p)}; }
+  template <bool kAnyAlignment = false>
+  __device__ __forceinline__ void store_stream(void *p) const { store16_stream<kAnyAlignment>(p, v); }
   template <typename T>
   __device__ __forceinline__ void unpack(float (&f)[8]) const { unpack8<T>(v, f); }
   template <typename T>

@@ -9,11 +9,11 @@
 // across both RMS reductions, so HBM sees 9*D elements read and 2*D written per
 // row (the reference re-reads the cell gate and reads out_cell back: 12*D).
 // Sums are DPP wave reductions plus an LDS combine.  Three kernels:
-// sum_lstm_staged_kernel (the speculator's shapes, rows of up to 8192 elements
-// with all four vectors: the nine loads are requested in stages, between the
-// stages of the arithmetic, one chunk per lane), sum_lstm_vec_kernel (every
-// other shape with 16-byte accesses: the loads are requested together) and
-// sum_lstm_scalar_kernel (any size and alignment, element by element).
+// sum_lstm_staged_kernel (rows of up to 8192 elements: the nine loads are
+// requested in stages, between the stages of the arithmetic, one chunk per lane),
+// sum_lstm_vec_kernel (rows of up to 16384 elements: two chunks per lane, the
+// loads requested together) and sum_lstm_scalar_kernel (what is left: very short
+// rows that are not 16-byte aligned and more than 16384 elements, element by element).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -49,51 +49,78 @@ struct LstmParams {
   float eps_state;
 };
 
-// Loads are issued in the order in which the arithmetic needs them - cell gate,
-// forget gate, previous cell, input gate, output gate - and memory returns them
-// in that order, so the first row sum, the candidate GELU and the early sigmoids
-// run while the later gates are still on their way, and only one sigmoid, one
-// multiply and the store remain after the last load has landed.
+// A row of any width from 8 elements on is covered by chunks of 8: chunk c starts at element 8 c, the last one at D - 8,
+// so that it ends with the row.  Where the width is no multiple of 8 the last chunk's first elements are the end of the
+// chunk before it: they are computed twice, bit for bit alike, stored twice and counted once.  `repeated` says how many
+// of a chunk's elements do not count: 0, 1 to 7 in such a last chunk, 8 or more for a lane behind the row's end.
+struct Place {
+  uint32_t off;   // bytes from the row's start
+  int repeated;
+  __device__ __forceinline__ Place(int chunk, int D) {
+    const int start = min(chunk * Chunk::kElems, D - Chunk::kElems);
+    off = (uint32_t)start * 2;
+    repeated = chunk * Chunk::kElems - start;
+  }
+  __device__ __forceinline__ bool live() const { return repeated < Chunk::kElems; }
+};
+
+// kFullWaves: rows 16-byte aligned, all four scale / shift vectors given, every lane of every wave owns a chunk of 8
+// elements; kRagged: the same with lanes to spare in the last wave; kAnyRow: everything else - vectors missing, rows
+// only element-aligned (odd widths, pitches or bases; see common.hpp).
+enum RowKind { kFullWaves, kRagged, kAnyRow };
+
 // kSharedZ: `z4` holds ONE gate-wide row per token ([rows, D]) that is added to all four
 // gates, as the speculator's z4 = emb.repeat(1, 1, 4) would; it is then read once, not four times.
-// kEarlyOutputGate: the output gate's sigmoid runs ahead of the second row sum (rows of up to 4096 elements: by
-// then the gate has arrived and the waves would otherwise idle at the barrier); it changes no result bit.
-// A null prev_cell stands for a cell of zeros: the lanes then read the forget gate's address a second time and
-// discard it.
+// A null prev_cell stands for a cell of zeros.  Absent scale / shift vectors stand for 1 / 0, which is exact: the norm
+// is one multiply and one fused multiply-add per element whichever vectors were given.  Every lane then reads the same
+// chunk of ones or zeros below, which leaves the kernels without a branch between a row's requests (one there costs
+// 0.25 us at 512 rows of 4096: requests in front of it are waited for behind it).  kMayMiss: a vector can be absent.
+__constant__ const uint32_t kChunkOfZeros[4] = {0, 0, 0, 0};
+__constant__ const uint32_t kChunkOfOnesF16[4] = {0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u};
+__constant__ const uint32_t kChunkOfOnesBF16[4] = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+template <typename T, bool kMayMiss>
+__device__ __forceinline__ Chunk load_scale(const char *w, uint32_t off) {
+  if constexpr (!kMayMiss) return Chunk::load(w + off);
+  const char *ones = (const char *)(T::kCode == ARCTIC_DTYPE_BF16 ? kChunkOfOnesBF16 : kChunkOfOnesF16);
+  return Chunk::load<true>((w ? w : ones) + (w ? off : 0u));
+}
+template <bool kMayMiss>
+__device__ __forceinline__ Chunk load_shift(const char *b, uint32_t off) {
+  if constexpr (!kMayMiss) return Chunk::load(b + off);
+  return Chunk::load<true>((b ? b : (const char *)kChunkOfZeros) + (b ? off : 0u));
+}
+
+// Rows beyond one chunk per lane of 1024 lanes.  Loads are issued in the order in which the arithmetic needs them -
+// cell gate, forget gate, previous cell, input gate, output gate - and memory returns them in that order, so the first
+// row sum, the candidate GELU and the early sigmoids run while the later gates are still on their way, and only one
+// sigmoid, one multiply and the store remain after the last load has landed.
 template <int K>
 struct LstmRow {
   Chunk sc[K], zc[K], sf[K], zf[K], si[K], zi[K], pc[K], so[K], zo[K];
 };
 
-template <typename T, int kChunksPerThread, bool kFastGelu, int kMaxThreads, bool kSharedZ, bool kEarlyOutputGate>
-__global__ __launch_bounds__(kMaxThreads) void sum_lstm_vec_kernel(const LstmParams p) {
+template <typename T, bool kFastGelu, bool kSharedZ, bool kAnyAlignment>
+__global__ __launch_bounds__(1024) void sum_lstm_vec_kernel(const LstmParams p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
-  constexpr int K = kChunksPerThread;
+  constexpr int K = 2;
   constexpr int E = Chunk::kElems;
   using C = Chunk;
   const int D = p.D;
-  const int chunks = D / E;
   const int64_t gate_bytes = (int64_t)D * 2;
+  const Place at[K] = {Place(threadIdx.x, D), Place(threadIdx.x + blockDim.x, D)};
+  auto load = [](const char *q) { return C::load_stream<kAnyAlignment>(q); };
 
-  bool live[K];
-  int64_t off[K];
   C wc[K], bc[K], ws[K], bs[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int c = threadIdx.x + k * blockDim.x;
-    live[k] = c < chunks;
-    off[k] = (int64_t)(live[k] ? c : 0) * C::kBytes;  // idle lanes re-read chunk 0 and discard it
-  }
   // The scale / shift vectors are the same for every row (cache resident).  They
   // are requested first: memory returns loads in issue order, so asking for them
   // later would park the arithmetic behind the whole row.
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    if (p.w_cell) wc[k] = C::load(p.w_cell + off[k]);
-    if (p.b_cell) bc[k] = C::load(p.b_cell + off[k]);
-    if (p.w_state) ws[k] = C::load(p.w_state + off[k]);
-    if (p.b_state) bs[k] = C::load(p.b_state + off[k]);
+    wc[k] = load_scale<T, true>(p.w_cell, at[k].off);
+    bc[k] = load_shift<true>(p.b_cell, at[k].off);
+    ws[k] = load_scale<T, true>(p.w_state, at[k].off);
+    bs[k] = load_shift<true>(p.b_state, at[k].off);
   }
 
   const int64_t row = blockIdx.x;
@@ -106,69 +133,55 @@ __global__ __launch_bounds__(kMaxThreads) void sum_lstm_vec_kernel(const LstmPar
     const char *pc_row = p.prev_cell ? p.prev_cell + row * p.pc_stride * 2 : s_row;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      r.zc[k] = C::load_stream(z_row + (kSharedZ ? 0 : 3 * gate_bytes) + off[k]);
-      r.sc[k] = C::load_stream(s_row + 3 * gate_bytes + off[k]);
+      r.zc[k] = load(z_row + (kSharedZ ? 0 : 3 * gate_bytes) + at[k].off);
+      r.sc[k] = load(s_row + 3 * gate_bytes + at[k].off);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      r.sf[k] = C::load_stream(s_row + off[k]);
-      r.zf[k] = kSharedZ ? r.zc[k] : C::load_stream(z_row + off[k]);
+      r.sf[k] = load(s_row + at[k].off);
+      r.zf[k] = kSharedZ ? r.zc[k] : load(z_row + at[k].off);
     }
     // (the previous cell and both outputs stream like the gates: a launch boundary writes the outputs back anyway,
     // and streaming stores leave the CU earlier - measured on the staged kernel below)
 #pragma unroll
-    for (int k = 0; k < K; ++k) r.pc[k] = C::load_stream(pc_row + off[k]);
+    for (int k = 0; k < K; ++k) r.pc[k] = load(pc_row + at[k].off);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      r.si[k] = C::load_stream(s_row + gate_bytes + off[k]);
-      r.zi[k] = kSharedZ ? r.zc[k] : C::load_stream(z_row + gate_bytes + off[k]);
+      r.si[k] = load(s_row + gate_bytes + at[k].off);
+      r.zi[k] = kSharedZ ? r.zc[k] : load(z_row + gate_bytes + at[k].off);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      r.so[k] = C::load_stream(s_row + 2 * gate_bytes + off[k]);
-      r.zo[k] = kSharedZ ? r.zc[k] : C::load_stream(z_row + 2 * gate_bytes + off[k]);
+      r.so[k] = load(s_row + 2 * gate_bytes + at[k].off);
+      r.zo[k] = kSharedZ ? r.zc[k] : load(z_row + 2 * gate_bytes + at[k].off);
     }
   }
 
   char *oc_row = p.out_cell + row * p.out_stride * 2;
   char *os_row = p.out_state + row * p.out_stride * 2;
-  // Lanes beyond the row take part in the sums with zeros.  (Each value is
-  // cleared where it is first used, not here: touching pc now would wait for it.)
   // phase 1: pre_c and its sum of squares (reference :65-82); needs the cell gate only
   float cact[K][E];
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     float a[E], b[E];
-    if (!live[k]) r.sc[k] = r.zc[k] = C::zero();
     r.sc[k].template unpack<T>(a);
     r.zc[k].template unpack<T>(b);
 #pragma unroll
     for (int j = 0; j < E; ++j) {
       cact[k][j] = fmaf(p.alpha, b[j], a[j]);
-      ss = fmaf(cact[k][j], cact[k][j], ss);
+      if (j >= at[k].repeated) ss = fmaf(cact[k][j], cact[k][j], ss);
     }
   }
   const float inv_cpre = rsqrtf(block_sum(ss, slots_cpre) * p.inv_D + p.eps_cell);
   // candidate = gelu(rmsnorm(pre_c)): runs while the other gates are still arriving
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    // an absent scale / shift vector acts as 1 / 0 (exact), so the norm is one multiply and
-    // one fused multiply-add per element whichever vectors were given
     float w[E], b[E];
+    wc[k].template unpack<T>(w);
+    bc[k].template unpack<T>(b);
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      w[j] = 1.f;
-      b[j] = 0.f;
-    }
-    if (p.w_cell) wc[k].template unpack<T>(w);
-    if (p.b_cell) bc[k].template unpack<T>(b);
-    const float mask = live[k] ? 1.f : 0.f;  // idle lanes must add nothing to the second sum
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-      const float cn = fmaf(cact[k][j] * inv_cpre, w[j], b[j]);
-      cact[k][j] = gelu<kFastGelu>(cn) * mask;
-    }
+    for (int j = 0; j < E; ++j) cact[k][j] = gelu<kFastGelu>(fmaf(cact[k][j] * inv_cpre, w[j], b[j]));
   }
 
   // phase 2: cell update; write out_cell (reference :104-140)
@@ -179,7 +192,7 @@ __global__ __launch_bounds__(kMaxThreads) void sum_lstm_vec_kernel(const LstmPar
     float a[E], b[E], c[E];
     r.sf[k].template unpack<T>(a);
     r.zf[k].template unpack<T>(b);
-    if (!live[k] || !p.prev_cell) r.pc[k] = C::zero();
+    if (!p.prev_cell) r.pc[k] = C::zero();
     r.pc[k].template unpack<T>(c);
 #pragma unroll
     for (int j = 0; j < E; ++j) cell[k][j] = sigmoid_f(fmaf(p.alpha, b[j], a[j])) * c[j];
@@ -191,23 +204,12 @@ __global__ __launch_bounds__(kMaxThreads) void sum_lstm_vec_kernel(const LstmPar
 #pragma unroll
     for (int j = 0; j < E; ++j) {
       const float cnew = fmaf(cact[k][j], sigmoid_f(fmaf(p.alpha, b[j], a[j])), cell[k][j]);
-      ss = fmaf(cnew, cnew, ss);  // unrounded, as in the reference (:136)
+      if (j >= at[k].repeated) ss = fmaf(cnew, cnew, ss);  // unrounded, as in the reference (:136)
       cell[k][j] = cnew;
     }
     const C packed = C::template pack<T>(cell[k]);
-    if (live[k]) packed.store_stream(oc_row + off[k]);
+    if (at[k].live()) packed.template store_stream<kAnyAlignment>(oc_row + at[k].off);
     packed.template unpack<T>(cell[k]);
-  }
-  float og[K][E];
-  if constexpr (kEarlyOutputGate) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      float a[E], g[E];
-      r.so[k].template unpack<T>(a);
-      r.zo[k].template unpack<T>(g);
-#pragma unroll
-      for (int j = 0; j < E; ++j) og[k][j] = sigmoid_f(fmaf(p.alpha, g[j], a[j]));
-    }
   }
   const float inv_cnew = rsqrtf(block_sum(ss, slots_cnew) * p.inv_D + p.eps_state);
 
@@ -215,32 +217,20 @@ __global__ __launch_bounds__(kMaxThreads) void sum_lstm_vec_kernel(const LstmPar
   // the output gate is the last load to arrive and is consumed last
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    float w[E], b[E], st[E];
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-      w[j] = 1.f;
-      b[j] = 0.f;
-    }
-    if (p.w_state) ws[k].template unpack<T>(w);
-    if (p.b_state) bs[k].template unpack<T>(b);
+    float w[E], b[E], st[E], a[E], g[E];
+    ws[k].template unpack<T>(w);
+    bs[k].template unpack<T>(b);
 #pragma unroll
     for (int j = 0; j < E; ++j) st[j] = gelu<kFastGelu>(fmaf(cell[k][j] * inv_cnew, w[j], b[j]));
-    if constexpr (kEarlyOutputGate) {
+    r.so[k].template unpack<T>(a);
+    r.zo[k].template unpack<T>(g);
 #pragma unroll
-      for (int j = 0; j < E; ++j) st[j] *= og[k][j];
-    } else {
-      float a[E], g[E];
-      r.so[k].template unpack<T>(a);
-      r.zo[k].template unpack<T>(g);
-#pragma unroll
-      for (int j = 0; j < E; ++j) st[j] *= sigmoid_f(fmaf(p.alpha, g[j], a[j]));
-    }
-    if (live[k]) C::template pack<T>(st).store_stream(os_row + off[k]);
+    for (int j = 0; j < E; ++j) st[j] *= sigmoid_f(fmaf(p.alpha, g[j], a[j]));
+    if (at[k].live()) C::template pack<T>(st).template store_stream<kAnyAlignment>(os_row + at[k].off);
   }
 }
 
-// The speculator's shape (every lane owns one 16-byte chunk of the row, all four scale / shift vectors given) with the
-// requests of a row issued in stages.  A CU accepts vector-memory requests only as fast as HBM answers them: a wave
+// Rows of up to 8192 elements, one chunk of 8 per lane, with the requests of a row issued in stages.  A CU accepts vector-memory requests only as fast as HBM answers them: a wave
 // that asks for its nine chunks at once sits in the ninth request for microseconds, long after the first chunks have
 // arrived and with nothing computed, and the younger workgroup of the CU does not get its first request in before
 // the older one's last.  Here a wave requests its chunks in the order cell gate z, s; forget gate s, z; previous
@@ -259,49 +249,48 @@ __global__ __launch_bounds__(kMaxThreads) void sum_lstm_vec_kernel(const LstmPar
 // are read by the next launches of the step, but a launch boundary writes them back anyway, and stores that stream
 // leave earlier).
 //
-// Same arithmetic, operation for operation, as sum_lstm_vec_kernel: results are bit-identical.
-// kMaxLanes: 512 for rows of up to 4096 elements, 1024 (half the registers per lane) for rows of up to 8192.
-// kRagged: the row's chunks do not fill the last wave; the lanes behind the last chunk run along on that chunk (the
-// barriers need every wave), add nothing to the row sums and store nothing.
 // kZeroCell: the previous cell is all zeros (the first step of a proposal round) and is not read.
-template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, int kMaxLanes, bool kRagged>
-__global__ __launch_bounds__(kMaxLanes) void sum_lstm_staged_kernel(const LstmParams p) {
+template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, RowKind kKind>
+__global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParams p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
   constexpr int E = Chunk::kElems;
   using C = Chunk;
   using std::integral_constant;
   const int64_t row = blockIdx.x;
-  const bool active = !kRagged || (int)threadIdx.x < p.D / E;
-  const int64_t off = (int64_t)(kRagged ? min((int)threadIdx.x, p.D / E - 1) : (int)threadIdx.x) * C::kBytes;
+  constexpr bool kAny = kKind == kAnyRow;
+  // the barriers need every wave, so the lanes behind the last chunk run along on it
+  const Place at(threadIdx.x, kKind == kFullWaves ? INT32_MAX : p.D);
+  const uint32_t off = at.off;
+  auto load = [off](const char *q) { return C::load_stream<kAny>(q + off); };
   const int64_t gate_bytes = (int64_t)p.D * 2;
-  const char *s_row = p.states + row * p.s_stride * 2 + off;
+  const char *s_row = p.states + row * p.s_stride * 2;
   int64_t zr = row;
   if (kSharedZ && p.z_index) zr = min(max(p.z_index[row], (int64_t)0), p.z_rows - 1);
-  const char *z_row = p.z4 + zr * p.z_stride * 2 + off;
-  const char *pc_row = kZeroCell ? s_row : p.prev_cell + row * p.pc_stride * 2 + off;
-  char *oc_row = p.out_cell + row * p.out_stride * 2 + off;
-  char *os_row = p.out_state + row * p.out_stride * 2 + off;
+  const char *z_row = p.z4 + zr * p.z_stride * 2;
+  const char *pc_row = kZeroCell ? s_row : p.prev_cell + row * p.pc_stride * 2;
+  char *oc_row = p.out_cell + row * p.out_stride * 2;
+  char *os_row = p.out_state + row * p.out_stride * 2;
 
   C in[9];   // zc sc sf zf pc si zi so zo; with kSharedZ the one z chunk stands for all four, with kZeroCell pc is unused
   // requests chunks kFrom ... kTo - 1 of the list above
   auto request = [&](auto from, auto to) {
     constexpr int kFrom = decltype(from)::value, kTo = decltype(to)::value;
     __builtin_amdgcn_sched_barrier(0);   // neither hoisted above the arithmetic in front nor sunk below what follows
-    if constexpr (kFrom <= 0 && 0 < kTo) in[0] = C::load_stream(z_row + (kSharedZ ? 0 : 3 * gate_bytes));
-    if constexpr (kFrom <= 1 && 1 < kTo) in[1] = C::load_stream(s_row + 3 * gate_bytes);
-    if constexpr (kFrom <= 2 && 2 < kTo) in[2] = C::load_stream(s_row);
-    if constexpr (kFrom <= 3 && 3 < kTo && !kSharedZ) in[3] = C::load_stream(z_row);
-    if constexpr (kFrom <= 4 && 4 < kTo && !kZeroCell) in[4] = C::load_stream(pc_row);
-    if constexpr (kFrom <= 5 && 5 < kTo) in[5] = C::load_stream(s_row + gate_bytes);
-    if constexpr (kFrom <= 6 && 6 < kTo && !kSharedZ) in[6] = C::load_stream(z_row + gate_bytes);
-    if constexpr (kFrom <= 7 && 7 < kTo) in[7] = C::load_stream(s_row + 2 * gate_bytes);
-    if constexpr (kFrom <= 8 && 8 < kTo && !kSharedZ) in[8] = C::load_stream(z_row + 2 * gate_bytes);
+    if constexpr (kFrom <= 0 && 0 < kTo) in[0] = load(z_row + (kSharedZ ? 0 : 3 * gate_bytes));
+    if constexpr (kFrom <= 1 && 1 < kTo) in[1] = load(s_row + 3 * gate_bytes);
+    if constexpr (kFrom <= 2 && 2 < kTo) in[2] = load(s_row);
+    if constexpr (kFrom <= 3 && 3 < kTo && !kSharedZ) in[3] = load(z_row);
+    if constexpr (kFrom <= 4 && 4 < kTo && !kZeroCell) in[4] = load(pc_row);
+    if constexpr (kFrom <= 5 && 5 < kTo) in[5] = load(s_row + gate_bytes);
+    if constexpr (kFrom <= 6 && 6 < kTo && !kSharedZ) in[6] = load(z_row + gate_bytes);
+    if constexpr (kFrom <= 7 && 7 < kTo) in[7] = load(s_row + 2 * gate_bytes);
+    if constexpr (kFrom <= 8 && 8 < kTo && !kSharedZ) in[8] = load(z_row + 2 * gate_bytes);
     __builtin_amdgcn_sched_barrier(0);
   };
   request(integral_constant<int, 0>(), integral_constant<int, 2>());
-  const C wc = C::load(p.w_cell + off);
-  const C bc = C::load(p.b_cell + off);
+  const C wc = load_scale<T, kAny>(p.w_cell, off), bc = load_shift<kAny>(p.b_cell, off);
+  __builtin_amdgcn_sched_barrier(0);
 
   // phase 1: pre_c and its sum of squares (reference :65-82)
   float cact[E], a[E], b[E], c[E];
@@ -311,10 +300,10 @@ __global__ __launch_bounds__(kMaxLanes) void sum_lstm_staged_kernel(const LstmPa
 #pragma unroll
   for (int j = 0; j < E; ++j) {
     cact[j] = fmaf(p.alpha, b[j], a[j]);
-    ss = fmaf(cact[j], cact[j], ss);
+    if (!kAny || j >= at.repeated) ss = fmaf(cact[j], cact[j], ss);
   }
   request(integral_constant<int, 2>(), integral_constant<int, 3>());
-  const float inv_cpre = rsqrtf(block_sum(active ? ss : 0.f, slots_cpre) * p.inv_D + p.eps_cell);
+  const float inv_cpre = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cpre) * p.inv_D + p.eps_cell);
   {
     float w[E], sh[E];
     wc.template unpack<T>(w);
@@ -322,8 +311,7 @@ __global__ __launch_bounds__(kMaxLanes) void sum_lstm_staged_kernel(const LstmPa
 #pragma unroll
     for (int j = 0; j < E; ++j) cact[j] = gelu<kFastGelu>(fmaf(cact[j] * inv_cpre, w[j], sh[j]));
   }
-  const C ws = C::load(p.w_state + off);
-  const C bs = C::load(p.b_state + off);
+  const C ws = load_scale<T, kAny>(p.w_state, off), bs = load_shift<kAny>(p.b_state, off);
   request(integral_constant<int, 3>(), integral_constant<int, 7>());
   __builtin_amdgcn_s_barrier();   // waits for no memory: only keeps the row's waves in step at their largest group of requests
   __builtin_amdgcn_sched_barrier(0);
@@ -342,16 +330,16 @@ __global__ __launch_bounds__(kMaxLanes) void sum_lstm_staged_kernel(const LstmPa
 #pragma unroll
   for (int j = 0; j < E; ++j) {
     const float cnew = fmaf(cact[j], sigmoid_f(fmaf(p.alpha, b[j], a[j])), cell[j]);
-    ss = fmaf(cnew, cnew, ss);  // unrounded, as in the reference (:136)
+    if (!kAny || j >= at.repeated) ss = fmaf(cnew, cnew, ss);  // unrounded, as in the reference (:136)
     cell[j] = cnew;
   }
   {
     const C packed = C::template pack<T>(cell);
-    if (active) packed.store_stream(oc_row);
+    if (kKind == kFullWaves || at.live()) packed.template store_stream<kAny>(oc_row + off);
     packed.template unpack<T>(cell);   // the state phase sees the rounded cell (:163,174)
   }
   request(integral_constant<int, 7>(), integral_constant<int, 9>());
-  const float inv_cnew = rsqrtf(block_sum(active ? ss : 0.f, slots_cnew) * p.inv_D + p.eps_state);
+  const float inv_cnew = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cnew) * p.inv_D + p.eps_state);
 
   // phase 3: state = gelu(rmsnorm(rounded cell)) * sigmoid(pre_o) (reference :160-190)
   float st[E];
@@ -367,7 +355,7 @@ __global__ __launch_bounds__(kMaxLanes) void sum_lstm_staged_kernel(const LstmPa
   (kSharedZ ? in[0] : in[8]).template unpack<T>(b);
 #pragma unroll
   for (int j = 0; j < E; ++j) st[j] *= sigmoid_f(fmaf(p.alpha, b[j], a[j]));
-  if (active) C::template pack<T>(st).store_stream(os_row);
+  if (kKind == kFullWaves || at.live()) C::template pack<T>(st).template store_stream<kAny>(os_row + off);
 }
 
 // Any D, any alignment: element-wise, three passes like the reference's scalar
@@ -421,53 +409,50 @@ __global__ __launch_bounds__(256) void sum_lstm_scalar_kernel(const LstmParams p
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-
 template <typename T, bool kFastGelu, bool kSharedZ>
 static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
-  const int chunks = p.D / 8;
   const bool multi = rows > 1;
-  const bool vec = (p.D % 8 == 0) && chunks <= 2 * 1024 &&
-                   (!multi || (p.s_stride % 8 == 0 && p.z_stride % 8 == 0 && p.pc_stride % 8 == 0 &&
-                               p.out_stride % 8 == 0)) &&
-                   (!p.z_index || p.z_stride % 8 == 0) &&
-                   aligned16(p.states) && aligned16(p.z4) && aligned16(p.prev_cell) &&   /* null counts as aligned */
-                   aligned16(p.out_state) && aligned16(p.out_cell) && aligned16(p.w_cell) &&
-                   aligned16(p.b_cell) && aligned16(p.w_state) && aligned16(p.b_state);
+  const bool aligned = p.D % 8 == 0 &&
+                       (!multi || (p.s_stride % 8 == 0 && p.z_stride % 8 == 0 && p.pc_stride % 8 == 0 &&
+                                   p.out_stride % 8 == 0)) &&
+                       (!p.z_index || p.z_stride % 8 == 0) &&
+                       aligned16(p.states) && aligned16(p.z4) && aligned16(p.prev_cell) &&   /* null counts as aligned */
+                       aligned16(p.out_state) && aligned16(p.out_cell) && aligned16(p.w_cell) &&
+                       aligned16(p.b_cell) && aligned16(p.w_state) && aligned16(p.b_state);
+  const int chunks = (p.D + 7) / 8;
+  const int lanes = (chunks + 63) & ~63;
   const dim3 grid((unsigned)rows);
-  if (vec) {
-    const int cpt = chunks > 512 ? 2 : 1;   // one 16-byte chunk per lane up to 512 lanes (D <= 4096)
-    int threads = (chunks + cpt - 1) / cpt;
-    threads = std::max(64, (threads + 63) & ~63);
-    // All four vectors given and a row of up to 8192 elements: the staged kernel, one chunk per lane (512 rows of
-    // 5120 / 6144 / 8192 elements: 12.0 / 13.9 / 17.9 us against 17.6 / 19.9 / 22.5 us with two chunks per lane in the
-    // kernel below), with idle lanes in the last wave when the row is no multiple of 512 elements.
-    const bool staged = chunks <= 1024 && p.w_cell && p.b_cell && p.w_state && p.b_state;
-    const int lanes = (chunks + 63) & ~63;
-#define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, MAX_LANES, RAGGED)                                                \
-  hipLaunchKernelGGL((sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, MAX_LANES, RAGGED>), grid, dim3(lanes), 0, \
-                     s, p)
-    if (staged) {
-      const bool zero = !p.prev_cell, ragged = lanes != chunks;
-      if (chunks <= 512) {
-        if (zero && ragged) ARCTIC_LSTM_STAGED_LAUNCH(true, 512, true);
-        else if (zero) ARCTIC_LSTM_STAGED_LAUNCH(true, 512, false);
-        else if (ragged) ARCTIC_LSTM_STAGED_LAUNCH(false, 512, true);
-        else ARCTIC_LSTM_STAGED_LAUNCH(false, 512, false);
-      } else {
-        if (zero && ragged) ARCTIC_LSTM_STAGED_LAUNCH(true, 1024, true);
-        else if (zero) ARCTIC_LSTM_STAGED_LAUNCH(true, 1024, false);
-        else if (ragged) ARCTIC_LSTM_STAGED_LAUNCH(false, 1024, true);
-        else ARCTIC_LSTM_STAGED_LAUNCH(false, 1024, false);
-      }
-    }
-#undef ARCTIC_LSTM_STAGED_LAUNCH
-    else if (cpt == 1)
-      hipLaunchKernelGGL((sum_lstm_vec_kernel<T, 1, kFastGelu, 512, kSharedZ, true>), grid, dim3(threads), 0, s, p);
+  // One chunk per lane up to 1024 lanes (512 rows of 5120 / 6144 / 8192 elements: 12.0 / 13.9 / 17.5 us against 17.6 /
+  // 19.9 / 22.5 us with two chunks per lane in the other kernel; without scale and shift 512 rows of 4096 / 8192: 9.6 /
+  // 17.3 us against 11.0 / 24.1 us).  Rows that are not 16-byte aligned take the same kernels with accesses at any
+  // alignment, which cost 6 to 35 % over aligned ones (300 rows of 1536: 5.3 us aligned, 5.8 us 4-byte and 6.4 us 2-byte
+  // aligned) and are 3 to 5 times faster than element by element (23 us; 300 rows of 4096: 10.9 against 58 us).  Below
+  // 128 elements a single wave does a row's whole arithmetic and the element-wise kernel's 256 lanes are level or ahead
+  // (300 rows of 36 / 100 / 260 elements: 3.5 / 4.0 / 6.0 us element by element, 4.2 / 4.3 / 4.4 us in chunks).
+  constexpr int kShortRow = 128;
+#define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND) \
+  hipLaunchKernelGGL((sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND>), grid, dim3(lanes), 0, s, p)
+#define ARCTIC_LSTM_STAGED(KIND)                                    \
+  do {                                                              \
+    if (p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND);        \
+    else ARCTIC_LSTM_STAGED_LAUNCH(true, KIND);                     \
+  } while (0)
+  if (p.D >= (aligned ? 8 : kShortRow) && chunks <= 1024) {
+    const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
+    if (!aligned || !all_vectors) ARCTIC_LSTM_STAGED(kAnyRow);
+    else if (lanes != chunks) ARCTIC_LSTM_STAGED(kRagged);
+    else ARCTIC_LSTM_STAGED(kFullWaves);
+  } else if (chunks > 1024 && chunks <= 2 * 1024) {
+    const int threads = (((chunks + 1) / 2) + 63) & ~63;
+    if (aligned)
+      hipLaunchKernelGGL((sum_lstm_vec_kernel<T, kFastGelu, kSharedZ, false>), grid, dim3(threads), 0, s, p);
     else
-      hipLaunchKernelGGL((sum_lstm_vec_kernel<T, 2, kFastGelu, 1024, kSharedZ, false>), grid, dim3(threads), 0, s, p);
+      hipLaunchKernelGGL((sum_lstm_vec_kernel<T, kFastGelu, kSharedZ, true>), grid, dim3(threads), 0, s, p);
   } else {
     hipLaunchKernelGGL((sum_lstm_scalar_kernel<T, kFastGelu>), grid, dim3(256), 0, s, p, kSharedZ ? 0 : p.D);
   }
+#undef ARCTIC_LSTM_STAGED
+#undef ARCTIC_LSTM_STAGED_LAUNCH
 }
 
 }  // namespace arctic

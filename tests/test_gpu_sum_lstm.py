@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import oracle
+from arcticinference_amd import _native
 from helpers import assert_close, make_lstm_case, speculator_alpha, to_device_pitched
 
 pytestmark = pytest.mark.gpu
@@ -314,3 +315,36 @@ def test_staged_kernel_shapes(ops, D, rows, dtype):
         staged = ops.sum_lstm_shared_z(d["states"], z, cell, d["w_cell"], d["b_cell"], ones, zeros, *tail)
         general = ops.sum_lstm_shared_z(d["states"], z, cell, d["w_cell"], d["b_cell"], None, None, *tail)
         same(staged, general)
+
+
+@pytest.mark.parametrize("D,pad4,padD", [(8, 1, 3), (127, 0, 0), (128, 1, 1), (129, 3, 2), (513, 0, 0), (1023, 1, 0), (1024, 0, 3),
+                                         (1537, 3, 3), (4100, 0, 0), (8191, 2, 1), (8193, 0, 0), (12289, 1, 3), (16383, 0, 0),
+                                         (16385, 0, 0)])
+@pytest.mark.parametrize("rows", [2, 67])
+def test_rows_that_are_not_16_byte_aligned(ops, D, pad4, padD, rows):
+    """Odd widths and pitches in chunks of 8 whose last one overlaps the one before it, on both sides of every change of
+    kernel: against the oracle, with and without vectors, and nothing written outside the rows."""
+    dtype = torch.float16 if D % 2 else torch.bfloat16
+    for affine in (True, False):
+        c = make_lstm_case(rows=rows, D=D, dtype=dtype, seed=D + rows, pad4=pad4, padD=padD, wb_cell=affine, wb_state=affine,
+                           repeat_z=True)
+        got_s, got_c, _, _ = run(ops, c, alpha=0.35, fast=not affine)
+        args = [dev(c[k]) for k in ("prev_cell", "w_cell", "b_cell", "w_state", "b_state")]
+        z = dev(c["z4"])[:, :D]
+        st, ce = ops.sum_lstm_shared_z(dev(c["states"]), z, *args, 0.35, 1e-6, 1e-6, not affine)
+        assert torch.equal(st, got_s) and torch.equal(ce, got_c)
+    # a vector that starts one element into its storage, and guards around rows placed inside larger tensors
+    guard = torch.full((rows + 2, D + 9), 7.0, dtype=dtype, device=DEV)
+    state, cell = guard.clone(), guard.clone()
+    lib = _native.load()
+    s, z4 = dev(c["states"]), dev(c["z4"])
+    pc = dev(c["prev_cell"])
+    w = torch.ones(D + 1, dtype=dtype, device=DEV)[1:]
+    _native.check(lib.arctic_sum_lstm(
+        state[1:, 5:].data_ptr(), cell[1:, 5:].data_ptr(), s.data_ptr(), z4.data_ptr(), pc.data_ptr(), w.data_ptr(), None, None,
+        None, rows, D, s.stride(0), z4.stride(0), pc.stride(0), D + 9, 0.35, 1e-6, 1e-6, 1,
+        _native.DTYPE_BF16 if dtype == torch.bfloat16 else _native.DTYPE_F16, torch.cuda.current_stream().cuda_stream))
+    for got, want in ((state, got_s), (cell, got_c)):
+        assert_close(got[1:-1, 5:5 + D], want, RTOL, ATOL)
+        got[1:-1, 5:5 + D] = 7.0
+        assert torch.equal(got, guard)
