@@ -408,6 +408,13 @@ extern "C" int floor_write_per_layer_and_token(const void *keys, const void *val
   return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 
+// eight bf16 elements of a row, stored through the caches (both decompositions below read a row again)
+__device__ __forceinline__ void store8(char *row, int chunk, const float (&f)[8]) {
+  const uint4 v = arctic::pack8<arctic::BF16>(f);
+  const arctic::u32x4 words = {v.x, v.y, v.z, v.w};
+  *(ARCTIC_GLOBAL arctic::u32x4 *)(row + (int64_t)chunk * 16) = words;
+}
+
 // sum_lstm as the reference decomposes it (csrc/custom_ops/sum_lstm.cu:28-191): one workgroup of 128 lanes per row,
 // 16 bytes per lane and step, and three passes over global memory - the cell's pre-activation alone for its sum of
 // squares; then the forget, input and cell pre-activations with the previous cell, for the new cell, which is stored;
@@ -477,7 +484,7 @@ __global__ __launch_bounds__(kLanes) void sum_lstm_kernel(char *out_state, char 
       cell[k] = p[k] * sigmoid(f[k]) + gelu(normed) * sigmoid(in[k]);
       ss += cell[k] * cell[k];
     }
-    arctic::Chunk::pack<arctic::BF16>(cell).store(cell_row + (int64_t)i * 16);
+    store8(cell_row, i, cell);
   }
   total = Reduce(scratch1).Sum(ss);
   if (threadIdx.x == 0) inv_rms_cell = rsqrtf(total / (float)D + eps_state);
@@ -496,7 +503,7 @@ __global__ __launch_bounds__(kLanes) void sum_lstm_kernel(char *out_state, char 
       normed += b[k];
       state[k] = gelu(normed) * sigmoid(o[k]);
     }
-    arctic::Chunk::pack<arctic::BF16>(state).store(state_row + (int64_t)i * 16);
+    store8(state_row, i, state);
   }
 }
 
@@ -556,7 +563,7 @@ __global__ __launch_bounds__(kLanes) void ln_kernel(char *out, const char *in, c
       y[k] *= w[k];
       y[k] += b[k];
     }
-    arctic::Chunk::pack<arctic::BF16>(y).store(row_out + (int64_t)i * 16);
+    store8(row_out, i, y);
   }
 }
 
