@@ -161,6 +161,21 @@ struct Chunk {
   __device__ static __forceinline__ Chunk pack(const float (&f)[8]) { return Chunk{pack8<T>(f)}; }
 };
 
+// A row of any width from 8 elements on is covered by chunks of 8: chunk c starts at element 8 c, the last one at D - 8,
+// so that it ends with the row.  Where the width is no multiple of 8 the last chunk's first elements are the end of the
+// chunk before it: they are computed twice, bit for bit alike, stored twice and counted once.  `repeated` says how many
+// of a chunk's elements do not count: 0, 1 to 7 in such a last chunk, 8 or more for a lane behind the row's end.
+struct Place {
+  uint32_t off;   // bytes from the row's start
+  int repeated;
+  __device__ __forceinline__ Place(int chunk, int D) {
+    const int start = min(chunk * Chunk::kElems, D - Chunk::kElems);
+    off = (uint32_t)start * 2;
+    repeated = chunk * Chunk::kElems - start;
+  }
+  __device__ __forceinline__ bool live() const { return repeated < Chunk::kElems; }
+};
+
 // ---- wave64 / workgroup reductions ------------------------------------------
 // DPP butterfly inside each row of 16 lanes, then the four row totals are read
 // with v_readlane.  Every lane returns the same wave total.

@@ -6,7 +6,8 @@
 // One workgroup per row.  On the vector path every lane keeps its 16-byte
 // chunks of the row in registers between the sum of squares and the scaling, so
 // the row is read from HBM once (the reference reads it twice); the sum is a DPP
-// wave reduction followed by a small LDS combine.
+// wave reduction followed by a small LDS combine.  Rows that are only element-aligned
+// take the same kernel with accesses at any alignment.
 //
 // The same kernel also carries the element-wise steps the speculator runs around
 // this norm (arctic_speculator.py:296-307,733-734,809-816), each with the rounding
@@ -46,13 +47,18 @@ __device__ __forceinline__ float glue_tail(float y, const LnGlue &g) {
   return y;
 }
 
-template <typename T, int kChunksPerThread, bool kGlue>
+// kAnyRow: rows that are only element-aligned (odd widths, pitches or bases): accesses at any alignment, and the last chunk
+// of a width that is no multiple of 8 overlaps the one before it (common.hpp).  Bound like the aligned rows by the node's
+// start and two dependent round trips; element by element and in two passes over the row (as such rows went before) every
+// pass was a round trip per 256 elements.
+template <typename T, int kChunksPerThread, bool kGlue, bool kAnyRow>
 __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     char *__restrict__ out, const char *__restrict__ in, const char *__restrict__ weight,
     const char *__restrict__ bias, int64_t in_row_stride_bytes, int hidden, float inv_hidden, float eps,
     LnGlue glue) {
   __shared__ float slots[16];
-  const int chunks = hidden >> 3;
+  const int chunks = kAnyRow ? (hidden + 7) >> 3 : hidden >> 3;
+  auto offset = [&](int c) { return kAnyRow ? (int64_t)Place(c, hidden).off : (int64_t)c * 16; };
   const char *row_in = in + (int64_t)blockIdx.x * in_row_stride_bytes;
   char *row_out = out + (int64_t)blockIdx.x * hidden * 2;
 
@@ -63,14 +69,14 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
 #pragma unroll
   for (int k = 0; k < kChunksPerThread; ++k) {
     const int c = threadIdx.x + k * blockDim.x;
-    if (weight && c < chunks) wv[k] = load16(weight + (int64_t)c * 16);
-    if (bias && c < chunks) bv[k] = load16(bias + (int64_t)c * 16);
+    if (weight && c < chunks) wv[k] = load16<kAnyRow>(weight + offset(c));
+    if (bias && c < chunks) bv[k] = load16<kAnyRow>(bias + offset(c));
   }
 #pragma unroll
   for (int k = 0; k < kChunksPerThread; ++k) {
     const int c = threadIdx.x + k * blockDim.x;
     raw[k] = make_uint4(0, 0, 0, 0);
-    if (c < chunks) raw[k] = load16_stream(row_in + (int64_t)c * 16);
+    if (c < chunks) raw[k] = load16_stream<kAnyRow>(row_in + offset(c));
   }
   if (kGlue && glue.z) {
     int64_t z_at = blockIdx.x;
@@ -81,7 +87,7 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     for (int k = 0; k < kChunksPerThread; ++k) {
       const int c = threadIdx.x + k * blockDim.x;
       zr[k] = make_uint4(0, 0, 0, 0);
-      if (c < chunks) zr[k] = load16_stream(row_z + (int64_t)c * 16);
+      if (c < chunks) zr[k] = load16_stream<kAnyRow>(row_z + offset(c));
     }
 #pragma unroll
     for (int k = 0; k < kChunksPerThread; ++k) {
@@ -98,7 +104,8 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     float x[8];
     unpack8<T>(raw[k], x);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+    for (int j = 0; j < 8; ++j)
+      if (!kAnyRow || j >= Place(threadIdx.x + k * blockDim.x, hidden).repeated) ss += x[j] * x[j];
   }
   const float total = block_sum(ss, slots);
   const float inv = rsqrtf(total * inv_hidden + eps);
@@ -127,11 +134,11 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = glue_tail<T>(x[j], glue);
     }
-    store16_stream(row_out + (int64_t)c * 16, pack8<T>(x));
+    store16_stream<kAnyRow>(row_out + offset(c), pack8<T>(x));
   }
 }
 
-// Any hidden size, any alignment: element-wise, two passes over the row.
+// What is left (short unaligned rows, rows beyond 65536 elements): element-wise, two passes over the row.
 template <typename T>
 __global__ __launch_bounds__(256) void spec_ln_scalar_kernel(
     uint16_t *__restrict__ out, const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
@@ -168,29 +175,33 @@ static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 template <typename T>
 static void launch_ln(void *out, const void *in, const void *w, const void *b, int64_t rows, int hidden,
                       int64_t in_row_stride, float eps, const LnGlue &glue, hipStream_t s) {
-  const int chunks = hidden / 8;
+  const int chunks = (hidden + 7) / 8;
   const float inv_hidden = 1.0f / (float)hidden;
-  const bool vec = (hidden % 8 == 0) && (in_row_stride % 8 == 0 || rows == 1) && aligned16(in) &&
-                   aligned16(out) && (!w || aligned16(w)) && (!b || aligned16(b)) && chunks <= 8 * 1024 &&
-                   (!glue.z || (aligned16(glue.z) && (glue.z_row_stride_bytes % 16 == 0 || (rows == 1 && !glue.z_index))));
+  const bool aligned = (hidden % 8 == 0) && (in_row_stride % 8 == 0 || rows == 1) && aligned16(in) &&
+                       aligned16(out) && (!w || aligned16(w)) && (!b || aligned16(b)) &&
+                       (!glue.z || (aligned16(glue.z) && (glue.z_row_stride_bytes % 16 == 0 || (rows == 1 && !glue.z_index))));
   const bool plain = !glue.z && glue.activation == ARCTIC_ACT_NONE && glue.out_scale == 1.0f;
   const dim3 grid((unsigned)rows);
-  if (vec) {
+  // Rows that are not 16-byte aligned take the same kernel with accesses at any alignment.  Us per call in a graph, element
+  // by element / in chunks: 300 x 1537 fp16 5.5 / 3.3, 64 x 4096 pitched by 4099 7.0 / 2.7, 4000 x 4097 34.6 / 17.5 (3.7
+  // TB/s), 300 x 20000 pitched by 20001 57 / 9.9; 4000 x 160 4.7 / 3.6 and 300 x 100 level at 2.2, so that rows of fewer
+  // than 128 elements, where a single wave would do a row's work, stay with the element-wise kernel.
+  constexpr int kShortRow = 128;
+  if (hidden >= (aligned ? 8 : kShortRow) && chunks <= 8 * 1024) {
     int cpt = 1;
     while (cpt < 8 && (chunks + cpt - 1) / cpt > 1024) cpt *= 2;
     int threads = (chunks + cpt - 1) / cpt;
     threads = std::max(64, (threads + 63) & ~63);
     const int64_t stride_bytes = in_row_stride * 2;
-#define ARCTIC_LN_LAUNCH(CPT)                                                                              \
-  do {                                                                                                     \
-    if (plain)                                                                                             \
-      hipLaunchKernelGGL((spec_ln_vec_kernel<T, CPT, false>), grid, dim3(threads), 0, s, (char *)out,       \
-                         (const char *)in, (const char *)w, (const char *)b, stride_bytes, hidden,          \
-                         inv_hidden, eps, glue);                                                           \
-    else                                                                                                   \
-      hipLaunchKernelGGL((spec_ln_vec_kernel<T, CPT, true>), grid, dim3(threads), 0, s, (char *)out,        \
-                         (const char *)in, (const char *)w, (const char *)b, stride_bytes, hidden,          \
-                         inv_hidden, eps, glue);                                                           \
+#define ARCTIC_LN_LAUNCH_AS(CPT, GLUE, ANY)                                                                       \
+  hipLaunchKernelGGL((spec_ln_vec_kernel<T, CPT, GLUE, ANY>), grid, dim3(threads), 0, s, (char *)out,             \
+                     (const char *)in, (const char *)w, (const char *)b, stride_bytes, hidden, inv_hidden, eps, glue)
+#define ARCTIC_LN_LAUNCH(CPT)                               \
+  do {                                                      \
+    if (plain && aligned) ARCTIC_LN_LAUNCH_AS(CPT, false, false); \
+    else if (plain) ARCTIC_LN_LAUNCH_AS(CPT, false, true);  \
+    else if (aligned) ARCTIC_LN_LAUNCH_AS(CPT, true, false); \
+    else ARCTIC_LN_LAUNCH_AS(CPT, true, true);              \
   } while (0)
     switch (cpt) {
       case 1: ARCTIC_LN_LAUNCH(1); break;
@@ -199,6 +210,7 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
       default: ARCTIC_LN_LAUNCH(8); break;
     }
 #undef ARCTIC_LN_LAUNCH
+#undef ARCTIC_LN_LAUNCH_AS
   } else {
     hipLaunchKernelGGL((spec_ln_scalar_kernel<T>), grid, dim3(256), 0, s, (uint16_t *)out,
                        (const uint16_t *)in, (const uint16_t *)w, (const uint16_t *)b, in_row_stride, hidden,

@@ -49,21 +49,6 @@ struct LstmParams {
   float eps_state;
 };
 
-// A row of any width from 8 elements on is covered by chunks of 8: chunk c starts at element 8 c, the last one at D - 8,
-// so that it ends with the row.  Where the width is no multiple of 8 the last chunk's first elements are the end of the
-// chunk before it: they are computed twice, bit for bit alike, stored twice and counted once.  `repeated` says how many
-// of a chunk's elements do not count: 0, 1 to 7 in such a last chunk, 8 or more for a lane behind the row's end.
-struct Place {
-  uint32_t off;   // bytes from the row's start
-  int repeated;
-  __device__ __forceinline__ Place(int chunk, int D) {
-    const int start = min(chunk * Chunk::kElems, D - Chunk::kElems);
-    off = (uint32_t)start * 2;
-    repeated = chunk * Chunk::kElems - start;
-  }
-  __device__ __forceinline__ bool live() const { return repeated < Chunk::kElems; }
-};
-
 // kFullWaves: rows 16-byte aligned, all four scale / shift vectors given, every lane of every wave owns a chunk of 8
 // elements; kRagged: the same with lanes to spare in the last wave; kAnyRow: everything else - vectors missing, rows
 // only element-aligned (odd widths, pitches or bases; see common.hpp).

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import oracle
+from arcticinference_amd import _native
 from helpers import assert_close, pitched, to_device_pitched
 
 pytestmark = pytest.mark.gpu
@@ -46,10 +47,37 @@ def test_config4_layernorm(ops, weight_only):
 
 @pytest.mark.parametrize("pad", [8, 3])
 def test_pitched_rows(ops, pad):
-    # row stride larger than hidden; pad 3 breaks 16-byte alignment and takes the element-wise kernel
+    # row stride larger than hidden; pad 3 breaks 16-byte alignment
     g = torch.Generator().manual_seed(1)
     x = pitched(19, 256, pad, torch.bfloat16, g)
     run(ops, x, None, None)
+
+
+@pytest.mark.parametrize("hidden,pad", [(7, 1), (127, 0), (128, 1), (129, 0), (135, 3), (513, 0), (1537, 3), (4096, 3), (8191, 1),
+                                        (8193, 0), (16385, 2), (32769, 0), (65535, 1), (65537, 0)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_rows_that_are_not_16_byte_aligned(ops, hidden, pad, dtype):
+    """Odd widths, pitches and bases on both sides of every change of kernel and of chunks per lane, with and without what
+    surrounds the norm, against the oracle; nothing is written outside the output's rows."""
+    rows = 5
+    g = torch.Generator().manual_seed(hidden + pad)
+    x = pitched(rows, hidden, pad, dtype, g)
+    w, b = torch.randn(hidden, generator=g).to(dtype), torch.randn(hidden, generator=g).to(dtype)
+    run(ops, x, w, b)
+    run(ops, x, None, None)
+    table = torch.randn(9, hidden, generator=g).to(dtype)
+    ids = torch.tensor([8, 0, 3, 3, 7])
+    xd = to_device_pitched(x, DEV)
+    got = ops.speculator_embed_add_ln_gelu(xd, table.to(DEV), ids.to(DEV), w.to(DEV), b.to(DEV), 1.7, 1e-6)
+    assert_close(got, oracle.speculator_add_ln_act(x, table[ids], w, b, 1.7, 1e-6, "gelu", 1.0), RTOL, ATOL, "embed_add_ln_gelu")
+    # vectors and output that start one element into their storage, guards around the output
+    out = torch.full((rows * hidden + 16,), 7.0, dtype=dtype, device=DEV)
+    one_off = [torch.cat([v[:1], v]).to(DEV)[1:] for v in (w, b)]
+    _native.check(_native.load().arctic_speculator_ln(
+        out[3:].data_ptr(), xd.data_ptr(), one_off[0].data_ptr(), one_off[1].data_ptr(), rows, hidden, xd.stride(0), 1e-6,
+        _native.DTYPE_BF16 if dtype == torch.bfloat16 else _native.DTYPE_F16, torch.cuda.current_stream().cuda_stream))
+    assert_close(out[3:3 + rows * hidden].view(rows, hidden), oracle.speculator_ln(x, w, b, 1e-6), RTOL, ATOL, "speculator_ln")
+    assert bool((out[:3] == 7.0).all()) and bool((out[3 + rows * hidden:] == 7.0).all())
 
 
 def test_large_magnitudes_and_eps(ops):
