@@ -38,10 +38,10 @@ struct LnGlue {
 };
 
 template <typename T>
-__device__ __forceinline__ float glue_tail(float y, const LnGlue &g) {
-  if (g.activation != ARCTIC_ACT_NONE) {
+__device__ __forceinline__ float glue_tail(float y, const LnGlue &g, int activation) {
+  if (activation != ARCTIC_ACT_NONE) {
     y = T::requant(y);
-    y = g.activation == ARCTIC_ACT_GELU ? gelu_erf(y) : gelu_tanh(y);
+    y = activation == ARCTIC_ACT_GELU ? gelu_erf(y) : gelu_tanh(y);
   }
   if (g.out_scale != 1.0f) y = T::requant(y) * g.out_scale;
   return y;
@@ -51,7 +51,12 @@ __device__ __forceinline__ float glue_tail(float y, const LnGlue &g) {
 // of a width that is no multiple of 8 overlaps the one before it (common.hpp).  Bound like the aligned rows by the node's
 // start and two dependent round trips; element by element and in two passes over the row (as such rows went before) every
 // pass was a round trip per 256 elements.
-template <typename T, int kChunksPerThread, bool kGlue, bool kAnyRow>
+// kGlue: what surrounds the norm: nothing (kPlain), or an add and a scale with or without the activation of that code - a
+// launch of few rows waits for its instructions as well, and a kernel that holds both activations is twice as long (us per
+// call in a graph, chosen at run time / here: embedding + add + norm + GELU of 64 x 2880 3.09 / 2.90, 1 x 4096 2.78 / 2.56,
+// the scaled norm of 7 x 4096 2.20 / 2.10).
+constexpr int kPlain = -1;
+template <typename T, int kChunksPerThread, int kGlue, bool kAnyRow>
 __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     char *__restrict__ out, const char *__restrict__ in, const char *__restrict__ weight,
     const char *__restrict__ bias, int64_t in_row_stride_bytes, int hidden, float inv_hidden, float eps,
@@ -78,7 +83,7 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     raw[k] = make_uint4(0, 0, 0, 0);
     if (c < chunks) raw[k] = load16_stream<kAnyRow>(row_in + offset(c));
   }
-  if (kGlue && glue.z) {
+  if (kGlue != kPlain && glue.z) {
     int64_t z_at = blockIdx.x;
     if (glue.z_index) z_at = min(max(glue.z_index[blockIdx.x], (int64_t)0), glue.z_rows - 1);
     const char *row_z = glue.z + z_at * glue.z_row_stride_bytes;
@@ -130,9 +135,9 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += b[j];
     }
-    if (kGlue) {
+    if (kGlue != kPlain) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = glue_tail<T>(x[j], glue);
+      for (int j = 0; j < 8; ++j) x[j] = glue_tail<T>(x[j], glue, kGlue);
     }
     store16_stream<kAnyRow>(row_out + offset(c), pack8<T>(x));
   }
@@ -166,7 +171,7 @@ __global__ __launch_bounds__(256) void spec_ln_scalar_kernel(
     float y = element(j) * inv;
     if (weight) y *= T::lo(weight[j]);
     if (bias) y += T::lo(bias[j]);
-    row_out[j] = (uint16_t)T::round_bits(glue_tail<T>(y, glue));
+    row_out[j] = (uint16_t)T::round_bits(glue_tail<T>(y, glue, glue.activation));
   }
 }
 
@@ -196,12 +201,17 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
 #define ARCTIC_LN_LAUNCH_AS(CPT, GLUE, ANY)                                                                       \
   hipLaunchKernelGGL((spec_ln_vec_kernel<T, CPT, GLUE, ANY>), grid, dim3(threads), 0, s, (char *)out,             \
                      (const char *)in, (const char *)w, (const char *)b, stride_bytes, hidden, inv_hidden, eps, glue)
-#define ARCTIC_LN_LAUNCH(CPT)                               \
+#define ARCTIC_LN_LAUNCH_GLUE(CPT, GLUE)                    \
   do {                                                      \
-    if (plain && aligned) ARCTIC_LN_LAUNCH_AS(CPT, false, false); \
-    else if (plain) ARCTIC_LN_LAUNCH_AS(CPT, false, true);  \
-    else if (aligned) ARCTIC_LN_LAUNCH_AS(CPT, true, false); \
-    else ARCTIC_LN_LAUNCH_AS(CPT, true, true);              \
+    if (aligned) ARCTIC_LN_LAUNCH_AS(CPT, GLUE, false);     \
+    else ARCTIC_LN_LAUNCH_AS(CPT, GLUE, true);              \
+  } while (0)
+#define ARCTIC_LN_LAUNCH(CPT)                                                                          \
+  do {                                                                                                 \
+    if (plain) ARCTIC_LN_LAUNCH_GLUE(CPT, kPlain);                                                     \
+    else if (glue.activation == ARCTIC_ACT_NONE) ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_NONE);          \
+    else if (glue.activation == ARCTIC_ACT_GELU) ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_GELU);          \
+    else ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_GELU_TANH);                                             \
   } while (0)
     switch (cpt) {
       case 1: ARCTIC_LN_LAUNCH(1); break;
@@ -210,6 +220,7 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
       default: ARCTIC_LN_LAUNCH(8); break;
     }
 #undef ARCTIC_LN_LAUNCH
+#undef ARCTIC_LN_LAUNCH_GLUE
 #undef ARCTIC_LN_LAUNCH_AS
   } else {
     hipLaunchKernelGGL((spec_ln_scalar_kernel<T>), grid, dim3(256), 0, s, (uint16_t *)out,
