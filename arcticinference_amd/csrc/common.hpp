@@ -23,6 +23,22 @@ inline bool pitch_ok(int64_t pitch_elems, int64_t rows, int elem_bytes) {
   return pitch_elems <= limit / (rows > 1 ? rows - 1 : 1);
 }
 
+// Division of numbers below 2^31 by one that is known at launch: a product and a shift in place of the thirty (32 bits) to
+// hundred (64 bits) instructions of a general division.  With s = ceil(log2 d) and m = floor(2^(31+s) / d) + 1, which is
+// at most 2^32 - 1, m d - 2^(31+s) lies in (0, 2^s], so that m n / 2^(31+s) exceeds n / d by less than 1 / d for every
+// n < 2^31 and has the same integer part.
+struct Divisor {
+  uint32_t m, shift, d;
+  Divisor() = default;
+  explicit Divisor(uint32_t by) : d(by) {
+    uint32_t s = 0;
+    while (((uint64_t)1 << s) < by) ++s;
+    shift = 31 + s;
+    m = (uint32_t)(((uint64_t)1 << shift) / by + 1);
+  }
+  __host__ __device__ uint32_t quotient(uint32_t n) const { return (uint32_t)(((uint64_t)n * m) >> shift); }
+};
+
 // ---- 16-bit floats ---------------------------------------------------------
 // Activation element types. to_float is exact; from_float rounds to nearest
 // even (what __float2bfloat16 / __float2half do in the reference,

@@ -33,24 +33,29 @@ struct Fp4Params {
   int64_t head_stride;
   int64_t total_groups;  // num_tokens * 2 * num_heads * groups_per_head
   int64_t num_slots;     // slots at or beyond this move nothing
-  int num_heads;
-  int groups_per_head;   // head_size / 16
   int block_size;
+  int64_t groups_per_row;
+  Divisor by_row;    // groups_per_row = num_heads * groups_per_head
+  Divisor by_head;   // groups_per_head = head_size / 16
+  Divisor by_block;  // block_size
 };
 
 // One group of 16 elements per lane, single-wave workgroups: a wave's 64 lanes stay on 64 consecutive groups (2 KiB
-// of source, 512 bytes of packed cache).
+// of source, 512 bytes of packed cache).  The three divisions that find a group's place were more than half of a wave's
+// 560 instructions when they were general ones; with products in their place (us per call in a graph, before / after)
+// 512 tokens of 8 x 128 2.43 / 2.31, 2048 4.00 / 3.68, 8192 9.9 / 9.45 (4.5 TB/s), 12640 14.4 / 13.5, 32768 33 / 33.
 constexpr int kFp4Lanes = 64;
 
-template <typename T>
+// kManyGroups: 2^31 groups or more, beyond what a Divisor takes.
+template <typename T, bool kManyGroups>
 __global__ __launch_bounds__(kFp4Lanes) void kv_write_fp4_kernel(const Fp4Params p) {
-  const int groups_per_row = p.num_heads * p.groups_per_head;
   // the slot is requested first and the group's 32 bytes right behind it: their address does not depend on the slot,
   // so one round trip to memory serves both (a padding token throws its group away)
   const int64_t idx = (int64_t)blockIdx.x * kFp4Lanes + threadIdx.x;
   const int64_t at_group = min(idx, p.total_groups - 1);   // lanes past the end read the last group and drop it
-  const int64_t row = at_group / groups_per_row;           // token * 2 + (0 = K, 1 = V)
-  const int in_row = (int)(at_group - row * groups_per_row);
+  // token * 2 + (0 = K, 1 = V)
+  const int64_t row = kManyGroups ? at_group / p.groups_per_row : (int64_t)p.by_row.quotient((uint32_t)at_group);
+  const uint32_t in_row = (uint32_t)(at_group - row * p.groups_per_row);
   const int64_t token = row >> 1;
   const int64_t slot = p.slot_mapping[token];
   const char *src = ((row & 1) ? p.value + token * p.value_stride_bytes : p.key + token * p.key_stride_bytes) +
@@ -60,10 +65,10 @@ __global__ __launch_bounds__(kFp4Lanes) void kv_write_fp4_kernel(const Fp4Params
   __builtin_amdgcn_sched_barrier(0);   // keeps the loads above the tests of the slot
   if (idx >= p.total_groups) return;
   if (slot < 0 || slot >= p.num_slots) return;  // padding token, or a slot outside the cache
-  const int head = in_row / p.groups_per_head;
-  const int group = in_row - head * p.groups_per_head;
+  const uint32_t head = p.by_head.quotient(in_row);
+  const uint32_t group = in_row - head * p.by_head.d;
   const bool is_v = row & 1;
-  const int64_t blk = slot / p.block_size;
+  const int64_t blk = slot < 0x80000000LL ? (int64_t)p.by_block.quotient((uint32_t)slot) : slot / p.block_size;
   const int64_t off = slot - blk * p.block_size;
 
   float x[16];
@@ -151,10 +156,12 @@ extern "C" int arctic_reshape_and_cache_flash_fp4(
   p.block_stride = block_stride;
   p.page_stride = page_stride;
   p.head_stride = head_stride;
-  p.num_heads = num_heads;
-  p.groups_per_head = head_size / 16;
   p.block_size = block_size;
-  p.total_groups = num_tokens * 2 * num_heads * p.groups_per_head;
+  p.groups_per_row = (int64_t)num_heads * (head_size / 16);
+  p.by_row = Divisor((uint32_t)p.groups_per_row);
+  p.by_head = Divisor((uint32_t)(head_size / 16));
+  p.by_block = Divisor((uint32_t)block_size);
+  p.total_groups = num_tokens * 2 * p.groups_per_row;
   p.num_slots = num_blocks > 0 ? num_blocks * (int64_t)block_size : INT64_MAX;
   hipStream_t s = (hipStream_t)stream;
   // One group per lane in workgroups of one wave: nothing is shared between lanes, and at 8192 tokens and beyond
@@ -162,9 +169,16 @@ extern "C" int arctic_reshape_and_cache_flash_fp4(
   // four groups per lane all measured slower.
   const int64_t grid = (p.total_groups + kFp4Lanes - 1) / kFp4Lanes;
   if (grid > 0x7fffffffLL) return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: too many tokens", fn);
-  if (dtype == ARCTIC_DTYPE_BF16)
-    hipLaunchKernelGGL((kv_write_fp4_kernel<BF16>), dim3((unsigned)grid), dim3(kFp4Lanes), 0, s, p);
-  else
-    hipLaunchKernelGGL((kv_write_fp4_kernel<F16>), dim3((unsigned)grid), dim3(kFp4Lanes), 0, s, p);
+  const bool many = p.total_groups > 0x7fffffffLL;
+#define ARCTIC_FP4_LAUNCH(TYPE, MANY) \
+  hipLaunchKernelGGL((kv_write_fp4_kernel<TYPE, MANY>), dim3((unsigned)grid), dim3(kFp4Lanes), 0, s, p)
+  if (dtype == ARCTIC_DTYPE_BF16) {
+    if (many) ARCTIC_FP4_LAUNCH(BF16, true);
+    else ARCTIC_FP4_LAUNCH(BF16, false);
+  } else {
+    if (many) ARCTIC_FP4_LAUNCH(F16, true);
+    else ARCTIC_FP4_LAUNCH(F16, false);
+  }
+#undef ARCTIC_FP4_LAUNCH
   return check_launch(fn);
 }

@@ -68,3 +68,20 @@ def test_degenerate_scales():
     x = np.array([0.0, -0.0, 1.0, -3.5, np.inf, -np.inf, np.nan, 1e-40, 3e38], dtype=np.float32)
     for sv in (0.0, -0.0, np.inf, -np.inf, np.nan, 1e-45, 3.4e38, -2.0):
         check(x, np.full_like(x, sv))
+
+
+def test_division_by_a_product_and_a_shift():
+    """The kernels divide group, slot and chunk numbers n < 2^31 by d as (n * m) >> (31 + s) with s = ceil(log2 d) and
+    m = floor(2^(31 + s) / d) + 1 in 32 bits: the integer quotient for every n, looked at where it could go wrong - on
+    both sides of the multiples of d, at the largest n and at random."""
+    rng = np.random.default_rng(5)
+    divisors = np.unique(np.concatenate([np.arange(1, 3000), 2 ** np.arange(31) + 1, 2 ** np.arange(31),
+                                         2 ** np.arange(1, 31) - 1, rng.integers(1, 2 ** 31, 3000), [2 ** 31 - 1]]))
+    for d in divisors.tolist():
+        s = (d - 1).bit_length()
+        m = (1 << (31 + s)) // d + 1
+        assert m < 1 << 32
+        q = rng.integers(0, 2 ** 31, 200) // d
+        n = np.concatenate([q * d, q * d + d - 1, np.maximum(q * d - 1, 0), [0, 2 ** 31 - 1], rng.integers(0, 2 ** 31, 50)])
+        n = n[n < 2 ** 31].astype(np.uint64)
+        assert np.array_equal((n * np.uint64(m)) >> np.uint64(31 + s), n // np.uint64(d)), d
