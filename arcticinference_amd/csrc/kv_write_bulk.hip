@@ -57,6 +57,12 @@ struct BulkParams {
   int block_size;
   int chunks_per_row;    // 16-byte source chunks per (token, layer) row
   int chunk_shift;       // log2(chunks_per_row) or -1
+  // The places of a chunk, a slot and a workgroup by products: general divisions stand between the slot's arrival and the
+  // first store, and in rows that are no power of two long one per chunk (us per call in a graph, before / after: 5 tokens
+  // x 16 layers of 8 x 128 to fp8 3.08 / 2.97, 64 x 33 of 3 x 96 4.52 / 4.11, 1024 x 33 15.1 / 14.4).
+  Divisor by_chunks;     // chunks_per_row
+  Divisor by_block;      // block_size
+  Divisor by_groups;     // groups_per_token
   // select variants: token t's source rows are also copied, unconverted, to the rows j of keys_out / values_out with
   // indices[j] == t.  With a row map (kSelectByRowMap) that is row row_map[t] of keys_out /
   // values_out (already offset to the first layer of this launch); a negative row or one >= num_out_rows = none
@@ -213,7 +219,7 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
     }
     block -= p.index_blocks;
   }
-  const int64_t token = block / (unsigned)p.groups_per_token;
+  const int64_t token = p.by_groups.quotient(block);
   const int group = block - (unsigned)token * (unsigned)p.groups_per_token;
   const int layer0 = group * p.layers_per_group;
   const int nlayers = min(p.layers_per_group, p.num_layers - layer0);
@@ -228,7 +234,7 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
       r = c >> p.chunk_shift;
       col = c & (cpr - 1);
     } else {
-      r = c / cpr;
+      r = (int)p.by_chunks.quotient((uint32_t)c);
       col = c - r * cpr;
     }
   };
@@ -290,9 +296,9 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
   if (to_cache) {
     int64_t blk, off;
     if (slot < 0x7fffffffLL) {
-      const uint32_t s32 = (uint32_t)slot, bs = (uint32_t)p.block_size;
-      blk = s32 / bs;
-      off = s32 - (uint32_t)blk * bs;
+      const uint32_t s32 = (uint32_t)slot;
+      blk = p.by_block.quotient(s32);
+      off = s32 - (uint32_t)blk * (uint32_t)p.block_size;
     } else {
       blk = slot / p.block_size;
       off = slot - blk * p.block_size;
@@ -741,6 +747,9 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       const Shape shape = {wide, !wide && num_tokens <= kMostThrough / per_token && !in_l2};
       p.layers_per_group = (count + groups - 1) / groups;
       p.groups_per_token = (count + p.layers_per_group - 1) / p.layers_per_group;
+      p.by_chunks = Divisor((uint32_t)std::max(1, p.chunks_per_row));
+      p.by_block = Divisor((uint32_t)block_size);
+      p.by_groups = Divisor((uint32_t)p.groups_per_token);
       // lanes of the shape launched below when rows are selected (the only case with index workgroups)
       const int lanes = !vec ? kScalarThreads : (wide && p.chunk_shift >= 0) ? 512 : 256;
       const int64_t index_blocks = p.indices ? (p.num_out_rows + lanes - 1) / lanes : 0;

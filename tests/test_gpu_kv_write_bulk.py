@@ -65,6 +65,16 @@ def test_both_sides_of_the_store_rule(ops, kv, shape, limit, beyond):
     run_both(ops, make_bulk_case(T=T, bs=16, NB=T // 16 + 2, kv_cache_dtype=kv, seed=17, std=1.5, pad_fraction=0.05, **shape))
 
 
+@pytest.mark.parametrize("shape", [
+    dict(T=5, L=3, H=1, D=8, bs=1, NB=40),          # one chunk per row, one slot per block
+    dict(T=70, L=64, H=7, D=72, bs=7, NB=12),       # several workgroups per token, blocks of no power of two
+    dict(T=9, L=1, H=5, D=4096, bs=3, NB=5),        # rows longer than a batch
+])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+def test_places_of_chunks_slots_and_workgroups(ops, kv, shape):
+    run_both(ops, make_bulk_case(kv_cache_dtype=kv, seed=19, std=1.5, **shape))
+
+
 def test_all_padding_leaves_cache_untouched(ops):
     case = make_bulk_case(T=16, L=3, H=2, D=64, bs=16, NB=4, kv_cache_dtype="fp8", seed=7)
     case["slot_mapping"].fill_(-1)
