@@ -15,25 +15,21 @@ __device__ __forceinline__ float fast_exp(float x) {            // e^x
 __device__ __forceinline__ float sigmoid_f(float x) {
   return __builtin_amdgcn_rcpf(1.0f + fast_exp(-x));
 }
-// gelu(x) = x * Phi(x) = max(x, 0) - |x| q(|x|) with q(z) = Phi(-z) = 2^P(z), P a polynomial of degree 8: one
-// transcendental instruction per value.  The rational form of Abramowitz & Stegun 7.1.26 takes two (a reciprocal as
-// well) and one more multiply, and where a launch of sum_lstm waits for its arithmetic that shows (us per call in a
-// graph, rational form / this one): 7 rows of 4096 4.23 / 4.00, 512 rows of 8192 13.7 / 13.0, 2048 of 2880 21.6 / 20.3.
-// P is the best uniform fit of log2 Phi(-z) on [0, 5.8] under the weight max(q max(z, 0.3), 5e-5), as a linear program
-// over 6000 points gives it: the error of z q, and in the tail the relative error of q.  Against 64 bits (rational form
-// in brackets): 2.6e-8 (5.4e-8) rms over N(0, 1), 2.5e-7 (3.3e-7) at the worst, relative 3e-5 (1.7e-4) where
-// |gelu| > 1e-3, 5e-5 (5e-4) at -4 and 2.4e-3 (3.6e-3) at -6.  Beyond 5.8 P goes on falling, from -28.
+// gelu(x) = x * Phi(x) with Phi from Abramowitz & Stegun 7.1.26
+//   erfc(z) = (a1 t + ... + a5 t^5) exp(-z^2),  t = 1 / (1 + 0.3275911 z),  z >= 0
+// (|error| <= 1.5e-7, the level of fp32 rounding).  With z = |x| / sqrt(2) and
+// q = erfc(z) / 2:   gelu(x) = x - x q  for x >= 0  and  x q  for x < 0,
+// i.e. max(x, 0) - |x| q.  One reciprocal and one exp2 per value.
 __device__ __forceinline__ float gelu_erf(float x) {
   const float ax = fabsf(x);
-  float p = fmaf(-9.312184374721255e-07f, ax, 1.5563609849778004e-05f);
-  p = fmaf(p, ax, -6.800304254284129e-05f);
-  p = fmaf(p, ax, -0.0004356678109616041f);
-  p = fmaf(p, ax, 0.0074738264083862305f);
-  p = fmaf(p, ax, -0.05279786139726639f);
-  p = fmaf(p, ax, -0.45910027623176575f);
-  p = fmaf(p, ax, -1.1511198282241821f);
-  p = fmaf(p, ax, -0.9999997019767761f);
-  return fmaf(-ax, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.0f));
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f * 0.70710678118654752440f, ax, 1.0f));
+  float poly = fmaf(0.5f * 1.061405429f, t, 0.5f * -1.453152027f);
+  poly = fmaf(poly, t, 0.5f * 1.421413741f);
+  poly = fmaf(poly, t, 0.5f * -0.284496736f);
+  poly = fmaf(poly, t, 0.5f * 0.254829592f);
+  poly *= t;
+  const float q = poly * __builtin_amdgcn_exp2f((x * (-0.5f * 1.4426950408889634f)) * x);
+  return fmaf(-ax, q, fmaxf(x, 0.0f));
 }
 __device__ __forceinline__ float gelu_tanh(float x) {
   // 0.5 x (1 + tanh(u)) = x * sigmoid(2u),  u = sqrt(2/pi) (x + 0.044715 x^3)
