@@ -136,17 +136,6 @@ __device__ __forceinline__ void store4_stream(void *p, uint32_t v) {
   __builtin_nontemporal_store(v, (ARCTIC_GLOBAL uint32_t *)p);
 }
 
-// Stores written through the L2 of the XCD into the memory-side cache (the scope of a store that other XCDs see).  The
-// 16-byte one has no builtin; its registers may be written again two cycles behind it, which the compiler sees to for its
-// own stores only.
-__device__ __forceinline__ void store8_through(void *p, const uint2 &v) {
-  __hip_atomic_store((ARCTIC_GLOBAL uint64_t *)p, ((uint64_t)v.y << 32) | v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void store16_through(void *p, const uint4 &v) {
-  const u32x4 t = {v.x, v.y, v.z, v.w};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"((ARCTIC_GLOBAL u32x4 *)p), "v"(t) : "memory");
-}
-
 // The same for addresses that are only element-aligned (rows of odd widths or pitches): still one 16-byte access per
 // lane, which the memory pipeline takes at any alignment; a wave's accesses then touch one 128-byte line more.
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));

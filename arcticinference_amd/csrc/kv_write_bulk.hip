@@ -15,7 +15,13 @@
 // consecutive lanes cover consecutive addresses along head_size, and the cache
 // row is written with 16-byte (copy) or 8-byte (fp8, 8 codes) stores.  Source
 // and destination are each touched exactly once, so both use streaming
-// (non-temporal) accesses.
+// (non-temporal) accesses.  Stores written through the L2 instead end in the
+// 256 MB memory-side cache and leave the launch sooner (5003 tokens x 33 layers
+// of 3 x 96 to fp8, launch behind launch: 58 us against 70), but the work behind
+// the launch then waits for those lines to reach HBM.  What a launch adds to a
+// step that goes on to read 1.05 GB of weights, streaming / through: that launch
+// 72 / 91 us, 1024 x 33 of it 16.2 / 22.9, 512 x 40 of 8 x 128 24.8 / 33.7,
+// 1024 x 40 48.5 / 59.2, 1024 x 16 as they are 26.8 / 37.7.
 //
 // The four per-layer pointer tables travel in the kernel-argument segment, so a
 // call uploads nothing and can be recorded into a HIP graph.
@@ -113,27 +119,25 @@ struct SrcF32 {
 
 struct Copy {};  // ARCTIC_KV_AUTO
 
-template <typename F8, bool kThrough>
+template <typename F8>
 __device__ __forceinline__ void quantize_store(char *dst, const float (&f)[8], double inv) {
   uint2 out;
   out.x = encode4<F8>(div_by_scale(f[0], inv), div_by_scale(f[1], inv),
                       div_by_scale(f[2], inv), div_by_scale(f[3], inv));
   out.y = encode4<F8>(div_by_scale(f[4], inv), div_by_scale(f[5], inv),
                       div_by_scale(f[6], inv), div_by_scale(f[7], inv));
-  if constexpr (kThrough) store8_through(dst, out);
-  else store8_stream(dst, out);
+  store8_stream(dst, out);
 }
 
 // One 16-byte source chunk -> cache.  `col` is the chunk's index inside its row.
-template <typename Src, typename Dst, bool kThrough>
+template <typename Src, typename Dst>
 __device__ __forceinline__ void emit_chunk(const uint4 &v, const RowDesc &d, int col) {
   if constexpr (std::is_same<Dst, Copy>::value) {
-    if constexpr (kThrough) store16_through(d.dst + (int64_t)col * 16, v);
-    else store16_stream(d.dst + (int64_t)col * 16, v);
+    store16_stream(d.dst + (int64_t)col * 16, v);
   } else if constexpr (Src::kElemsPerChunk == 8) {
     float f[8];
     Src::to_float(v, f);
-    quantize_store<Dst, kThrough>(d.dst + (int64_t)col * 8, f, d.inv);
+    quantize_store<Dst>(d.dst + (int64_t)col * 8, f, d.inv);
   } else {
     const uint32_t w = encode4<Dst>(div_by_scale(__uint_as_float(v.x), d.inv),
                                     div_by_scale(__uint_as_float(v.y), d.inv),
@@ -204,8 +208,7 @@ __device__ __forceinline__ void select_leftover_rows(const BulkParams &p, unsign
 // kBulkThreads x kUnroll 16-byte chunks form one batch of a workgroup.  Three shapes are built, all with batches
 // of 1024 chunks: 1024 x 1 (launches of more than 8192 tokens: a workgroup moves up to five batches), 512 x 2 (the
 // same launches when rows are selected as well) and 256 x 4 (everything smaller: one or two batches per workgroup).
-// kThrough: cache rows are stored through the L2 instead of streaming (bulk_entry says when).
-template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, bool kThrough>
+template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect>
 __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables &tab, unsigned block) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
   constexpr int kDstElemBytes = kCopy ? Src::kBytes : 1;
@@ -345,7 +348,7 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
       if (cu < total) {
         int r, col;
         locate(cu, r, col);
-        if (!kSelect || to_cache) emit_chunk<Src, Dst, kThrough>(cur[u], rows[r], col);
+        if (!kSelect || to_cache) emit_chunk<Src, Dst>(cur[u], rows[r], col);
         if constexpr (kSelect == kSelectByRowMap) {
           if (to_out) store16_stream(((r & 1) ? vout : kout) + ((int64_t)(r >> 1) * cpr + col) * 16, cur[u]);
         }
@@ -366,10 +369,10 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
   }
 }
 
-template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, bool kThrough>
+template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect>
 __global__ __launch_bounds__(kBulkThreads) void kv_write_bulk_kernel(
     const BulkParams p, const LayerTables tab) {
-  bulk_item<Src, Dst, kPow2, kBulkThreads, kUnroll, kSelect, kThrough>(p, tab, blockIdx.x);
+  bulk_item<Src, Dst, kPow2, kBulkThreads, kUnroll, kSelect>(p, tab, blockIdx.x);
 }
 
 
@@ -477,42 +480,26 @@ __global__ __launch_bounds__(kScalarThreads) void kv_write_bulk_scalar_kernel(
   }
 }
 
-// How a launch of the vector kernels is shaped (bulk_entry chooses).
-struct Shape {
-  bool wide;      // 1024 or 512 lanes instead of 256
-  bool through;   // cache rows stored through the L2; only with 256 lanes, and not for fp32 to fp8
-};
-
-template <typename Src, typename Dst, bool kPow2, int kSelect>
-static void launch_vec_small(const BulkParams &p, const LayerTables &tab, dim3 g, bool through, hipStream_t s) {
-  if constexpr (std::is_same<Dst, Copy>::value || Src::kBytes == 2) {
-    if (through) {
-      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, kPow2, 256, 4, kSelect, true>), g, dim3(256), 0, s, p, tab);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, kPow2, 256, 4, kSelect, false>), g, dim3(256), 0, s, p, tab);
-}
 template <typename Src, typename Dst, int kSelect>
-static void launch_vec_shape(const BulkParams &p, const LayerTables &tab, int64_t grid, Shape shape, hipStream_t s) {
+static void launch_vec_shape(const BulkParams &p, const LayerTables &tab, int64_t grid, bool wide, hipStream_t s) {
   const dim3 g((unsigned)grid);
   if (p.chunk_shift >= 0) {
-    if (shape.wide && kSelect == kSelectNone)   // the same batch of 1024 chunks by 1024 lanes: 0.5-2 % faster than 512 x 2
-      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 1024, 1, kSelectNone, false>), g, dim3(1024), 0, s, p, tab);
-    else if (shape.wide)
-      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 512, 2, kSelect, false>), g, dim3(512), 0, s, p, tab);
+    if (wide && kSelect == kSelectNone)   // the same batch of 1024 chunks by 1024 lanes: 0.5-2 % faster than 512 x 2
+      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 1024, 1, kSelectNone>), g, dim3(1024), 0, s, p, tab);
+    else if (wide)
+      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 512, 2, kSelect>), g, dim3(512), 0, s, p, tab);
     else
-      launch_vec_small<Src, Dst, true, kSelect>(p, tab, g, shape.through, s);
+      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 256, 4, kSelect>), g, dim3(256), 0, s, p, tab);
   } else {
-    launch_vec_small<Src, Dst, false, kSelect>(p, tab, g, shape.through, s);
+    hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, false, 256, 4, kSelect>), g, dim3(256), 0, s, p, tab);
   }
 }
 template <typename Src, typename Dst>
-static void launch_vec(const BulkParams &p, const LayerTables &tab, int64_t grid, Shape shape, hipStream_t s) {
+static void launch_vec(const BulkParams &p, const LayerTables &tab, int64_t grid, bool wide, hipStream_t s) {
   switch (p.select_mode) {
-    case kSelectByScan: launch_vec_shape<Src, Dst, kSelectByScan>(p, tab, grid, shape, s); break;
-    case kSelectByRowMap: launch_vec_shape<Src, Dst, kSelectByRowMap>(p, tab, grid, shape, s); break;
-    default: launch_vec_shape<Src, Dst, kSelectNone>(p, tab, grid, shape, s); break;
+    case kSelectByScan: launch_vec_shape<Src, Dst, kSelectByScan>(p, tab, grid, wide, s); break;
+    case kSelectByRowMap: launch_vec_shape<Src, Dst, kSelectByRowMap>(p, tab, grid, wide, s); break;
+    default: launch_vec_shape<Src, Dst, kSelectNone>(p, tab, grid, wide, s); break;
   }
 }
 template <typename SrcElem, typename Dst>
@@ -523,13 +510,13 @@ static void launch_scalar(const BulkParams &p, const LayerTables &tab, int64_t g
 }
 
 template <typename Dst>
-static void dispatch_src(bool vec, Shape shape, int src_dtype, const BulkParams &p, const LayerTables &tab,
+static void dispatch_src(bool vec, bool wide, int src_dtype, const BulkParams &p, const LayerTables &tab,
                          int64_t grid, hipStream_t s) {
   if (vec) {
     switch (src_dtype) {
-      case ARCTIC_DTYPE_BF16: launch_vec<SrcBF16, Dst>(p, tab, grid, shape, s); break;
-      case ARCTIC_DTYPE_F16: launch_vec<SrcF16, Dst>(p, tab, grid, shape, s); break;
-      default: launch_vec<SrcF32, Dst>(p, tab, grid, shape, s); break;
+      case ARCTIC_DTYPE_BF16: launch_vec<SrcBF16, Dst>(p, tab, grid, wide, s); break;
+      case ARCTIC_DTYPE_F16: launch_vec<SrcF16, Dst>(p, tab, grid, wide, s); break;
+      default: launch_vec<SrcF32, Dst>(p, tab, grid, wide, s); break;
     }
   } else {
     if (src_dtype == ARCTIC_DTYPE_F32)
@@ -730,21 +717,6 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       } else {
         groups = (int)std::max<int64_t>(1, std::min<int64_t>(count, (2048 + num_tokens - 1) / num_tokens));
       }
-      // Streaming stores or stores through the L2.  Streaming (non-temporal) ones end in HBM; those through the L2 end in
-      // the 256 MB memory-side cache, which also puts partial lines together (rows that are no multiple of 128 bytes),
-      // and leave nothing dirty in the L2 for the end of the launch to write back.  Us per launch, streaming / through:
-      //  - between other work that moves a GB: 1024 tokens x 40 layers of 8 x 128 to fp8 51.3 / 43.0, 1024 x 16 bf16 as
-      //    they are 29.0 / 24.1, 5003 x 33 of 3 x 96 to fp8 75.9 / 59.4; the same way up to 180 MB written;
-      //  - three launches in turn, which share the cache: 2560 x 16 of 8 x 128 48.2 / 42.5, 128 x 16 4.5 / 3.6, 5003 x 33
-      //    of 3 x 96 70.5 / 59.5; level at about 110 MB written each (5003 x 40 of 3 x 96 88.9 / 87.9), slower beyond
-      //    (8192 x 40 of 3 x 96 145 / 162), hence the upper limit.  Whole lines of 10 to 19 MB stay in the 32 MB of L2s
-      //    when they stream and go on streaming (224 x 16 bf16 as they are 5.6 / 5.7, 179 x 40 to fp8 8.9 / 10.0).
-      // fp32 to fp8, 4 bytes per lane, is level at every size and streams.
-      constexpr int64_t kMostThrough = (int64_t)96 << 20, kInL2Low = (int64_t)8 << 20, kInL2High = (int64_t)20 << 20;
-      const int64_t per_token = (int64_t)2 * count * n * des;
-      const bool whole_lines = (int64_t)n * des % 128 == 0 && block_stride * des % 128 == 0;
-      const bool in_l2 = whole_lines && num_tokens > kInL2Low / per_token && num_tokens <= kInL2High / per_token;
-      const Shape shape = {wide, !wide && num_tokens <= kMostThrough / per_token && !in_l2};
       p.layers_per_group = (count + groups - 1) / groups;
       p.groups_per_token = (count + p.layers_per_group - 1) / p.layers_per_group;
       p.by_chunks = Divisor((uint32_t)std::max(1, p.chunks_per_row));
@@ -760,9 +732,9 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       if (pass == 0) continue;
 
       switch (kv_cache_dtype) {
-        case ARCTIC_KV_AUTO: dispatch_src<Copy>(vec, shape, src_dtype, p, tab, grid, s); break;
-        case ARCTIC_KV_FP8_E4M3: dispatch_src<E4M3>(vec, shape, src_dtype, p, tab, grid, s); break;
-        default: dispatch_src<E5M2>(vec, shape, src_dtype, p, tab, grid, s); break;
+        case ARCTIC_KV_AUTO: dispatch_src<Copy>(vec, wide, src_dtype, p, tab, grid, s); break;
+        case ARCTIC_KV_FP8_E4M3: dispatch_src<E4M3>(vec, wide, src_dtype, p, tab, grid, s); break;
+        default: dispatch_src<E5M2>(vec, wide, src_dtype, p, tab, grid, s); break;
       }
       const int rc = check_launch(fn);
       if (rc) return rc;

@@ -58,9 +58,8 @@ def test_flashinfer_layout_and_row_pitch(ops, kv):
     ("fp8", dict(L=16, H=8, D=128), 8 << 20), ("fp8", dict(L=16, H=8, D=128), 20 << 20), ("auto", dict(L=64, H=8, D=128), 20 << 20),
     ("auto", dict(L=16, H=8, D=128), 96 << 20), ("fp8_e5m2", dict(L=64, H=3, D=80), 96 << 20)])
 @pytest.mark.parametrize("beyond", [0, 1])
-def test_both_sides_of_the_store_rule(ops, kv, shape, limit, beyond):
-    """The largest launch whose rows are stored one way and the smallest one stored the other way, whole and partial
-    128-byte lines, 16- and 8-byte stores."""
+def test_launches_of_8_to_96_mebibytes(ops, kv, shape, limit, beyond):
+    """Middling launches of whole and partial 128-byte lines, 16- and 8-byte stores, and one token more."""
     T = limit // (2 * shape["L"] * shape["H"] * shape["D"] * (2 if kv == "auto" else 1)) + beyond
     run_both(ops, make_bulk_case(T=T, bs=16, NB=T // 16 + 2, kv_cache_dtype=kv, seed=17, std=1.5, pad_fraction=0.05, **shape))
 
