@@ -12,8 +12,8 @@
 // sum_lstm_staged_kernel (rows of up to 8192 elements: the nine loads are
 // requested in stages, between the stages of the arithmetic, one chunk per lane),
 // sum_lstm_vec_kernel (rows of up to 16384 elements: two chunks per lane, the
-// loads requested together) and sum_lstm_scalar_kernel (what is left: very short
-// rows that are not 16-byte aligned and more than 16384 elements, element by element).
+// loads requested together) and sum_lstm_scalar_kernel (what is left: short rows
+// that are not 16-byte aligned and more than 16384 elements, element by element).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -411,10 +411,12 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
   // 19.9 / 22.5 us with two chunks per lane in the other kernel; without scale and shift 512 rows of 4096 / 8192: 9.6 /
   // 17.3 us against 11.0 / 24.1 us).  Rows that are not 16-byte aligned take the same kernels with accesses at any
   // alignment, which cost 6 to 35 % over aligned ones (300 rows of 1536: 5.3 us aligned, 5.8 us 4-byte and 6.4 us 2-byte
-  // aligned) and are 3 to 5 times faster than element by element (23 us; 300 rows of 4096: 10.9 against 58 us).  Below
-  // 128 elements a single wave does a row's whole arithmetic and the element-wise kernel's 256 lanes are level or ahead
-  // (300 rows of 36 / 100 / 260 elements: 3.5 / 4.0 / 6.0 us element by element, 4.2 / 4.3 / 4.4 us in chunks).
-  constexpr int kShortRow = 128;
+  // aligned) and are 3 to 5 times faster than element by element (23 us; 300 rows of 4096: 10.9 against 58 us).  Up to 256
+  // elements the element-wise kernel gives every element a lane of its own where one to four half-idle waves would do a
+  // row's whole arithmetic in chunks (us element by element / in chunks, rows x elements, without vectors: 64 x 128 2.67 /
+  // 3.30, 512 x 128 3.01 / 3.87, 64 x 256 2.77 / 3.27, 4096 x 256 8.7 / 9.5; with all of them 512 x 128 3.31 / 3.88, 64 x
+  // 256 3.07 / 3.24); with all vectors and more than 256 rows it is chunks from 129 on (300 x 136 level, 512 x 160 7 % and
+  // 2048 x 256 8 % faster).  From 257 on chunks are faster at every row count (64 x 257 by 10 to 23 %, 64 x 513 by 21 to 35).
 #define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND) \
   hipLaunchKernelGGL((sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND>), grid, dim3(lanes), 0, s, p)
 #define ARCTIC_LSTM_STAGED(KIND)                                    \
@@ -422,8 +424,9 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
     if (p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND);        \
     else ARCTIC_LSTM_STAGED_LAUNCH(true, KIND);                     \
   } while (0)
-  if (p.D >= (aligned ? 8 : kShortRow) && chunks <= 1024) {
-    const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
+  const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
+  const bool element_wise = !aligned && p.D <= (all_vectors && rows > 256 ? 128 : 256);
+  if (!element_wise && chunks <= 1024) {
     if (!aligned || !all_vectors) ARCTIC_LSTM_STAGED(kAnyRow);
     else if (lanes != chunks) ARCTIC_LSTM_STAGED(kRagged);
     else ARCTIC_LSTM_STAGED(kFullWaves);

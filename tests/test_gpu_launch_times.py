@@ -57,3 +57,34 @@ def test_a_write_costs_a_step_what_it_takes(ops, tokens, layers, heads, head_siz
     t = times({"product": product}, 12)
     t.update(times({"write": lambda k: writes[k % 4](), "step": step}, 12))
     assert t["step"] - t["product"] <= 1.2 * t["write"], t
+
+
+def graph_of(calls, per_replay=60):
+    """A captured graph of `per_replay` calls, the given ones in turn."""
+    for call in calls:
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for k in range(per_replay):
+            calls[k % len(calls)]()
+    return lambda _: graph.replay()
+
+
+def gates(ops, rows, width, pad, vectors):
+    """Captured calls of sum_lstm over three sets of rows `pad` elements apart."""
+    def pitched(columns):
+        return torch.randn(rows, columns + pad, device=DEV, dtype=torch.bfloat16)[:, :columns]
+
+    given = [torch.randn(width, device=DEV, dtype=torch.bfloat16) if k in vectors else None for k in range(4)]
+    cell = pitched(width)
+    sets = [(pitched(4 * width), pitched(4 * width)) for _ in range(3)]
+    return graph_of([lambda s=s, z=z: ops.sum_lstm(s, z, cell, *given, 0.35, 1e-6, 1e-6, False) for s, z in sets])
+
+
+@pytest.mark.parametrize("rows", [64, 512])
+def test_a_narrow_unaligned_row_has_a_lane_per_element(ops, rows):
+    """Rows of 128 elements at an odd pitch cost what rows of 127 do; in chunks of 8 elements they cost 1.2 to 1.3 times
+    that."""
+    t = times({"128": gates(ops, rows, 128, 3, ()), "127": gates(ops, rows, 127, 3, ())}, 4)
+    assert t["128"] <= 1.12 * t["127"], t

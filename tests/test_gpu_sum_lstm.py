@@ -319,8 +319,8 @@ def test_staged_kernel_shapes(ops, D, rows, dtype):
 
 @pytest.mark.parametrize("D,pad4,padD", [(8, 1, 3), (127, 0, 0), (128, 1, 1), (129, 3, 2), (513, 0, 0), (1023, 1, 0), (1024, 0, 3),
                                          (1537, 3, 3), (4100, 0, 0), (8191, 2, 1), (8193, 0, 0), (12289, 1, 3), (16383, 0, 0),
-                                         (16385, 0, 0)])
-@pytest.mark.parametrize("rows", [2, 67])
+                                         (16385, 0, 0), (200, 1, 3), (256, 3, 3), (257, 0, 0)])
+@pytest.mark.parametrize("rows", [2, 67, 257])
 def test_rows_that_are_not_16_byte_aligned(ops, D, pad4, padD, rows):
     """Odd widths and pitches in chunks of 8 whose last one overlaps the one before it, on both sides of every change of
     kernel: against the oracle, with and without vectors, and nothing written outside the rows."""
