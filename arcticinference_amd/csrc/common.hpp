@@ -184,6 +184,7 @@ struct Chunk {
 struct Place {
   uint32_t off;   // bytes from the row's start
   int repeated;
+  Place() = default;
   __device__ __forceinline__ Place(int chunk, int D) {
     const int start = min(chunk * Chunk::kElems, D - Chunk::kElems);
     off = (uint32_t)start * 2;

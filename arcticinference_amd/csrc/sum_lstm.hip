@@ -11,8 +11,8 @@
 // Sums are DPP wave reductions plus an LDS combine.  Three kernels:
 // sum_lstm_staged_kernel (rows of up to 8192 elements: the nine loads are
 // requested in stages, between the stages of the arithmetic, one chunk per lane),
-// sum_lstm_vec_kernel (rows of up to 16384 elements: two chunks per lane, the
-// loads requested together) and sum_lstm_scalar_kernel (what is left: short rows
+// sum_lstm_vec_kernel (the loads requested together: rows of up to 16384 elements
+// with two chunks per lane, and short ones without all vectors) and sum_lstm_scalar_kernel (what is left: short rows
 // that are not 16-byte aligned and more than 16384 elements, element by element).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -75,33 +75,42 @@ __device__ __forceinline__ Chunk load_shift(const char *b, uint32_t off) {
   return Chunk::load<true>((b ? b : (const char *)kChunkOfZeros) + (b ? off : 0u));
 }
 
-// Rows beyond one chunk per lane of 1024 lanes.  Loads are issued in the order in which the arithmetic needs them -
+// Rows beyond one chunk per lane of 1024 lanes, with two of them, and aligned rows of up to 2048 elements that lack a
+// scale or shift vector, with one (launch_lstm has the rule).  Loads are issued in the order in which the arithmetic needs them -
 // cell gate, forget gate, previous cell, input gate, output gate - and memory returns them in that order, so the first
 // row sum, the candidate GELU and the early sigmoids run while the later gates are still on their way, and only one
 // sigmoid, one multiply and the store remain after the last load has landed.
+// kBare: none of the four vectors is given, and nothing stands in for them (us per call in a graph, ones and zeros read /
+// not read: 64 rows of 12288 with one z for all gates 10.9 / 9.9, 300 of 16384 29.0 / 26.4).
 template <int K>
 struct LstmRow {
   Chunk sc[K], zc[K], sf[K], zf[K], si[K], zi[K], pc[K], so[K], zo[K];
 };
 
-template <typename T, bool kFastGelu, bool kSharedZ, bool kAnyAlignment>
-__global__ __launch_bounds__(1024) void sum_lstm_vec_kernel(const LstmParams p) {
+template <typename T, int K, bool kFastGelu, bool kSharedZ, bool kAnyAlignment, bool kBare>
+__global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const LstmParams p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
-  constexpr int K = 2;
   constexpr int E = Chunk::kElems;
   using C = Chunk;
   const int D = p.D;
   const int64_t gate_bytes = (int64_t)D * 2;
-  const Place at[K] = {Place(threadIdx.x, D), Place(threadIdx.x + blockDim.x, D)};
+  Place at[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) at[k] = Place(threadIdx.x + k * blockDim.x, D);
   auto load = [](const char *q) { return C::load_stream<kAnyAlignment>(q); };
+  auto vector = [](const C &given, float (&f)[E], float absent) {
+    if constexpr (!kBare) given.template unpack<T>(f);
+#pragma unroll
+    for (int j = 0; j < E && kBare; ++j) f[j] = absent;
+  };
 
   C wc[K], bc[K], ws[K], bs[K];
   // The scale / shift vectors are the same for every row (cache resident).  They
   // are requested first: memory returns loads in issue order, so asking for them
   // later would park the arithmetic behind the whole row.
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
+  for (int k = 0; k < K && !kBare; ++k) {
     wc[k] = load_scale<T, true>(p.w_cell, at[k].off);
     bc[k] = load_shift<true>(p.b_cell, at[k].off);
     ws[k] = load_scale<T, true>(p.w_state, at[k].off);
@@ -163,8 +172,8 @@ __global__ __launch_bounds__(1024) void sum_lstm_vec_kernel(const LstmParams p) 
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     float w[E], b[E];
-    wc[k].template unpack<T>(w);
-    bc[k].template unpack<T>(b);
+    vector(wc[k], w, 1.f);
+    vector(bc[k], b, 0.f);
 #pragma unroll
     for (int j = 0; j < E; ++j) cact[k][j] = gelu<kFastGelu>(fmaf(cact[k][j] * inv_cpre, w[j], b[j]));
   }
@@ -203,8 +212,8 @@ __global__ __launch_bounds__(1024) void sum_lstm_vec_kernel(const LstmParams p) 
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     float w[E], b[E], st[E], a[E], g[E];
-    ws[k].template unpack<T>(w);
-    bs[k].template unpack<T>(b);
+    vector(ws[k], w, 1.f);
+    vector(bs[k], b, 0.f);
 #pragma unroll
     for (int j = 0; j < E; ++j) st[j] = gelu<kFastGelu>(fmaf(cell[k][j] * inv_cnew, w[j], b[j]));
     r.so[k].template unpack<T>(a);
@@ -426,19 +435,33 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
   } while (0)
   const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
   const bool element_wise = !aligned && p.D <= (all_vectors && rows > 256 ? 128 : 256);
-  if (!element_wise && chunks <= 1024) {
+  // Aligned rows of up to 2048 elements that lack a vector: at most four waves per row, whose loads are few enough to be
+  // requested together.  Us per call in a graph, in stages (ones and zeros read in place of an absent vector) / together:
+  // 64 x 256 without vectors 4.0 / 3.2, 512 x 512 4.2 / 3.3, 300 x 2048 5.6 / 4.8, 512 x 512 with the scales alone 4.1 / 3.4;
+  // from 513 elements and 513 rows on the stages are faster (2048 x 1024 8.8 / 9.4), but for one z for all gates (8.4 / 7.7).
+  const bool together = aligned && !all_vectors && chunks <= 256 && (chunks <= 64 || rows <= 512 || kSharedZ);
+#define ARCTIC_LSTM_VEC_LAUNCH(K, ANY, BARE) \
+  hipLaunchKernelGGL((sum_lstm_vec_kernel<T, K, kFastGelu, kSharedZ, ANY, BARE>), grid, dim3(threads), 0, s, p)
+#define ARCTIC_LSTM_VEC(K, ANY)                                       \
+  do {                                                                \
+    const int threads = ((chunks + (K) - 1) / (K) + 63) & ~63;        \
+    if (p.w_cell || p.b_cell || p.w_state || p.b_state) ARCTIC_LSTM_VEC_LAUNCH(K, ANY, false); \
+    else ARCTIC_LSTM_VEC_LAUNCH(K, ANY, true);                        \
+  } while (0)
+  if (together) {
+    ARCTIC_LSTM_VEC(1, false);
+  } else if (!element_wise && chunks <= 1024) {
     if (!aligned || !all_vectors) ARCTIC_LSTM_STAGED(kAnyRow);
     else if (lanes != chunks) ARCTIC_LSTM_STAGED(kRagged);
     else ARCTIC_LSTM_STAGED(kFullWaves);
   } else if (chunks > 1024 && chunks <= 2 * 1024) {
-    const int threads = (((chunks + 1) / 2) + 63) & ~63;
-    if (aligned)
-      hipLaunchKernelGGL((sum_lstm_vec_kernel<T, kFastGelu, kSharedZ, false>), grid, dim3(threads), 0, s, p);
-    else
-      hipLaunchKernelGGL((sum_lstm_vec_kernel<T, kFastGelu, kSharedZ, true>), grid, dim3(threads), 0, s, p);
+    if (aligned) ARCTIC_LSTM_VEC(2, false);
+    else ARCTIC_LSTM_VEC(2, true);
   } else {
     hipLaunchKernelGGL((sum_lstm_scalar_kernel<T, kFastGelu>), grid, dim3(256), 0, s, p, kSharedZ ? 0 : p.D);
   }
+#undef ARCTIC_LSTM_VEC
+#undef ARCTIC_LSTM_VEC_LAUNCH
 #undef ARCTIC_LSTM_STAGED
 #undef ARCTIC_LSTM_STAGED_LAUNCH
 }

@@ -348,3 +348,24 @@ def test_rows_that_are_not_16_byte_aligned(ops, D, pad4, padD, rows):
         assert_close(got[1:-1, 5:5 + D], want, RTOL, ATOL)
         got[1:-1, 5:5 + D] = 7.0
         assert torch.equal(got, guard)
+
+
+@pytest.mark.parametrize("D,rows", [(8, 513), (504, 1), (512, 600), (520, 512), (520, 513), (2040, 3), (2048, 512), (2048, 513),
+                                    (2056, 2), (8192, 2), (8200, 3), (16384, 2), (16383, 2)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_absent_vectors_equal_ones_and_zeros(ops, D, rows, dtype):
+    """None of the four vectors, or the shifts alone missing: bit for bit what ones and zeros in their place give, on both
+    sides of every change of kernel, with and without a previous cell, with one z for all gates and with four; and within
+    the tolerance of the oracle."""
+    c = make_lstm_case(rows=rows, D=D, dtype=dtype, seed=D + rows, wb_cell=False, wb_state=False, repeat_z=True)
+    d = {k: dev(v) for k, v in c.items() if v is not None}
+    ones, zeros = torch.ones(D, dtype=dtype, device=DEV), torch.zeros(D, dtype=dtype, device=DEV)
+    scale = torch.randn(D, generator=torch.Generator().manual_seed(D)).to(dtype).to(DEV)
+    tail = (0.35, 1e-6, 1e-5, False)
+    z = d["z4"][:, :D]
+    for cell in (d["prev_cell"], None):
+        for absent, full in (((None,) * 4, (ones, zeros, ones, zeros)), ((scale, None, scale, None), (scale, zeros, scale, zeros))):
+            for op, z_given in ((ops.sum_lstm, d["z4"]), (ops.sum_lstm_shared_z, z)):
+                got, want = (op(d["states"], z_given, cell, *v, *tail) for v in (absent, full))
+                assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    run(ops, c, alpha=0.35)
