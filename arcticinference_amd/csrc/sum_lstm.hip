@@ -403,6 +403,22 @@ __global__ __launch_bounds__(256) void sum_lstm_scalar_kernel(const LstmParams p
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
+// Whether an output shares memory with a gate or the previous cell: `columns` elements of each of `rows` rows, `stride`
+// elements apart, looked at as whole ranges.
+static bool in_place(const LstmParams &p, int64_t rows, bool shared_z) {
+  const auto overlaps = [&](const char *out, const char *in, int64_t in_rows, int64_t stride, int64_t columns) {
+    const uintptr_t o = (uintptr_t)out, i = (uintptr_t)in;
+    return in && o < i + (uintptr_t)((in_rows - 1) * stride + columns) * 2 &&
+           i < o + (uintptr_t)((rows - 1) * p.out_stride + p.D) * 2;
+  };
+  const int64_t gates = 4 * (int64_t)p.D;
+  for (const char *out : {p.out_state, p.out_cell})
+    if (overlaps(out, p.states, rows, p.s_stride, gates) || overlaps(out, p.prev_cell, rows, p.pc_stride, p.D) ||
+        overlaps(out, p.z4, p.z_index ? p.z_rows : rows, p.z_stride, shared_z ? p.D : gates))
+      return true;
+  return false;
+}
+
 template <typename T, bool kFastGelu, bool kSharedZ>
 static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
   const bool multi = rows > 1;
@@ -434,7 +450,13 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
     else ARCTIC_LSTM_STAGED_LAUNCH(true, KIND);                     \
   } while (0)
   const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
-  const bool element_wise = !aligned && p.D <= (all_vectors && rows > 256 ? 128 : 256);
+  const bool narrow = !aligned && p.D <= (all_vectors && rows > 256 ? 128 : 256);
+  // A call that updates a tensor in place relies on every element being read before it is written.  In a width that is no
+  // multiple of 8 two lanes, at some widths (513, 1537) of two waves, read the last elements of a row and both store them,
+  // and nothing orders the one's load before the other's store: such a call goes element by element.  Aligned rows that
+  // lack a vector are requested together, since the stages read the output gate behind the first store.
+  const bool aliased = (p.D % 8 || !all_vectors) && in_place(p, rows, kSharedZ);
+  const bool element_wise = narrow || (aliased && p.D % 8);
   // Aligned rows of up to 2048 elements that lack a vector: at most four waves per row, whose loads are few enough to be
   // requested together.  Us per call in a graph, in stages (ones and zeros read in place of an absent vector) / together:
   // 64 x 256 without vectors 4.0 / 3.2, 512 x 512 4.2 / 3.3, 300 x 2048 5.6 / 4.8, 512 x 512 with the scales alone 4.1 / 3.4;
@@ -450,11 +472,13 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
   } while (0)
   if (together) {
     ARCTIC_LSTM_VEC(1, false);
+  } else if (aliased && aligned && chunks <= 2 * 1024) {
+    ARCTIC_LSTM_VEC(2, false);
   } else if (!element_wise && chunks <= 1024) {
     if (!aligned || !all_vectors) ARCTIC_LSTM_STAGED(kAnyRow);
     else if (lanes != chunks) ARCTIC_LSTM_STAGED(kRagged);
     else ARCTIC_LSTM_STAGED(kFullWaves);
-  } else if (chunks > 1024 && chunks <= 2 * 1024) {
+  } else if (!element_wise && chunks > 1024 && chunks <= 2 * 1024) {
     if (aligned) ARCTIC_LSTM_VEC(2, false);
     else ARCTIC_LSTM_VEC(2, true);
   } else {

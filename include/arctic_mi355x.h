@@ -307,7 +307,8 @@ int arctic_speculator_embed_add_ln_act(void *out, const void *in, const void *em
  *   prev_cell      device; rows of D elements, pc_stride apart.  NULL = a cell of zeros, which is what the
  *                  speculator starts every proposal round from (arctic_speculator.py:899-903): the result is that
  *                  of a zero tensor bit for bit, without the tensor, its clearing or its read; pc_stride is ignored
- *   out_state, out_cell   device; rows of D elements, out_stride apart
+ *   out_state, out_cell   device; rows of D elements, out_stride apart.  out_cell may be prev_cell itself (the same
+ *                  address and pitch), which updates the cell in place
  *   w_cell, b_cell, w_state, b_state   device [>= D] or NULL
  * All strides are in ELEMENTS.  dtype is F16 or BF16.
  */

@@ -369,3 +369,27 @@ def test_absent_vectors_equal_ones_and_zeros(ops, D, rows, dtype):
                 got, want = (op(d["states"], z_given, cell, *v, *tail) for v in (absent, full))
                 assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     run(ops, c, alpha=0.35)
+
+
+@pytest.mark.parametrize("D,rows,vectors,into", [
+    (513, 300, True, "cell"), (1537, 300, False, "cell"), (8193, 40, True, "cell"), (300, 20, False, "cell"),   # widths of no multiple of 8
+    (1024, 600, False, "output gate"), (4096, 64, False, "output gate"), (8192, 3, False, "output gate"),        # no vectors
+    (4096, 64, True, "cell")])
+def test_updates_in_place(ops, D, rows, vectors, into):
+    """Through the C entry point the new cell may be stored over the previous one, and, without vectors, over the output
+    gate: the results are the oracle's."""
+    dtype = torch.bfloat16
+    c = make_lstm_case(rows=rows, D=D, dtype=dtype, seed=D, wb_cell=vectors, wb_state=vectors)
+    want_s, want_c = oracle.sum_lstm(c["states"], c["z4"], c["prev_cell"], c["w_cell"], c["b_cell"], c["w_state"], c["b_state"],
+                                     0.35, 1e-6, 1e-6, False)
+    d = {k: dev(v) for k, v in c.items()}
+    pitch = D if into == "cell" else 4 * D
+    cell = d["prev_cell"] if into == "cell" else d["states"][:, 2 * D:3 * D]
+    state = torch.empty(rows, pitch, dtype=dtype, device=DEV)[:, :D]
+    ptr = lambda t: None if t is None else t.data_ptr()
+    _native.check(_native.load().arctic_sum_lstm(
+        state.data_ptr(), cell.data_ptr(), ptr(d["states"]), ptr(d["z4"]), ptr(d["prev_cell"]), ptr(d["w_cell"]), ptr(d["b_cell"]),
+        ptr(d["w_state"]), ptr(d["b_state"]), rows, D, 4 * D, 4 * D, D, pitch, 0.35, 1e-6, 1e-6, 0, _native.DTYPE_BF16,
+        torch.cuda.current_stream().cuda_stream))
+    assert_close(cell, want_c, RTOL, ATOL, "cell")
+    assert_close(state, want_s, RTOL, ATOL, "state")
