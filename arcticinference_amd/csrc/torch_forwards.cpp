@@ -528,7 +528,11 @@ at::Tensor argmax_clamp(const at::Tensor &logits, int64_t max_index) {
   check_rc(arctic_argmax_clamp_split((int64_t *)out.data_ptr(), in_2d.data_ptr(), rows, (int)cols, in_2d.stride(0), max_index,
                                      code, workspace ? (int64_t *)out.data_ptr() + rows : nullptr, workspace,
                                      current_stream()));
-  if (workspace) out.resize_(shape);   // keeps the memory
+  if (workspace) {
+    // the answers keep the block, but what a caller saves, shares or looks at is their own size
+    out.resize_(shape);
+    out.storage().set_nbytes((size_t)rows * sizeof(int64_t));
+  }
   return out;
 }
 

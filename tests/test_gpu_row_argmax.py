@@ -175,3 +175,19 @@ def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
         static.copy_(x[:, :cols])
         graph.replay()
         assert torch.equal(got.cpu(), reference(x[:, :cols], cols - 1))
+
+
+@pytest.mark.parametrize("shape", [(3, 128256), (2, 2, 100000), (4, 1000)])
+def test_the_result_is_the_answers_alone(ops, shape, tmp_path):
+    """What the workgroups of a split row exchange is no part of the tensor's storage: it is not saved with it, and the
+    tensor can be resized."""
+    logits = torch.randn(*shape, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16)
+    got = ops.speculator_argmax(logits.to(DEV), shape[-1])
+    want = reference(logits, shape[-1])
+    assert got.untyped_storage().nbytes() == want.numel() * 8
+    torch.save(got, tmp_path / "tokens.pt")
+    saved = torch.load(tmp_path / "tokens.pt", weights_only=True)
+    assert saved.untyped_storage().nbytes() == want.numel() * 8 and torch.equal(saved.cpu(), want)
+    grown = got.clone().resize_(want.numel() + 1000)
+    got.resize_(want.numel() + 1000)[want.numel():] = 0
+    assert torch.equal(got[:want.numel()].cpu(), want.flatten()) and torch.equal(grown[:want.numel()].cpu(), want.flatten())
