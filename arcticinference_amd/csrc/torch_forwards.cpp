@@ -519,11 +519,11 @@ at::Tensor argmax_clamp(const at::Tensor &logits, int64_t max_index) {
   const at::Tensor in_2d = rows_of(logits, cols);
   const int64_t rows = in_2d.size(0);
   const auto shape = logits.sizes().slice(0, logits.dim() - 1);
+  const auto options = logits.options().dtype(at::kLong);
+  if (rows == 0) return at::empty(shape, options);
   // a few long rows are split over workgroups that exchange their winners in memory behind the answers: one allocation
   const int64_t workspace = arctic_argmax_workspace_bytes(rows, to_int(cols, "cols"), code);
-  const auto options = logits.options().dtype(at::kLong);
   at::Tensor out = workspace ? at::empty({rows + (workspace + 7) / 8}, options) : at::empty(shape, options);
-  if (rows == 0) return out;
   const DeviceGuard guard(logits.device());
   check_rc(arctic_argmax_clamp_split((int64_t *)out.data_ptr(), in_2d.data_ptr(), rows, (int)cols, in_2d.stride(0), max_index,
                                      code, workspace ? (int64_t *)out.data_ptr() + rows : nullptr, workspace,

@@ -191,3 +191,8 @@ def test_the_result_is_the_answers_alone(ops, shape, tmp_path):
     grown = got.clone().resize_(want.numel() + 1000)
     got.resize_(want.numel() + 1000)[want.numel():] = 0
     assert torch.equal(got[:want.numel()].cpu(), want.flatten()) and torch.equal(grown[:want.numel()].cpu(), want.flatten())
+
+
+def test_no_rows_of_any_width(ops):
+    got = ops.speculator_argmax(torch.empty(0, 2 ** 31 + 8, device=DEV, dtype=torch.bfloat16), 7)
+    assert got.shape == (0,) and got.dtype == torch.int64
