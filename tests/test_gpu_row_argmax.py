@@ -148,33 +148,67 @@ def test_row_counts_around_the_in_step_kernel(ops, rows, dtype):
     (85, 128257, torch.float16, 0), (86, 128256, torch.bfloat16, 0),   # six workgroups per row, and no longer
     (5, 131103, torch.bfloat16, 3), (3, 40960, torch.float32, 0), (2, 300001, torch.float32, 1)])
 def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
-    """Long rows of a small batch are cut into segments: ties, NaNs and infinities on both sides of the cuts, rows of one
-    value, and a captured graph whose inputs change between replays (the workspace keeps what the last replay left)."""
+    """Long rows of a small batch are cut into segments: single maxima, tied pairs, infinities and NaNs on both sides of
+    the cuts, in the middle and at the ends, another answer every time, in eager calls whose outputs take the blocks of
+    the ones before and in a captured graph whose inputs change between replays (the workspace keeps what the last replay
+    left)."""
     g = torch.Generator().manual_seed(cols)
-    levels = torch.tensor([-float("inf"), -2.0, -0.0, 0.0, 1.5, 3.0])
+    parts = min(16, cols * (2 if dtype == torch.float32 else 1) // 8192, 512 // rows)
+    segment = -(-cols // parts) + 63 & ~63
+    places = [segment, 0, cols - 1, segment - 1, parts // 2 * segment + 17, cols - 2, (parts - 1) * segment]
+    at = lambda r, k: places[(r + k) % len(places)]
+    levels = torch.tensor([-float("inf"), -2.0, -0.0, 0.0, 1.5])
     batches = []
-    for k in range(4):
-        x = levels[torch.randint(0, 4 if k == 1 else 6, (rows, cols + pad), generator=g)].to(dtype)
-        x[0] = -float("inf")
-        if k == 2:
-            for r in range(1, rows):
-                x[r, torch.randint(0, cols, (2,), generator=g)] = float("nan")
-        if k == 3 and rows > 1:
-            x[1] = -7.0
-            x[1, cols - 1] = -6.5
-        batches.append(x)
+    for k in range(9):
+        x = levels[torch.randint(0, 5, (rows, cols + pad), generator=g)]
+        for r in range(rows):
+            if k < 4:      # one maximum
+                x[r, at(r, k)] = 3.0
+            elif k == 4:   # a tied pair
+                x[r, at(r, 0)] = x[r, at(r, 3)] = 3.0
+            elif k == 5:   # infinity, with the other one in its chunk
+                p = at(r, 2)
+                x[r, p ^ 1 if p ^ 1 < cols else p - 1] = -float("inf")
+                x[r, p] = float("inf")
+            elif k == 6:   # NaNs beat infinity, the first one wins
+                x[r, at(r, 1)] = float("inf")
+                x[r, at(r, 2)] = x[r, at(r, 5)] = float("nan")
+            elif k == 7:   # nothing but the lowest value
+                x[r] = -float("inf")
+        batches.append(x.to(dtype))   # the last batch: many equal maxima
+    on_gpu = [x.to(DEV)[:, :cols] for x in batches]
+    for _ in range(2):
+        for x, y in zip(batches, on_gpu):
+            assert torch.equal(ops.speculator_argmax(y, cols).cpu(), reference(x[:, :cols], cols))
     static = torch.empty(rows, cols + pad, dtype=dtype, device=DEV)[:, :cols]
-    static.copy_(batches[0][:, :cols])
-    assert torch.equal(ops.speculator_argmax(static, cols).cpu(), reference(batches[0][:, :cols], cols))
+    static.copy_(on_gpu[0])
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         got = ops.speculator_argmax(static, cols - 1)
     assert got.shape == (rows,) and got.is_contiguous()
-    for x in batches + batches[:2]:
-        static.copy_(x[:, :cols])
+    for x, y in zip(batches + batches[:2], on_gpu + on_gpu[:2]):
+        static.copy_(y)
         graph.replay()
         assert torch.equal(got.cpu(), reference(x[:, :cols], cols - 1))
+
+
+def test_split_rows_on_two_streams_at_once(ops):
+    """Each call exchanges winners in memory of its own: calls of two streams that run at the same time do not meet."""
+    cols = 128256
+    logits = [torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16) for rows in (5, 32)]
+    want = [reference(x, cols) for x in logits]
+    on_gpu = [x.to(DEV) for x in logits]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(60):
+        for k in (0, 1):
+            with torch.cuda.stream(streams[k]):
+                got[k].append(ops.speculator_argmax(on_gpu[k], cols))
+    torch.cuda.synchronize()
+    for k in (0, 1):
+        assert all(torch.equal(t.cpu(), want[k]) for t in got[k])
 
 
 @pytest.mark.parametrize("shape", [(3, 128256), (2, 2, 100000), (4, 1000)])
