@@ -1177,7 +1177,8 @@ def bench_lstm_rows(ops, dev, steps):
 def bench_lstm_widths(ops, dev, steps):
     """sum_lstm at 512 rows against the row width: the kernel that requests a row in stages (all four scale / shift
     vectors given, rows of up to 8192 elements, spare lanes in the last wave when the width is no multiple of 512)
-    next to the general kernel, which the same call takes when a vector is missing (here: the cell norm's pair)."""
+    next to what the same call takes when a vector is missing (here: the cell norm's pair): all loads at once up to 2048
+    elements and beyond 8192, ones and zeros read in the staged kernel between."""
     T = 512
     g = torch.Generator(device=dev).manual_seed(9)
     rn = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)

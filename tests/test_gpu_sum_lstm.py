@@ -289,10 +289,10 @@ def test_saturated_gates_zero_rows_and_extreme_magnitudes(ops, dtype, D):
 def test_staged_kernel_shapes(ops, D, rows, dtype):
     """Rows of up to 8192 elements with all four vectors take the kernel that requests a row in stages (one 16-byte
     chunk per lane; rows that are no multiple of 512 elements leave lanes of the last wave idle): against the oracle
-    with and without a previous cell, with pitched rows and the tanh GELU, and bit for bit against the general kernel,
-    which the same row takes as soon as one vector is missing (an absent scale acts as 1, an absent shift as 0, so
-    ones and zeros in their place change no bit).  Beyond 4096 elements the general kernel gives a lane two chunks, so
-    its row sums add up in another order: there the two are compared within the tolerance."""
+    with and without a previous cell, with pitched rows and the tanh GELU, and bit for bit against what the same row
+    takes as soon as one vector is missing (an absent scale acts as 1, an absent shift as 0, so ones and zeros in their
+    place change no bit): the kernel that requests all of a row at once up to 2048 elements, another instance of the
+    staged one beyond, both with one chunk per lane and so with sums in the same order."""
     pad = 8 if rows > 1 else 0   # pitches stay multiples of 16 bytes
     c = make_lstm_case(rows=rows, D=D, dtype=dtype, seed=900 + D // 8 + rows, pad4=pad, padD=pad)
     for fast in (False, True):
@@ -302,19 +302,15 @@ def test_staged_kernel_shapes(ops, D, rows, dtype):
     tail = (0.35, 1e-6, 1e-5, False)
     for cell in (d["prev_cell"], None):
         def same(a, b):
-            for x, y in zip(a, b):
-                if D <= 4096:
-                    assert torch.equal(x, y)
-                else:
-                    assert_close(x, y, RTOL, ATOL, "staged against general")
+            assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
 
         staged = ops.sum_lstm(d["states"], d["z4"], cell, ones, zeros, d["w_state"], d["b_state"], *tail)
-        general = ops.sum_lstm(d["states"], d["z4"], cell, None, None, d["w_state"], d["b_state"], *tail)
-        same(staged, general)
+        missing = ops.sum_lstm(d["states"], d["z4"], cell, None, None, d["w_state"], d["b_state"], *tail)
+        same(staged, missing)
         z = d["z4"][:, :D].contiguous()
         staged = ops.sum_lstm_shared_z(d["states"], z, cell, d["w_cell"], d["b_cell"], ones, zeros, *tail)
-        general = ops.sum_lstm_shared_z(d["states"], z, cell, d["w_cell"], d["b_cell"], None, None, *tail)
-        same(staged, general)
+        missing = ops.sum_lstm_shared_z(d["states"], z, cell, d["w_cell"], d["b_cell"], None, None, *tail)
+        same(staged, missing)
 
 
 @pytest.mark.parametrize("D,pad4,padD", [(8, 1, 3), (127, 0, 0), (128, 1, 1), (129, 3, 2), (513, 0, 0), (1023, 1, 0), (1024, 0, 3),
@@ -333,19 +329,22 @@ def test_rows_that_are_not_16_byte_aligned(ops, D, pad4, padD, rows):
         z = dev(c["z4"])[:, :D]
         st, ce = ops.sum_lstm_shared_z(dev(c["states"]), z, *args, 0.35, 1e-6, 1e-6, not affine)
         assert torch.equal(st, got_s) and torch.equal(ce, got_c)
-    # a vector that starts one element into its storage, and guards around rows placed inside larger tensors
+    # vectors that start one element into their storage, and guards around rows placed inside larger tensors
+    g = torch.Generator().manual_seed(D)
+    vectors = [torch.randn(D, generator=g).to(dtype) for _ in range(4)]
+    want = oracle.sum_lstm(c["states"], c["z4"], c["prev_cell"], *vectors, 0.35, 1e-6, 1e-6, True)
+    one_off = [torch.cat([v[:1] + 1, v]).to(DEV)[1:] for v in vectors]
     guard = torch.full((rows + 2, D + 9), 7.0, dtype=dtype, device=DEV)
     state, cell = guard.clone(), guard.clone()
     lib = _native.load()
     s, z4 = dev(c["states"]), dev(c["z4"])
     pc = dev(c["prev_cell"])
-    w = torch.ones(D + 1, dtype=dtype, device=DEV)[1:]
     _native.check(lib.arctic_sum_lstm(
-        state[1:, 5:].data_ptr(), cell[1:, 5:].data_ptr(), s.data_ptr(), z4.data_ptr(), pc.data_ptr(), w.data_ptr(), None, None,
-        None, rows, D, s.stride(0), z4.stride(0), pc.stride(0), D + 9, 0.35, 1e-6, 1e-6, 1,
+        state[1:, 5:].data_ptr(), cell[1:, 5:].data_ptr(), s.data_ptr(), z4.data_ptr(), pc.data_ptr(),
+        *[v.data_ptr() for v in one_off], rows, D, s.stride(0), z4.stride(0), pc.stride(0), D + 9, 0.35, 1e-6, 1e-6, 1,
         _native.DTYPE_BF16 if dtype == torch.bfloat16 else _native.DTYPE_F16, torch.cuda.current_stream().cuda_stream))
-    for got, want in ((state, got_s), (cell, got_c)):
-        assert_close(got[1:-1, 5:5 + D], want, RTOL, ATOL)
+    for got, expected in zip((state, cell), want):
+        assert_close(got[1:-1, 5:5 + D], expected, RTOL, ATOL)
         got[1:-1, 5:5 + D] = 7.0
         assert torch.equal(got, guard)
 
