@@ -248,7 +248,7 @@ __global__ __launch_bounds__(1024) void row_argmax_kernel(int64_t *__restrict__ 
 // ---- rows split over several workgroups ----------------------------------------------------------------------
 // One workgroup pulls at most about 50 GB/s out of HBM (what a CU keeps outstanding over the latency), 5 us for the
 // 256 KB of a row of 128256 16-bit logits, so a few rows leave the chip idle.  Here each row is cut into `parts`
-// segments of two to four chunks per lane.  Every workgroup leaves its segment's winner in the workspace and then reads
+// segments of at least two chunks per lane.  Every workgroup leaves its segment's winner in the workspace and then reads
 // the winners of the whole row; a workgroup that finds all of them there merges them and stores the row's answer.
 //
 // The workspace is memory of the call's own with unknown contents: nothing has to be cleared beforehand and nothing is

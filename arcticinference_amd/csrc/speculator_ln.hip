@@ -189,8 +189,9 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
   const dim3 grid((unsigned)rows);
   // Rows that are not 16-byte aligned take the same kernel with accesses at any alignment.  Us per call in a graph, element
   // by element / in chunks: 300 x 1537 fp16 5.5 / 3.3, 64 x 4096 pitched by 4099 7.0 / 2.7, 4000 x 4097 34.6 / 17.5 (3.7
-  // TB/s), 300 x 20000 pitched by 20001 57 / 9.9; 4000 x 160 4.7 / 3.6 and 300 x 100 level at 2.2, so that rows of fewer
-  // than 128 elements, where a single wave would do a row's work, stay with the element-wise kernel.
+  // TB/s), 300 x 20000 pitched by 20001 57 / 9.9, 300 x 65535 171 / 34 (eight chunks per lane, some of them in scratch);
+  // 4000 x 160 4.7 / 3.6 and 300 x 100 level at 2.2, so that rows of fewer than 128 elements, where a single wave would do
+  // a row's work, stay with the element-wise kernel.
   constexpr int kShortRow = 128;
   if (hidden >= (aligned ? 8 : kShortRow) && chunks <= 8 * 1024) {
     int cpt = 1;

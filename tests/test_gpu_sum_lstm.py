@@ -354,8 +354,8 @@ def test_rows_that_are_not_16_byte_aligned(ops, D, pad4, padD, rows):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_absent_vectors_equal_ones_and_zeros(ops, D, rows, dtype):
     """None of the four vectors, or the shifts alone missing: bit for bit what ones and zeros in their place give, on both
-    sides of every change of kernel, with and without a previous cell, with one z for all gates and with four; and within
-    the tolerance of the oracle."""
+    sides of every change of kernel, with and without a previous cell, with one z for all gates and with four, which agree
+    bit for bit as well; and within the tolerance of the oracle."""
     c = make_lstm_case(rows=rows, D=D, dtype=dtype, seed=D + rows, wb_cell=False, wb_state=False, repeat_z=True)
     d = {k: dev(v) for k, v in c.items() if v is not None}
     ones, zeros = torch.ones(D, dtype=dtype, device=DEV), torch.zeros(D, dtype=dtype, device=DEV)
@@ -364,9 +364,10 @@ def test_absent_vectors_equal_ones_and_zeros(ops, D, rows, dtype):
     z = d["z4"][:, :D]
     for cell in (d["prev_cell"], None):
         for absent, full in (((None,) * 4, (ones, zeros, ones, zeros)), ((scale, None, scale, None), (scale, zeros, scale, zeros))):
-            for op, z_given in ((ops.sum_lstm, d["z4"]), (ops.sum_lstm_shared_z, z)):
-                got, want = (op(d["states"], z_given, cell, *v, *tail) for v in (absent, full))
-                assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+            results = [op(d["states"], z_given, cell, *v, *tail)
+                       for op, z_given in ((ops.sum_lstm, d["z4"]), (ops.sum_lstm_shared_z, z)) for v in (absent, full)]
+            for state, new_cell in results[1:]:
+                assert torch.equal(state, results[0][0]) and torch.equal(new_cell, results[0][1])
     run(ops, c, alpha=0.35)
 
 
