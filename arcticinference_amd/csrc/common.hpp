@@ -39,6 +39,18 @@ struct Divisor {
   __host__ __device__ uint32_t quotient(uint32_t n) const { return (uint32_t)(((uint64_t)n * m) >> shift); }
 };
 
+// A launch.  The host writes a launch's arguments into the GPU's memory, and what that costs is the processor's stores over
+// the bus: an empty kernel with one structure of up to 112 bytes is issued in 2.4 to 2.8 us (two levels, by where the process
+// runs), with one of 256 to 768 bytes in 2.5 to 3.5 us, with 2288 bytes in 2.6 to 3.8 us, and with ten scalars in place of a
+// structure of 64 bytes in 2.5 to 3.3 us.  The kernels that small calls take therefore have one structure or two, as small as
+// their contents allow, and none of them asks for blockDim or gridDim: for those the runtime appends 256 bytes.  The structures
+// go to the runtime from where they are, without the copy that passing them by value to the kernel's host-side function makes.
+template <typename... Args>
+inline void launch(void (*kernel)(Args...), dim3 grid, int lanes, hipStream_t s, const Args &...args) {
+  void *list[] = {const_cast<Args *>(&args)...};
+  (void)hipLaunchKernel((const void *)kernel, grid, dim3((unsigned)lanes), list, 0, s);   // check_launch() reports an error
+}
+
 // ---- 16-bit floats ---------------------------------------------------------
 // Activation element types. to_float is exact; from_float rounds to nearest
 // even (what __float2bfloat16 / __float2half do in the reference,
@@ -215,15 +227,15 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
-// Sum over the whole workgroup (blockDim.x a multiple of 64, at most 1024 = 16
-// waves).  `slots` is LDS for 16 floats, private to this call site.  Each wave
+// Sum over the whole workgroup of `nwaves` full waves (at most 16).  `slots` is
+// LDS for 16 floats, private to this call site.  Each wave
 // leaves its total in slots[wave]; after the barrier every row of 16 lanes reads
 // the 16 slots (zero beyond the last wave) and folds them with the same DPP
 // butterfly, so all lanes of all waves end with the identical total and no loop
-// or branch depends on the number of waves.
-__device__ __forceinline__ float block_sum(float v, float *slots) {
+// or branch depends on the number of waves.  (The callers know the number of waves from their arguments: blockDim is
+// among 256 bytes that the runtime appends to the arguments of a kernel that asks for it.)
+__device__ __forceinline__ float block_sum(float v, float *slots, int nwaves) {
   v = wave_sum(v);
-  const int nwaves = blockDim.x >> 6;
   if (nwaves == 1) return v;
   const int lane = threadIdx.x & 63;
   if (lane == 0) slots[threadIdx.x >> 6] = v;

@@ -40,12 +40,15 @@ namespace arctic {
 
 constexpr int kScalarThreads = 256;
 constexpr int kLayersPerLaunch = 64;  // 4 tables x 64 pointers = 2 KiB of kernel arguments
+// Launches of up to this many layers take tables of that size where the launch's own cost counts (launch_vec_shape).
+constexpr int kFewLayers = 16;
 
+template <int kLayers>
 struct LayerTables {
-  const void *key_cache[kLayersPerLaunch];
-  const void *value_cache[kLayersPerLaunch];
-  const float *k_scale[kLayersPerLaunch];
-  const float *v_scale[kLayersPerLaunch];
+  const void *key_cache[kLayers];
+  const void *value_cache[kLayers];
+  const float *k_scale[kLayers];
+  const float *v_scale[kLayers];
 };
 
 struct BulkParams {
@@ -69,6 +72,9 @@ struct BulkParams {
   Divisor by_chunks;     // chunks_per_row
   Divisor by_block;      // block_size
   Divisor by_groups;     // groups_per_token
+};
+
+struct BulkSelectParams : BulkParams {
   // select variants: token t's source rows are also copied, unconverted, to the rows j of keys_out / values_out with
   // indices[j] == t.  With a row map (kSelectByRowMap) that is row row_map[t] of keys_out /
   // values_out (already offset to the first layer of this launch); a negative row or one >= num_out_rows = none
@@ -95,6 +101,13 @@ struct BulkParams {
 // built beforehand, or by scanning the index list itself (short lists: one or a few loads per lane, no launch and
 // no workspace for the inverse).
 enum : int { kSelectNone = 0, kSelectByRowMap = 1, kSelectByScan = 2 };
+
+template <int kSelect>
+struct ParamsFor { using type = BulkSelectParams; };
+template <>
+struct ParamsFor<kSelectNone> { using type = BulkParams; };
+template <int kSelect>
+using BulkParamsOf = typename ParamsFor<kSelect>::type;
 
 struct __align__(16) RowDesc {
   char *dst;    // first byte of this token's row in the layer's K or V cache
@@ -151,7 +164,7 @@ __device__ __forceinline__ void emit_chunk(const uint4 &v, const RowDesc &d, int
 // the source.  By row map: the token's workgroup serves the one output row the map credits the token with.  By scan:
 // it serves every output row that names the token, so only source rows beyond the slot mapping are left.
 template <int kSelect>
-__device__ __forceinline__ int64_t leftover_source_row(const BulkParams &p, int64_t j) {
+__device__ __forceinline__ int64_t leftover_source_row(const BulkSelectParams &p, int64_t j) {
   const int64_t t = p.index_is_64 ? ((const int64_t *)p.indices)[j] : (int64_t)((const int32_t *)p.indices)[j];
   if (t < 0 || t >= p.num_src_rows) return -1;
   if (t < p.num_tokens && (kSelect == kSelectByScan || p.row_map[t] == j)) return -1;
@@ -162,7 +175,7 @@ __device__ __forceinline__ int64_t leftover_source_row(const BulkParams &p, int6
 // left over (SwiftKV selects each token once) and the workgroup is done after two dependent lookups.  The rows that
 // are left over are listed in LDS and copied by the whole workgroup, all layers of the launch, one row after the other.
 template <int kThreads, int kSelect>
-__device__ __forceinline__ int list_leftover_rows(const BulkParams &p, unsigned b, int64_t (&todo_j)[kThreads],
+__device__ __forceinline__ int list_leftover_rows(const BulkSelectParams &p, unsigned b, int64_t (&todo_j)[kThreads],
                                                   int64_t (&todo_t)[kThreads], int &count) {
   if (threadIdx.x == 0) count = 0;
   __syncthreads();
@@ -180,7 +193,7 @@ __device__ __forceinline__ int list_leftover_rows(const BulkParams &p, unsigned 
 }
 
 template <typename Src, bool kPow2, int kBulkThreads, int kSelect>
-__device__ __forceinline__ void select_leftover_rows(const BulkParams &p, unsigned b) {
+__device__ __forceinline__ void select_leftover_rows(const BulkSelectParams &p, unsigned b) {
   __shared__ int64_t todo_j[kBulkThreads], todo_t[kBulkThreads];
   __shared__ int count;
   const int n = list_leftover_rows<kBulkThreads, kSelect>(p, b, todo_j, todo_t, count);
@@ -208,8 +221,8 @@ __device__ __forceinline__ void select_leftover_rows(const BulkParams &p, unsign
 // kBulkThreads x kUnroll 16-byte chunks form one batch of a workgroup.  Three shapes are built, all with batches
 // of 1024 chunks: 1024 x 1 (launches of more than 8192 tokens: a workgroup moves up to five batches), 512 x 2 (the
 // same launches when rows are selected as well) and 256 x 4 (everything smaller: one or two batches per workgroup).
-template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect>
-__device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables &tab, unsigned block) {
+template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, typename Params, typename Tables>
+__device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, unsigned block) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
   constexpr int kDstElemBytes = kCopy ? Src::kBytes : 1;
 
@@ -267,7 +280,7 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
   constexpr int kIndicesPerLane = ARCTIC_SELECT_SCAN_MAX_INDICES / kBulkThreads;
   __shared__ int hits[kSelect == kSelectByScan ? ARCTIC_SELECT_SCAN_MAX_INDICES : 1];
   __shared__ int num_hits;
-  int64_t mine[kIndicesPerLane];
+  [[maybe_unused]] int64_t mine[kIndicesPerLane];
   if constexpr (kSelect == kSelectByScan) {
 #pragma unroll
     for (int k = 0; k < kIndicesPerLane; ++k) {
@@ -369,19 +382,17 @@ __device__ __forceinline__ void bulk_item(const BulkParams &p, const LayerTables
   }
 }
 
-template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect>
-__global__ __launch_bounds__(kBulkThreads) void kv_write_bulk_kernel(
-    const BulkParams p, const LayerTables tab) {
+template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, int kLayers>
+__global__ __launch_bounds__(kBulkThreads) void kv_write_bulk_kernel(const BulkParamsOf<kSelect> p,
+                                                                         const LayerTables<kLayers> tab) {
   bulk_item<Src, Dst, kPow2, kBulkThreads, kUnroll, kSelect>(p, tab, blockIdx.x);
 }
-
-
 
 // Fallback for shapes or addresses that do not allow 16-byte accesses: one
 // element per lane per step, any alignment.  Same arithmetic, no vector access.
 template <typename SrcElem, typename Dst>
 __global__ __launch_bounds__(kScalarThreads) void kv_write_bulk_scalar_kernel(
-    const BulkParams p, const LayerTables tab, const int src_dtype) {
+    const BulkSelectParams p, const LayerTables<kLayersPerLaunch> tab, const int src_dtype) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
   if (blockIdx.x < p.index_blocks) {  // the index list's own workgroups (select variant only)
     __shared__ int64_t todo_j[kScalarThreads], todo_t[kScalarThreads];
@@ -480,49 +491,79 @@ __global__ __launch_bounds__(kScalarThreads) void kv_write_bulk_scalar_kernel(
   }
 }
 
-template <typename Src, typename Dst, int kSelect>
-static void launch_vec_shape(const BulkParams &p, const LayerTables &tab, int64_t grid, bool wide, hipStream_t s) {
-  const dim3 g((unsigned)grid);
-  if (p.chunk_shift >= 0) {
-    if (wide && kSelect == kSelectNone)   // the same batch of 1024 chunks by 1024 lanes: 0.5-2 % faster than 512 x 2
-      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 1024, 1, kSelectNone>), g, dim3(1024), 0, s, p, tab);
-    else if (wide)
-      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 512, 2, kSelect>), g, dim3(512), 0, s, p, tab);
-    else
-      hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, true, 256, 4, kSelect>), g, dim3(256), 0, s, p, tab);
-  } else {
-    hipLaunchKernelGGL((kv_write_bulk_kernel<Src, Dst, false, 256, 4, kSelect>), g, dim3(256), 0, s, p, tab);
+// The per-layer pointers of a call, from the first layer of a launch on; scales are nullptr for a copy.
+struct LayerPointers {
+  const void *const *key_cache;
+  const void *const *value_cache;
+  const float *const *k_scale;
+  const float *const *v_scale;
+  template <int kLayers>
+  void fill(LayerTables<kLayers> &tab, int count) const {   // the entries behind `count` are never read
+    std::copy_n(key_cache, count, tab.key_cache);
+    std::copy_n(value_cache, count, tab.value_cache);
+    if (k_scale) std::copy_n(k_scale, count, tab.k_scale);
+    if (v_scale) std::copy_n(v_scale, count, tab.v_scale);
   }
+};
+
+template <typename Src, typename Dst, int kSelect>
+static void launch_vec_shape(const BulkSelectParams &p, const LayerPointers &layers, int64_t grid, bool wide,
+                             hipStream_t s) {
+  const dim3 g((unsigned)grid);
+#define ARCTIC_BULK_LAUNCH(POW2, LANES, UNROLL, LAYERS)                                                             \
+  do {                                                                                                             \
+    LayerTables<LAYERS> tab;                                                                                       \
+    layers.fill(tab, p.num_layers);                                                                                \
+    launch<BulkParamsOf<kSelect>>(kv_write_bulk_kernel<Src, Dst, POW2, LANES, UNROLL, kSelect, LAYERS>, g, LANES, s, p, tab); \
+  } while (0)
+  if constexpr (kSelect == kSelectNone) {
+    // The 256-lane shape is also that of the small launches, which cost what it takes to issue them: few layers leave
+    // 1.5 KB of their arguments out.
+    const bool few = p.num_layers <= kFewLayers;
+    if (p.chunk_shift < 0 && few) ARCTIC_BULK_LAUNCH(false, 256, 4, kFewLayers);
+    else if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch);
+    else if (wide) ARCTIC_BULK_LAUNCH(true, 1024, 1, kLayersPerLaunch);   // 0.5-2 % faster than the same batch as 512 x 2
+    else if (few) ARCTIC_BULK_LAUNCH(true, 256, 4, kFewLayers);
+    else ARCTIC_BULK_LAUNCH(true, 256, 4, kLayersPerLaunch);
+  } else {
+    if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch);
+    else if (wide) ARCTIC_BULK_LAUNCH(true, 512, 2, kLayersPerLaunch);
+    else ARCTIC_BULK_LAUNCH(true, 256, 4, kLayersPerLaunch);
+  }
+#undef ARCTIC_BULK_LAUNCH
 }
 template <typename Src, typename Dst>
-static void launch_vec(const BulkParams &p, const LayerTables &tab, int64_t grid, bool wide, hipStream_t s) {
+static void launch_vec(const BulkSelectParams &p, const LayerPointers &layers, int64_t grid, bool wide,
+                       hipStream_t s) {
   switch (p.select_mode) {
-    case kSelectByScan: launch_vec_shape<Src, Dst, kSelectByScan>(p, tab, grid, wide, s); break;
-    case kSelectByRowMap: launch_vec_shape<Src, Dst, kSelectByRowMap>(p, tab, grid, wide, s); break;
-    default: launch_vec_shape<Src, Dst, kSelectNone>(p, tab, grid, wide, s); break;
+    case kSelectByScan: launch_vec_shape<Src, Dst, kSelectByScan>(p, layers, grid, wide, s); break;
+    case kSelectByRowMap: launch_vec_shape<Src, Dst, kSelectByRowMap>(p, layers, grid, wide, s); break;
+    default: launch_vec_shape<Src, Dst, kSelectNone>(p, layers, grid, wide, s); break;
   }
 }
 template <typename SrcElem, typename Dst>
-static void launch_scalar(const BulkParams &p, const LayerTables &tab, int64_t grid, int src_dtype,
+static void launch_scalar(const BulkSelectParams &p, const LayerPointers &layers, int64_t grid, int src_dtype,
                           hipStream_t s) {
+  LayerTables<kLayersPerLaunch> tab;
+  layers.fill(tab, p.num_layers);
   hipLaunchKernelGGL((kv_write_bulk_scalar_kernel<SrcElem, Dst>), dim3((unsigned)grid),
                      dim3(kScalarThreads), 0, s, p, tab, src_dtype);
 }
 
 template <typename Dst>
-static void dispatch_src(bool vec, bool wide, int src_dtype, const BulkParams &p, const LayerTables &tab,
-                         int64_t grid, hipStream_t s) {
+static void dispatch_src(bool vec, bool wide, int src_dtype, const BulkSelectParams &p,
+                         const LayerPointers &layers, int64_t grid, hipStream_t s) {
   if (vec) {
     switch (src_dtype) {
-      case ARCTIC_DTYPE_BF16: launch_vec<SrcBF16, Dst>(p, tab, grid, wide, s); break;
-      case ARCTIC_DTYPE_F16: launch_vec<SrcF16, Dst>(p, tab, grid, wide, s); break;
-      default: launch_vec<SrcF32, Dst>(p, tab, grid, wide, s); break;
+      case ARCTIC_DTYPE_BF16: launch_vec<SrcBF16, Dst>(p, layers, grid, wide, s); break;
+      case ARCTIC_DTYPE_F16: launch_vec<SrcF16, Dst>(p, layers, grid, wide, s); break;
+      default: launch_vec<SrcF32, Dst>(p, layers, grid, wide, s); break;
     }
   } else {
     if (src_dtype == ARCTIC_DTYPE_F32)
-      launch_scalar<uint32_t, Dst>(p, tab, grid, src_dtype, s);
+      launch_scalar<uint32_t, Dst>(p, layers, grid, src_dtype, s);
     else
-      launch_scalar<uint16_t, Dst>(p, tab, grid, src_dtype, s);
+      launch_scalar<uint16_t, Dst>(p, layers, grid, src_dtype, s);
   }
 }
 
@@ -650,15 +691,9 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
   for (int pass = (check_only || num_layers > kLayersPerLaunch) ? 0 : 1; pass < (check_only ? 1 : 2); ++pass) {
     for (int first = 0; first < num_layers; first += kLayersPerLaunch) {
       const int count = std::min(kLayersPerLaunch, num_layers - first);
-      LayerTables tab;
-      for (int l = 0; l < kLayersPerLaunch; ++l) {
-        const bool in = l < count;
-        tab.key_cache[l] = in ? key_cache_ptrs[first + l] : nullptr;
-        tab.value_cache[l] = in ? value_cache_ptrs[first + l] : nullptr;
-        tab.k_scale[l] = (in && quant) ? k_scale_ptrs[first + l] : nullptr;
-        tab.v_scale[l] = (in && quant) ? v_scale_ptrs[first + l] : nullptr;
-      }
-      BulkParams p;
+      const LayerPointers layers = {key_cache_ptrs + first, value_cache_ptrs + first, quant ? k_scale_ptrs + first : nullptr,
+                                    quant ? v_scale_ptrs + first : nullptr};
+      BulkSelectParams p;
       p.keys = (const char *)keys + (int64_t)first * n * es;
       p.values = (const char *)values + (int64_t)first * n * es;
       p.slot_mapping = slot_mapping;
@@ -732,9 +767,9 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       if (pass == 0) continue;
 
       switch (kv_cache_dtype) {
-        case ARCTIC_KV_AUTO: dispatch_src<Copy>(vec, wide, src_dtype, p, tab, grid, s); break;
-        case ARCTIC_KV_FP8_E4M3: dispatch_src<E4M3>(vec, wide, src_dtype, p, tab, grid, s); break;
-        default: dispatch_src<E5M2>(vec, wide, src_dtype, p, tab, grid, s); break;
+        case ARCTIC_KV_AUTO: dispatch_src<Copy>(vec, wide, src_dtype, p, layers, grid, s); break;
+        case ARCTIC_KV_FP8_E4M3: dispatch_src<E4M3>(vec, wide, src_dtype, p, layers, grid, s); break;
+        default: dispatch_src<E5M2>(vec, wide, src_dtype, p, layers, grid, s); break;
       }
       const int rc = check_launch(fn);
       if (rc) return rc;

@@ -171,7 +171,7 @@ extern "C" int arctic_reshape_and_cache_flash_fp4(
   if (grid > 0x7fffffffLL) return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: too many tokens", fn);
   const bool many = p.total_groups > 0x7fffffffLL;
 #define ARCTIC_FP4_LAUNCH(TYPE, MANY) \
-  hipLaunchKernelGGL((kv_write_fp4_kernel<TYPE, MANY>), dim3((unsigned)grid), dim3(kFp4Lanes), 0, s, p)
+  launch(kv_write_fp4_kernel<TYPE, MANY>, dim3((unsigned)grid), kFp4Lanes, s, p)
   if (dtype == ARCTIC_DTYPE_BF16) {
     if (many) ARCTIC_FP4_LAUNCH(BF16, true);
     else ARCTIC_FP4_LAUNCH(BF16, false);

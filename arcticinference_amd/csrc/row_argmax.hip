@@ -114,9 +114,10 @@ struct HalfElem {
 // asked for batch k before any wave asks for batch k + 1 (a CU serves its oldest wave first: without the barrier the
 // oldest wave runs through all its batches before the youngest gets its first one in).
 // kHead: rows may start between two 16-byte boundaries (without it the host has checked that none does).
-// Returns the winner of the `cols` elements at `row` as a key whose index counts from `first`, in every lane of wave 0.
+// Returns the winner of the `cols` elements at `row` as a key whose index counts from `first`, in every lane of wave 0 of
+// a workgroup of `lanes`.
 template <typename Elem, bool kVec, int kUnroll, bool kLockstep, bool kHead>
-__device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, int cols, int first) {
+__device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, int cols, int first, int lanes) {
   __shared__ uint64_t wave_key[16];
   // Per lane: the largest number seen, the chunk it was first seen in and that chunk's words (a strict ">" keeps the
   // earlier of equal values, the lane's chunk indices only grow); which of the chunk's elements it was is worked out
@@ -146,11 +147,11 @@ __device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, in
   if (kVec) {
     int best_chunk = -1;
     uint4 best_words = make_uint4(0, 0, 0, 0);
-    const int stride = kUnroll * blockDim.x;
+    const int stride = kUnroll * lanes;
     auto request = [&](int c0, uint4 (&raw)[kUnroll]) {
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        const int c = c0 + u * blockDim.x;
+        const int c = c0 + u * lanes;
         if (c < chunks) raw[u] = load16_stream(body + (int64_t)c * 16);
       }
     };
@@ -175,7 +176,7 @@ __device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, in
     auto look_at = [&](int c0, const uint4 (&raw)[kUnroll]) {
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        const int c = c0 + u * blockDim.x;
+        const int c = c0 + u * lanes;
         if (c < chunks) look_at_chunk(c, raw[u]);
       }
     };
@@ -214,7 +215,7 @@ __device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, in
   }
   // (a lane without chunks takes its first tail element, if it has one, the same way: a row of -inf must answer 0)
   if (best_at < 0 && done + (int)threadIdx.x < cols) best_at = done + (int)threadIdx.x;
-  for (int i = done + threadIdx.x; i < cols; i += blockDim.x) {
+  for (int i = done + threadIdx.x; i < cols; i += lanes) {
     const float v = Elem::one(row, i);
     number(v, i);
     if (v != v) nan_at = min(nan_at, i);
@@ -227,7 +228,7 @@ __device__ __forceinline__ uint64_t find_winner(const char *__restrict__ row, in
   if (lane == 0) wave_key[wave] = w;
   __syncthreads();
   if (wave > 0) return 0;
-  const int waves = blockDim.x >> 6;
+  const int waves = lanes >> 6;
   return wave_winner<1>(lane < waves ? wave_key[lane] : 0);   // at most 16 waves
 }
 
@@ -237,12 +238,30 @@ __device__ __forceinline__ void store_winner(int64_t *out, uint64_t key, int64_t
   *out = idx > max_index ? max_index : idx;
 }
 
+struct Segment {
+  uint64_t key;
+  uint64_t seal;
+};
+static_assert(sizeof(Segment) == ARCTIC_ARGMAX_SEGMENT_BYTES, "the workspace holds one Segment per workgroup");
+
+struct ArgmaxParams {
+  int64_t *out;
+  const char *in;
+  int64_t row_stride_bytes;
+  int64_t max_index;
+  int cols;
+  int lanes;   // of a workgroup
+  // rows split over several workgroups:
+  int segment, parts;
+  uint64_t call;
+  Segment *workspace;
+};
+
 template <typename Elem, bool kVec, int kUnroll = 4, bool kLockstep = false, bool kHead = false>
-__global__ __launch_bounds__(1024) void row_argmax_kernel(int64_t *__restrict__ out, const char *__restrict__ in,
-                                                          int64_t row_stride_bytes, int cols, int64_t max_index) {
-  const uint64_t w =
-      find_winner<Elem, kVec, kUnroll, kLockstep, kHead>(in + (int64_t)blockIdx.x * row_stride_bytes, cols, 0);
-  if (threadIdx.x == 0) store_winner(out + blockIdx.x, w, max_index);
+__global__ __launch_bounds__(1024) void row_argmax_kernel(const ArgmaxParams p) {
+  const uint64_t w = find_winner<Elem, kVec, kUnroll, kLockstep, kHead>(p.in + (int64_t)blockIdx.x * p.row_stride_bytes,
+                                                                        p.cols, 0, p.lanes);
+  if (threadIdx.x == 0) store_winner(p.out + blockIdx.x, w, p.max_index);
 }
 
 // ---- rows split over several workgroups ----------------------------------------------------------------------
@@ -263,12 +282,6 @@ __global__ __launch_bounds__(1024) void row_argmax_kernel(int64_t *__restrict__ 
 // are agent-scope atomics, which go to the memory all XCDs see whatever their L2s hold, so the wait for the stores'
 // acknowledgement is all the order that is needed; a sequentially consistent fence in its place writes back and
 // invalidates the L2 once per workgroup, and those queue up (64 rows of 16 segments: 22.3 us instead of 7.0).
-struct Segment {
-  uint64_t key;
-  uint64_t seal;
-};
-static_assert(sizeof(Segment) == ARCTIC_ARGMAX_SEGMENT_BYTES, "the workspace holds one Segment per workgroup");
-
 __device__ __forceinline__ uint64_t seal_of(uint64_t key, uint64_t call) { return (key * 0x9E3779B97F4A7C15ull) ^ call; }
 __device__ __forceinline__ void share(uint64_t *p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -301,17 +314,14 @@ __device__ __forceinline__ void merge_segments(int64_t *out, Segment *row, int p
 constexpr int kSplitLanes = 512;
 
 template <typename Elem, bool kHead>
-__global__ __launch_bounds__(kSplitLanes) void row_argmax_split_kernel(int64_t *__restrict__ out,
-                                                                       const char *__restrict__ in,
-                                                                       int64_t row_stride_bytes, int cols,
-                                                                       int segment, int parts, uint64_t call,
-                                                                       int64_t max_index, Segment *workspace) {
-  const unsigned row = blockIdx.x / (unsigned)parts;
-  const int part = (int)(blockIdx.x - row * (unsigned)parts);
-  const int first = part * segment;
-  const char *at = in + (int64_t)row * row_stride_bytes + (int64_t)first * (16 / Elem::kPerChunk);
-  const uint64_t w = find_winner<Elem, true, 4, false, kHead>(at, min(segment, cols - first), first);
-  if (threadIdx.x < 64) merge_segments(out + row, workspace + (int64_t)row * parts, part, parts, w, call, max_index);
+__global__ __launch_bounds__(kSplitLanes) void row_argmax_split_kernel(const ArgmaxParams p) {
+  const unsigned row = blockIdx.x / (unsigned)p.parts;
+  const int part = (int)(blockIdx.x - row * (unsigned)p.parts);
+  const int first = part * p.segment;
+  const char *at = p.in + (int64_t)row * p.row_stride_bytes + (int64_t)first * (16 / Elem::kPerChunk);
+  const uint64_t w = find_winner<Elem, true, 4, false, kHead>(at, min(p.segment, p.cols - first), first, kSplitLanes);
+  if (threadIdx.x < 64)
+    merge_segments(p.out + row, p.workspace + (int64_t)row * p.parts, part, p.parts, w, p.call, p.max_index);
 }
 
 }  // namespace arctic
@@ -378,10 +388,10 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
     if ((uintptr_t)workspace % 8 || workspace_bytes < rows * parts * (int64_t)sizeof(Segment))
       return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: the workspace must be 8-byte aligned and hold %lld bytes", fn,
                   (long long)(rows * parts * (int64_t)sizeof(Segment)));
-    const uint64_t call = call_number();
-#define ARCTIC_ARGMAX_SPLIT(ELEM, HEAD)                                                                            \
-  hipLaunchKernelGGL((row_argmax_split_kernel<ELEM, HEAD>), dim3((unsigned)(rows * parts)), dim3(kSplitLanes), 0, s, out, \
-                     (const char *)logits, stride_bytes, cols, segment, parts, call, max_index, (Segment *)workspace)
+    const ArgmaxParams p = {out, (const char *)logits, stride_bytes, max_index, cols, kSplitLanes, segment, parts,
+                            call_number(), (Segment *)workspace};
+#define ARCTIC_ARGMAX_SPLIT(ELEM, HEAD) \
+  launch(row_argmax_split_kernel<ELEM, HEAD>, dim3((unsigned)(rows * parts)), kSplitLanes, s, p)
     if (dtype == ARCTIC_DTYPE_F32) {
       if (aligned_rows) ARCTIC_ARGMAX_SPLIT(F32Elem, false);
       else ARCTIC_ARGMAX_SPLIT(F32Elem, true);
@@ -396,39 +406,26 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
     return check_launch(fn);
   }
   int threads = (int)std::min<int64_t>(1024, std::max<int64_t>(64, ((cols / per_chunk / 4 + 63) / 64) * 64));
-  const dim3 grid((unsigned)rows), block((unsigned)threads);
+  const dim3 grid((unsigned)rows);
   // Launches of about one and a half to three workgroups per CU (the 256 CUs of this GPU; a decode batch of a few
   // hundred rows) keep their waves in step, a chunk at a time: the two workgroups of a CU then finish together with
   // little left to do, 5 % faster at 384 and 512 rows.  With fewer rows a wave needs four chunks in flight to cover
   // the latency, with more the generations of workgroups overlap by themselves (measured 16 to 4096 rows).
   const bool lockstep = rows > 256 && rows <= 768;
-#define ARCTIC_ARGMAX_VEC(ELEM)                                                                                   \
-  do {                                                                                                            \
-    if (!aligned_rows && lockstep)                                                                                \
-      hipLaunchKernelGGL((row_argmax_kernel<ELEM, true, 1, true, true>), grid, block, 0, s, out,    \
-                         (const char *)logits, stride_bytes, cols, max_index);                                    \
-    else if (!aligned_rows)                                                                                       \
-      hipLaunchKernelGGL((row_argmax_kernel<ELEM, true, 4, false, true>), grid, block, 0, s, out,   \
-                         (const char *)logits, stride_bytes, cols, max_index);                                    \
-    else if (lockstep)                                                                                            \
-      hipLaunchKernelGGL((row_argmax_kernel<ELEM, true, 1, true>), grid, block, 0, s, out,          \
-                         (const char *)logits, stride_bytes, cols, max_index);                                    \
-    else                                                                                                          \
-      hipLaunchKernelGGL((row_argmax_kernel<ELEM, true>), grid, block, 0, s, out, (const char *)logits,           \
-                         stride_bytes, cols, max_index);                                                          \
-  } while (0)
-#define ARCTIC_ARGMAX_LAUNCH(ELEM)                                                                          \
-  do {                                                                                                      \
-    if (vec)                                                                                                \
-      ARCTIC_ARGMAX_VEC(ELEM);                                                                              \
-    else                                                                                                    \
-      hipLaunchKernelGGL((row_argmax_kernel<ELEM, false>), grid, block, 0, s, out, (const char *)logits,    \
-                         stride_bytes, cols, max_index);                                                    \
+  const ArgmaxParams p = {out, (const char *)logits, stride_bytes, max_index, cols, threads, cols, 1, 0, nullptr};
+#define ARCTIC_ARGMAX_KERNEL(...) launch(row_argmax_kernel<__VA_ARGS__>, grid, threads, s, p)
+#define ARCTIC_ARGMAX_LAUNCH(ELEM)                                                       \
+  do {                                                                                   \
+    if (!vec) ARCTIC_ARGMAX_KERNEL(ELEM, false);                                         \
+    else if (!aligned_rows && lockstep) ARCTIC_ARGMAX_KERNEL(ELEM, true, 1, true, true); \
+    else if (!aligned_rows) ARCTIC_ARGMAX_KERNEL(ELEM, true, 4, false, true);            \
+    else if (lockstep) ARCTIC_ARGMAX_KERNEL(ELEM, true, 1, true);                        \
+    else ARCTIC_ARGMAX_KERNEL(ELEM, true);                                               \
   } while (0)
   if (dtype == ARCTIC_DTYPE_F32) ARCTIC_ARGMAX_LAUNCH(F32Elem);
   else if (dtype == ARCTIC_DTYPE_BF16) ARCTIC_ARGMAX_LAUNCH(HalfElem<BF16>);
   else ARCTIC_ARGMAX_LAUNCH(HalfElem<F16>);
 #undef ARCTIC_ARGMAX_LAUNCH
-#undef ARCTIC_ARGMAX_VEC
+#undef ARCTIC_ARGMAX_KERNEL
   return check_launch(fn);
 }

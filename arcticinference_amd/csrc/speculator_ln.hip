@@ -26,19 +26,28 @@
 
 namespace arctic {
 
-// What surrounds the norm; all fields are uniform over the launch.
-struct LnGlue {
+// A launch's arguments, in one piece (common.hpp says what that is worth).
+struct LnParams {
+  char *out;
+  const char *in;
+  const char *weight;       // may be nullptr, like bias
+  const char *bias;
   const char *z;            // nullptr: no add
-  int64_t z_row_stride_bytes;
   const int64_t *z_index;   // row of z to add to each row (an embedding lookup); nullptr = the row itself
+  int64_t in_row_stride_bytes;
+  int64_t z_row_stride_bytes;
   int64_t z_rows;           // rows of z when z_index is given; an index is clamped into [0, z_rows)
+  int hidden;
+  int waves;                // of the workgroup
+  float inv_hidden;         // 1 / hidden
+  float eps;
   float alpha;
-  int activation;           // ARCTIC_ACT_*
   float out_scale;          // applied when != 1
+  int activation;           // ARCTIC_ACT_* (the vector kernels take it as a template argument)
 };
 
 template <typename T>
-__device__ __forceinline__ float glue_tail(float y, const LnGlue &g, int activation) {
+__device__ __forceinline__ float glue_tail(float y, const LnParams &g, int activation) {
   if (activation != ARCTIC_ACT_NONE) {
     y = T::requant(y);
     y = activation == ARCTIC_ACT_GELU ? gelu_erf(y) : gelu_tanh(y);
@@ -57,15 +66,14 @@ __device__ __forceinline__ float glue_tail(float y, const LnGlue &g, int activat
 // the scaled norm of 7 x 4096 2.20 / 2.10).
 constexpr int kPlain = -1;
 template <typename T, int kChunksPerThread, int kGlue, bool kAnyRow>
-__global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
-    char *__restrict__ out, const char *__restrict__ in, const char *__restrict__ weight,
-    const char *__restrict__ bias, int64_t in_row_stride_bytes, int hidden, float inv_hidden, float eps,
-    LnGlue glue) {
+__global__ __launch_bounds__(1024) void spec_ln_vec_kernel(const LnParams p) {
   __shared__ float slots[16];
+  const char *__restrict__ weight = p.weight, *__restrict__ bias = p.bias;
+  const int hidden = p.hidden, lanes = p.waves * 64;
   const int chunks = kAnyRow ? (hidden + 7) >> 3 : hidden >> 3;
   auto offset = [&](int c) { return kAnyRow ? (int64_t)Place(c, hidden).off : (int64_t)c * 16; };
-  const char *row_in = in + (int64_t)blockIdx.x * in_row_stride_bytes;
-  char *row_out = out + (int64_t)blockIdx.x * hidden * 2;
+  const char *__restrict__ row_in = p.in + (int64_t)blockIdx.x * p.in_row_stride_bytes;
+  char *__restrict__ row_out = p.out + (int64_t)blockIdx.x * hidden * 2;
 
   uint4 raw[kChunksPerThread], wv[kChunksPerThread], bv[kChunksPerThread];
   float ss = 0.f;
@@ -73,24 +81,24 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
   // order, so asking for them after the row sum would add a full round trip
 #pragma unroll
   for (int k = 0; k < kChunksPerThread; ++k) {
-    const int c = threadIdx.x + k * blockDim.x;
+    const int c = threadIdx.x + k * lanes;
     if (weight && c < chunks) wv[k] = load16<kAnyRow>(weight + offset(c));
     if (bias && c < chunks) bv[k] = load16<kAnyRow>(bias + offset(c));
   }
 #pragma unroll
   for (int k = 0; k < kChunksPerThread; ++k) {
-    const int c = threadIdx.x + k * blockDim.x;
+    const int c = threadIdx.x + k * lanes;
     raw[k] = make_uint4(0, 0, 0, 0);
     if (c < chunks) raw[k] = load16_stream<kAnyRow>(row_in + offset(c));
   }
-  if (kGlue != kPlain && glue.z) {
+  if (kGlue != kPlain && p.z) {
     int64_t z_at = blockIdx.x;
-    if (glue.z_index) z_at = min(max(glue.z_index[blockIdx.x], (int64_t)0), glue.z_rows - 1);
-    const char *row_z = glue.z + z_at * glue.z_row_stride_bytes;
+    if (p.z_index) z_at = min(max(p.z_index[blockIdx.x], (int64_t)0), p.z_rows - 1);
+    const char *row_z = p.z + z_at * p.z_row_stride_bytes;
     uint4 zr[kChunksPerThread];
 #pragma unroll
     for (int k = 0; k < kChunksPerThread; ++k) {
-      const int c = threadIdx.x + k * blockDim.x;
+      const int c = threadIdx.x + k * lanes;
       zr[k] = make_uint4(0, 0, 0, 0);
       if (c < chunks) zr[k] = load16_stream<kAnyRow>(row_z + offset(c));
     }
@@ -100,7 +108,7 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
       unpack8<T>(raw[k], x);
       unpack8<T>(zr[k], z);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = fmaf(glue.alpha, z[j], x[j]);
+      for (int j = 0; j < 8; ++j) x[j] = fmaf(p.alpha, z[j], x[j]);
       raw[k] = pack8<T>(x);   // the sum stands in the tensor's own type, as after the in-place add
     }
   }
@@ -110,14 +118,14 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     unpack8<T>(raw[k], x);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (!kAnyRow || j >= Place(threadIdx.x + k * blockDim.x, hidden).repeated) ss += x[j] * x[j];
+      if (!kAnyRow || j >= Place(threadIdx.x + k * lanes, hidden).repeated) ss += x[j] * x[j];
   }
-  const float total = block_sum(ss, slots);
-  const float inv = rsqrtf(total * inv_hidden + eps);
+  const float total = block_sum(ss, slots, p.waves);
+  const float inv = rsqrtf(total * p.inv_hidden + p.eps);
 
 #pragma unroll
   for (int k = 0; k < kChunksPerThread; ++k) {
-    const int c = threadIdx.x + k * blockDim.x;
+    const int c = threadIdx.x + k * lanes;
     if (c >= chunks) continue;
     float x[8];
     unpack8<T>(raw[k], x);
@@ -137,55 +145,53 @@ __global__ __launch_bounds__(1024) void spec_ln_vec_kernel(
     }
     if (kGlue != kPlain) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = glue_tail<T>(x[j], glue, kGlue);
+      for (int j = 0; j < 8; ++j) x[j] = glue_tail<T>(x[j], p, kGlue);
     }
     store16_stream<kAnyRow>(row_out + offset(c), pack8<T>(x));
   }
 }
 
 // What is left (short unaligned rows, rows beyond 65536 elements): element-wise, two passes over the row.
+constexpr int kScalarLanes = 256;
 template <typename T>
-__global__ __launch_bounds__(256) void spec_ln_scalar_kernel(
-    uint16_t *__restrict__ out, const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
-    const uint16_t *__restrict__ bias, int64_t in_row_stride, int hidden, float inv_hidden, float eps,
-    LnGlue glue) {
+__global__ __launch_bounds__(kScalarLanes) void spec_ln_scalar_kernel(const LnParams p) {
   __shared__ float slots[16];
-  const uint16_t *row_in = in + (int64_t)blockIdx.x * in_row_stride;
+  const uint16_t *__restrict__ weight = (const uint16_t *)p.weight, *__restrict__ bias = (const uint16_t *)p.bias;
+  const int hidden = p.hidden;
+  const uint16_t *__restrict__ row_in = (const uint16_t *)(p.in + (int64_t)blockIdx.x * p.in_row_stride_bytes);
   int64_t z_at = blockIdx.x;
-  if (glue.z && glue.z_index) z_at = min(max(glue.z_index[blockIdx.x], (int64_t)0), glue.z_rows - 1);
-  const uint16_t *row_z = glue.z ? (const uint16_t *)(glue.z + z_at * glue.z_row_stride_bytes) : nullptr;
-  uint16_t *row_out = out + (int64_t)blockIdx.x * hidden;
+  if (p.z && p.z_index) z_at = min(max(p.z_index[blockIdx.x], (int64_t)0), p.z_rows - 1);
+  const uint16_t *row_z = p.z ? (const uint16_t *)(p.z + z_at * p.z_row_stride_bytes) : nullptr;
+  uint16_t *__restrict__ row_out = (uint16_t *)p.out + (int64_t)blockIdx.x * hidden;
   auto element = [&](int j) {
     float x = T::lo(row_in[j]);
-    if (row_z) x = T::requant(fmaf(glue.alpha, T::lo(row_z[j]), x));
+    if (row_z) x = T::requant(fmaf(p.alpha, T::lo(row_z[j]), x));
     return x;
   };
   float ss = 0.f;
-  for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+  for (int j = threadIdx.x; j < hidden; j += kScalarLanes) {
     const float x = element(j);
     ss += x * x;
   }
-  const float total = block_sum(ss, slots);
-  const float inv = rsqrtf(total * inv_hidden + eps);
-  for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+  const float total = block_sum(ss, slots, kScalarLanes / 64);
+  const float inv = rsqrtf(total * p.inv_hidden + p.eps);
+  for (int j = threadIdx.x; j < hidden; j += kScalarLanes) {
     float y = element(j) * inv;
     if (weight) y *= T::lo(weight[j]);
     if (bias) y += T::lo(bias[j]);
-    row_out[j] = (uint16_t)T::round_bits(glue_tail<T>(y, glue, glue.activation));
+    row_out[j] = (uint16_t)T::round_bits(glue_tail<T>(y, p, p.activation));
   }
 }
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 template <typename T>
-static void launch_ln(void *out, const void *in, const void *w, const void *b, int64_t rows, int hidden,
-                      int64_t in_row_stride, float eps, const LnGlue &glue, hipStream_t s) {
-  const int chunks = (hidden + 7) / 8;
-  const float inv_hidden = 1.0f / (float)hidden;
-  const bool aligned = (hidden % 8 == 0) && (in_row_stride % 8 == 0 || rows == 1) && aligned16(in) &&
-                       aligned16(out) && (!w || aligned16(w)) && (!b || aligned16(b)) &&
-                       (!glue.z || (aligned16(glue.z) && (glue.z_row_stride_bytes % 16 == 0 || (rows == 1 && !glue.z_index))));
-  const bool plain = !glue.z && glue.activation == ARCTIC_ACT_NONE && glue.out_scale == 1.0f;
+static void launch_ln(LnParams p, int64_t rows, hipStream_t s) {
+  const int activation = p.activation, hidden = p.hidden, chunks = (hidden + 7) / 8;
+  const bool aligned = (hidden % 8 == 0) && (p.in_row_stride_bytes % 16 == 0 || rows == 1) && aligned16(p.in) &&
+                       aligned16(p.out) && aligned16(p.weight) && aligned16(p.bias) &&   /* null counts as aligned */
+                       (!p.z || (aligned16(p.z) && (p.z_row_stride_bytes % 16 == 0 || (rows == 1 && !p.z_index))));
+  const bool plain = !p.z && activation == ARCTIC_ACT_NONE && p.out_scale == 1.0f;
   const dim3 grid((unsigned)rows);
   // Rows that are not 16-byte aligned take the same kernel with accesses at any alignment.  Us per call in a graph, element
   // by element / in chunks: 300 x 1537 fp16 5.5 / 3.3, 64 x 4096 pitched by 4099 7.0 / 2.7, 4000 x 4097 34.6 / 17.5 (3.7
@@ -198,10 +204,9 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
     while (cpt < 8 && (chunks + cpt - 1) / cpt > 1024) cpt *= 2;
     int threads = (chunks + cpt - 1) / cpt;
     threads = std::max(64, (threads + 63) & ~63);
-    const int64_t stride_bytes = in_row_stride * 2;
-#define ARCTIC_LN_LAUNCH_AS(CPT, GLUE, ANY)                                                                       \
-  hipLaunchKernelGGL((spec_ln_vec_kernel<T, CPT, GLUE, ANY>), grid, dim3(threads), 0, s, (char *)out,             \
-                     (const char *)in, (const char *)w, (const char *)b, stride_bytes, hidden, inv_hidden, eps, glue)
+    p.waves = threads / 64;
+#define ARCTIC_LN_LAUNCH_AS(CPT, GLUE, ANY) \
+  launch(spec_ln_vec_kernel<T, CPT, GLUE, ANY>, grid, threads, s, p)
 #define ARCTIC_LN_LAUNCH_GLUE(CPT, GLUE)                    \
   do {                                                      \
     if (aligned) ARCTIC_LN_LAUNCH_AS(CPT, GLUE, false);     \
@@ -210,8 +215,8 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
 #define ARCTIC_LN_LAUNCH(CPT)                                                                          \
   do {                                                                                                 \
     if (plain) ARCTIC_LN_LAUNCH_GLUE(CPT, kPlain);                                                     \
-    else if (glue.activation == ARCTIC_ACT_NONE) ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_NONE);          \
-    else if (glue.activation == ARCTIC_ACT_GELU) ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_GELU);          \
+    else if (activation == ARCTIC_ACT_NONE) ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_NONE);          \
+    else if (activation == ARCTIC_ACT_GELU) ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_GELU);          \
     else ARCTIC_LN_LAUNCH_GLUE(CPT, ARCTIC_ACT_GELU_TANH);                                             \
   } while (0)
     switch (cpt) {
@@ -224,15 +229,24 @@ static void launch_ln(void *out, const void *in, const void *w, const void *b, i
 #undef ARCTIC_LN_LAUNCH_GLUE
 #undef ARCTIC_LN_LAUNCH_AS
   } else {
-    hipLaunchKernelGGL((spec_ln_scalar_kernel<T>), grid, dim3(256), 0, s, (uint16_t *)out,
-                       (const uint16_t *)in, (const uint16_t *)w, (const uint16_t *)b, in_row_stride, hidden,
-                       inv_hidden, eps, glue);
+    launch(spec_ln_scalar_kernel<T>, grid, kScalarLanes, s, p);
   }
 }
 
 }  // namespace arctic
 
 using namespace arctic;
+
+// What surrounds the norm, as in LnParams.
+struct LnGlue {
+  const char *z;
+  int64_t z_row_stride_bytes;
+  const int64_t *z_index;
+  int64_t z_rows;
+  float alpha;
+  int activation;
+  float out_scale;
+};
 
 static int ln_entry(const char *fn, void *out, const void *in, const void *weight, const void *bias,
                     int64_t rows, int hidden, int64_t in_row_stride, float eps, const LnGlue &glue, int dtype,
@@ -249,11 +263,12 @@ static int ln_entry(const char *fn, void *out, const void *in, const void *weigh
   if (!out || !in) return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: null tensor pointer", fn);
   if (!pitch_ok(in_row_stride, rows, 2) || !pitch_ok(hidden, rows, 2))
     return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: row pitch out of range", fn);
+  const LnParams p = {(char *)out, (const char *)in, (const char *)weight, (const char *)bias, glue.z, glue.z_index,
+                      in_row_stride * 2, glue.z_row_stride_bytes, glue.z_rows, hidden, 0, 1.0f / (float)hidden, eps,
+                      glue.alpha, glue.out_scale, glue.activation};
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == ARCTIC_DTYPE_BF16)
-    launch_ln<BF16>(out, in, weight, bias, rows, hidden, in_row_stride, eps, glue, s);
-  else
-    launch_ln<F16>(out, in, weight, bias, rows, hidden, in_row_stride, eps, glue, s);
+  if (dtype == ARCTIC_DTYPE_BF16) launch_ln<BF16>(p, rows, s);
+  else launch_ln<F16>(p, rows, s);
   return check_launch(fn);
 }
 

@@ -25,6 +25,9 @@
 
 namespace arctic {
 
+// A launch's arguments (common.hpp has what their size costs): 112 bytes with pitches and rows of 32 bits, as the vector
+// kernels take them, 120 with an embedding lookup.
+template <typename Size>
 struct LstmParams {
   char *out_state;
   char *out_cell;
@@ -35,19 +38,32 @@ struct LstmParams {
   const char *b_cell;
   const char *w_state;
   const char *b_state;
-  const int64_t *z_index;  // shared-z only: row of z4 to use for each row (an embedding lookup); nullptr = the row itself
-  int64_t z_rows;          // rows of z4 when z_index is given; an index is clamped into [0, z_rows)
-  int64_t s_stride;   // all strides in elements
-  int64_t z_stride;
-  int64_t pc_stride;
-  int64_t out_stride;
-  int64_t rows;
+  Size s_stride;   // all strides in elements
+  Size z_stride;
+  Size pc_stride;
+  Size out_stride;
+  Size z_rows;     // rows of z4 when z_index is given; an index is clamped into [0, z_rows)
   int D;
-  float inv_D;        // 1 / D
+  float inv_D;     // 1 / D
   float alpha;
   float eps_cell;
   float eps_state;
 };
+template <typename Size>
+struct LstmSharedParams : LstmParams<Size> {
+  const int64_t *z_index;  // row of z4 to use for each row (an embedding lookup); nullptr = the row itself
+};
+template <bool kSharedZ>
+using LstmParamsOf = std::conditional_t<kSharedZ, LstmSharedParams<uint32_t>, LstmParams<uint32_t>>;
+using LstmCall = LstmSharedParams<int64_t>;   // what an entry point was given
+
+// The row of z4 that a row adds.
+template <bool kSharedZ, typename Params>
+__device__ __forceinline__ int64_t z_row_of(const Params &p, int64_t row) {
+  if constexpr (kSharedZ)
+    if (p.z_index) return min(max(p.z_index[row], (int64_t)0), (int64_t)p.z_rows - 1);
+  return row;
+}
 
 // kFullWaves: rows 16-byte aligned, all four scale / shift vectors given, every lane of every wave owns a chunk of 8
 // elements; kRagged: the same with lanes to spare in the last wave; kAnyRow: everything else - vectors missing, rows
@@ -88,7 +104,7 @@ struct LstmRow {
 };
 
 template <typename T, int K, bool kFastGelu, bool kSharedZ, bool kAnyAlignment, bool kBare>
-__global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const LstmParams p) {
+__global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const LstmParamsOf<kSharedZ> p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
   constexpr int E = Chunk::kElems;
@@ -96,8 +112,9 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
   const int D = p.D;
   const int64_t gate_bytes = (int64_t)D * 2;
   Place at[K];
+  const int waves = (((D + 7) / 8 + K - 1) / K + 63) / 64;   // of the workgroup, as launched
 #pragma unroll
-  for (int k = 0; k < K; ++k) at[k] = Place(threadIdx.x + k * blockDim.x, D);
+  for (int k = 0; k < K; ++k) at[k] = Place(threadIdx.x + k * waves * 64, D);
   auto load = [](const char *q) { return C::load_stream<kAnyAlignment>(q); };
   auto vector = [](const C &given, float (&f)[E], float absent) {
     if constexpr (!kBare) given.template unpack<T>(f);
@@ -121,9 +138,7 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
   LstmRow<K> r;
   {
     const char *s_row = p.states + row * p.s_stride * 2;
-    int64_t zr = row;
-    if (kSharedZ && p.z_index) zr = min(max(p.z_index[row], (int64_t)0), p.z_rows - 1);
-    const char *z_row = p.z4 + zr * p.z_stride * 2;
+    const char *z_row = p.z4 + z_row_of<kSharedZ>(p, row) * p.z_stride * 2;
     const char *pc_row = p.prev_cell ? p.prev_cell + row * p.pc_stride * 2 : s_row;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -167,7 +182,7 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
       if (j >= at[k].repeated) ss = fmaf(cact[k][j], cact[k][j], ss);
     }
   }
-  const float inv_cpre = rsqrtf(block_sum(ss, slots_cpre) * p.inv_D + p.eps_cell);
+  const float inv_cpre = rsqrtf(block_sum(ss, slots_cpre, waves) * p.inv_D + p.eps_cell);
   // candidate = gelu(rmsnorm(pre_c)): runs while the other gates are still arriving
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -205,7 +220,7 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
     if (at[k].live()) packed.template store_stream<kAnyAlignment>(oc_row + at[k].off);
     packed.template unpack<T>(cell[k]);
   }
-  const float inv_cnew = rsqrtf(block_sum(ss, slots_cnew) * p.inv_D + p.eps_state);
+  const float inv_cnew = rsqrtf(block_sum(ss, slots_cnew, waves) * p.inv_D + p.eps_state);
 
   // phase 3: state = gelu(rmsnorm(rounded cell)) * sigmoid(pre_o) (reference :160-190);
   // the output gate is the last load to arrive and is consumed last
@@ -245,7 +260,7 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
 //
 // kZeroCell: the previous cell is all zeros (the first step of a proposal round) and is not read.
 template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, RowKind kKind>
-__global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParams p) {
+__global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParamsOf<kSharedZ> p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
   constexpr int E = Chunk::kElems;
@@ -253,15 +268,14 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParams 
   using std::integral_constant;
   const int64_t row = blockIdx.x;
   constexpr bool kAny = kKind == kAnyRow;
+  const int waves = ((p.D + 7) / 8 + 63) / 64;   // of the workgroup, as launched
   // the barriers need every wave, so the lanes behind the last chunk run along on it
   const Place at(threadIdx.x, kKind == kFullWaves ? INT32_MAX : p.D);
   const uint32_t off = at.off;
   auto load = [off](const char *q) { return C::load_stream<kAny>(q + off); };
   const int64_t gate_bytes = (int64_t)p.D * 2;
   const char *s_row = p.states + row * p.s_stride * 2;
-  int64_t zr = row;
-  if (kSharedZ && p.z_index) zr = min(max(p.z_index[row], (int64_t)0), p.z_rows - 1);
-  const char *z_row = p.z4 + zr * p.z_stride * 2;
+  const char *z_row = p.z4 + z_row_of<kSharedZ>(p, row) * p.z_stride * 2;
   const char *pc_row = kZeroCell ? s_row : p.prev_cell + row * p.pc_stride * 2;
   char *oc_row = p.out_cell + row * p.out_stride * 2;
   char *os_row = p.out_state + row * p.out_stride * 2;
@@ -297,7 +311,7 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParams 
     if (!kAny || j >= at.repeated) ss = fmaf(cact[j], cact[j], ss);
   }
   request(integral_constant<int, 2>(), integral_constant<int, 3>());
-  const float inv_cpre = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cpre) * p.inv_D + p.eps_cell);
+  const float inv_cpre = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cpre, waves) * p.inv_D + p.eps_cell);
   {
     float w[E], sh[E];
     wc.template unpack<T>(w);
@@ -333,7 +347,7 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParams 
     packed.template unpack<T>(cell);   // the state phase sees the rounded cell (:163,174)
   }
   request(integral_constant<int, 7>(), integral_constant<int, 9>());
-  const float inv_cnew = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cnew) * p.inv_D + p.eps_state);
+  const float inv_cnew = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cnew, waves) * p.inv_D + p.eps_state);
 
   // phase 3: state = gelu(rmsnorm(rounded cell)) * sigmoid(pre_o) (reference :160-190)
   float st[E];
@@ -354,16 +368,18 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParams 
 
 // Any D, any alignment: element-wise, three passes like the reference's scalar
 // kernel (sum_lstm.cu:193-291).
+constexpr int kScalarLanes = 256;
+struct LstmScalarParams : LstmCall {
+  int z_gate_stride;   // elements between two gates of z4: 0 when they share one
+};
 template <typename T, bool kFastGelu>
-__global__ __launch_bounds__(256) void sum_lstm_scalar_kernel(const LstmParams p, const int z_gate_stride) {
+__global__ __launch_bounds__(kScalarLanes) void sum_lstm_scalar_kernel(const LstmScalarParams p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
   const int D = p.D;
   const int64_t row = blockIdx.x;
   const uint16_t *s = (const uint16_t *)p.states + row * p.s_stride;
-  int64_t zr = row;
-  if (p.z_index) zr = min(max(p.z_index[row], (int64_t)0), p.z_rows - 1);
-  const uint16_t *z = (const uint16_t *)p.z4 + zr * p.z_stride;
+  const uint16_t *z = (const uint16_t *)p.z4 + z_row_of<true>(p, row) * p.z_stride;
   const uint16_t *pc = (const uint16_t *)p.prev_cell + row * p.pc_stride;
   uint16_t *oc = (uint16_t *)p.out_cell + row * p.out_stride;
   uint16_t *os = (uint16_t *)p.out_state + row * p.out_stride;
@@ -371,17 +387,17 @@ __global__ __launch_bounds__(256) void sum_lstm_scalar_kernel(const LstmParams p
   const uint16_t *ws = (const uint16_t *)p.w_state, *bs = (const uint16_t *)p.b_state;
 
   float ss = 0.f;
-  for (int j = threadIdx.x; j < D; j += blockDim.x) {
-    const float c = T::lo(s[3 * (int64_t)D + j]) + p.alpha * T::lo(z[3 * (int64_t)z_gate_stride + j]);
+  for (int j = threadIdx.x; j < D; j += kScalarLanes) {
+    const float c = T::lo(s[3 * (int64_t)D + j]) + p.alpha * T::lo(z[3 * (int64_t)p.z_gate_stride + j]);
     ss += c * c;
   }
-  const float inv_cpre = rsqrtf(block_sum(ss, slots_cpre) * p.inv_D + p.eps_cell);
+  const float inv_cpre = rsqrtf(block_sum(ss, slots_cpre, kScalarLanes / 64) * p.inv_D + p.eps_cell);
 
   ss = 0.f;
-  for (int j = threadIdx.x; j < D; j += blockDim.x) {
+  for (int j = threadIdx.x; j < D; j += kScalarLanes) {
     const float pre_f = T::lo(s[j]) + p.alpha * T::lo(z[j]);
-    const float pre_i = T::lo(s[(int64_t)D + j]) + p.alpha * T::lo(z[(int64_t)z_gate_stride + j]);
-    const float cpre = T::lo(s[3 * (int64_t)D + j]) + p.alpha * T::lo(z[3 * (int64_t)z_gate_stride + j]);
+    const float pre_i = T::lo(s[(int64_t)D + j]) + p.alpha * T::lo(z[(int64_t)p.z_gate_stride + j]);
+    const float cpre = T::lo(s[3 * (int64_t)D + j]) + p.alpha * T::lo(z[3 * (int64_t)p.z_gate_stride + j]);
     float cn = cpre * inv_cpre;
     if (wc) cn *= T::lo(wc[j]);
     if (bc) cn += T::lo(bc[j]);
@@ -389,14 +405,14 @@ __global__ __launch_bounds__(256) void sum_lstm_scalar_kernel(const LstmParams p
     ss += cnew * cnew;
     oc[j] = (uint16_t)T::round_bits(cnew);
   }
-  const float inv_cnew = rsqrtf(block_sum(ss, slots_cnew) * p.inv_D + p.eps_state);
+  const float inv_cnew = rsqrtf(block_sum(ss, slots_cnew, kScalarLanes / 64) * p.inv_D + p.eps_state);
 
   // each thread re-reads only the out_cell elements it wrote itself
-  for (int j = threadIdx.x; j < D; j += blockDim.x) {
+  for (int j = threadIdx.x; j < D; j += kScalarLanes) {
     float cn = T::lo(oc[j]) * inv_cnew;
     if (ws) cn *= T::lo(ws[j]);
     if (bs) cn += T::lo(bs[j]);
-    const float pre_o = T::lo(s[2 * (int64_t)D + j]) + p.alpha * T::lo(z[2 * (int64_t)z_gate_stride + j]);
+    const float pre_o = T::lo(s[2 * (int64_t)D + j]) + p.alpha * T::lo(z[2 * (int64_t)p.z_gate_stride + j]);
     os[j] = (uint16_t)T::round_bits(gelu<kFastGelu>(cn) * sigmoid_f(pre_o));
   }
 }
@@ -405,7 +421,7 @@ static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 // Whether an output shares memory with a gate or the previous cell: `columns` elements of each of `rows` rows, `stride`
 // elements apart, looked at as whole ranges.
-static bool in_place(const LstmParams &p, int64_t rows, bool shared_z) {
+static bool in_place(const LstmCall &p, int64_t rows, bool shared_z) {
   const auto overlaps = [&](const char *out, const char *in, int64_t in_rows, int64_t stride, int64_t columns) {
     const uintptr_t o = (uintptr_t)out, i = (uintptr_t)in;
     return in && o < i + (uintptr_t)((in_rows - 1) * stride + columns) * 2 &&
@@ -420,7 +436,7 @@ static bool in_place(const LstmParams &p, int64_t rows, bool shared_z) {
 }
 
 template <typename T, bool kFastGelu, bool kSharedZ>
-static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
+static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   const bool multi = rows > 1;
   const bool aligned = p.D % 8 == 0 &&
                        (!multi || (p.s_stride % 8 == 0 && p.z_stride % 8 == 0 && p.pc_stride % 8 == 0 &&
@@ -443,7 +459,7 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
   // 256 3.07 / 3.24); with all vectors and more than 256 rows it is chunks from 129 on (300 x 136 level, 512 x 160 7 % and
   // 2048 x 256 8 % faster).  From 257 on chunks are faster at every row count (64 x 257 by 10 to 23 %, 64 x 513 by 21 to 35).
 #define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND) \
-  hipLaunchKernelGGL((sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND>), grid, dim3(lanes), 0, s, p)
+  launch(sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND>, grid, lanes, s, compact)
 #define ARCTIC_LSTM_STAGED(KIND)                                    \
   do {                                                              \
     if (p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND);        \
@@ -456,33 +472,44 @@ static void launch_lstm(const LstmParams &p, int64_t rows, hipStream_t s) {
   // and nothing orders the one's load before the other's store: such a call goes element by element.  Aligned rows that
   // lack a vector are requested together, since the stages read the output gate behind the first store.
   const bool aliased = (p.D % 8 || !all_vectors) && in_place(p, rows, kSharedZ);
-  const bool element_wise = narrow || (aliased && p.D % 8);
+  // (strides and rows of 2^32 elements and more are the element-wise kernel's: the others' arguments are 32 bits wide)
+  const auto fits = [](int64_t v) { return v <= (int64_t)UINT32_MAX; };
+  const bool wide = (multi && !(fits(p.s_stride) && fits(p.pc_stride) && fits(p.out_stride))) ||
+                    ((multi || p.z_index) && !fits(p.z_stride)) || !fits(p.z_rows);
+  const bool element_wise = narrow || (aliased && p.D % 8) || wide || chunks > 2 * 1024;
+  LstmParamsOf<kSharedZ> compact;
+  static_cast<LstmParams<uint32_t> &>(compact) = {
+      p.out_state, p.out_cell, p.states, p.z4, p.prev_cell, p.w_cell, p.b_cell, p.w_state, p.b_state, (uint32_t)p.s_stride,
+      (uint32_t)p.z_stride, (uint32_t)p.pc_stride, (uint32_t)p.out_stride, (uint32_t)p.z_rows, p.D, p.inv_D, p.alpha,
+      p.eps_cell, p.eps_state};
+  if constexpr (kSharedZ) compact.z_index = p.z_index;
   // Aligned rows of up to 2048 elements that lack a vector: at most four waves per row, whose loads are few enough to be
   // requested together.  Us per call in a graph, in stages (ones and zeros read in place of an absent vector) / together:
   // 64 x 256 without vectors 4.0 / 3.2, 512 x 512 4.2 / 3.3, 300 x 2048 5.6 / 4.8, 512 x 512 with the scales alone 4.1 / 3.4;
   // from 513 elements and 513 rows on the stages are faster (2048 x 1024 8.8 / 9.4), but for one z for all gates (8.4 / 7.7).
   const bool together = aligned && !all_vectors && chunks <= 256 && (chunks <= 64 || rows <= 512 || kSharedZ);
 #define ARCTIC_LSTM_VEC_LAUNCH(K, ANY, BARE) \
-  hipLaunchKernelGGL((sum_lstm_vec_kernel<T, K, kFastGelu, kSharedZ, ANY, BARE>), grid, dim3(threads), 0, s, p)
+  launch(sum_lstm_vec_kernel<T, K, kFastGelu, kSharedZ, ANY, BARE>, grid, threads, s, compact)
 #define ARCTIC_LSTM_VEC(K, ANY)                                       \
   do {                                                                \
     const int threads = ((chunks + (K) - 1) / (K) + 63) & ~63;        \
     if (p.w_cell || p.b_cell || p.w_state || p.b_state) ARCTIC_LSTM_VEC_LAUNCH(K, ANY, false); \
     else ARCTIC_LSTM_VEC_LAUNCH(K, ANY, true);                        \
   } while (0)
-  if (together) {
+  if (element_wise) {
+    launch(sum_lstm_scalar_kernel<T, kFastGelu>, grid, kScalarLanes, s, LstmScalarParams{p, kSharedZ ? 0 : p.D});
+  } else if (together) {
     ARCTIC_LSTM_VEC(1, false);
-  } else if (aliased && aligned && chunks <= 2 * 1024) {
+  } else if (aliased && aligned) {
     ARCTIC_LSTM_VEC(2, false);
-  } else if (!element_wise && chunks <= 1024) {
+  } else if (chunks <= 1024) {
     if (!aligned || !all_vectors) ARCTIC_LSTM_STAGED(kAnyRow);
     else if (lanes != chunks) ARCTIC_LSTM_STAGED(kRagged);
     else ARCTIC_LSTM_STAGED(kFullWaves);
-  } else if (!element_wise && chunks > 1024 && chunks <= 2 * 1024) {
-    if (aligned) ARCTIC_LSTM_VEC(2, false);
-    else ARCTIC_LSTM_VEC(2, true);
+  } else if (aligned) {
+    ARCTIC_LSTM_VEC(2, false);
   } else {
-    hipLaunchKernelGGL((sum_lstm_scalar_kernel<T, kFastGelu>), grid, dim3(256), 0, s, p, kSharedZ ? 0 : p.D);
+    ARCTIC_LSTM_VEC(2, true);
   }
 #undef ARCTIC_LSTM_VEC
 #undef ARCTIC_LSTM_VEC_LAUNCH
@@ -511,7 +538,7 @@ static int sum_lstm_entry(const char *fn, bool shared_z, void *out_state, void *
   if (!pitch_ok(s_stride, rows, 2) || !pitch_ok(z_stride, z_index ? z_rows : rows, 2) ||
       !pitch_ok(pc_stride, rows, 2) || !pitch_ok(out_stride, rows, 2))
     return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: row pitch out of range", fn);
-  LstmParams p;
+  LstmCall p;
   p.z_index = z_index;
   p.z_rows = z_rows;
   p.out_state = (char *)out_state;
@@ -527,7 +554,6 @@ static int sum_lstm_entry(const char *fn, bool shared_z, void *out_state, void *
   p.z_stride = z_stride;
   p.pc_stride = prev_cell ? pc_stride : 0;
   p.out_stride = out_stride;
-  p.rows = rows;
   p.D = D;
   p.inv_D = 1.0f / (float)D;
   p.alpha = alpha;

@@ -74,6 +74,14 @@ def test_places_of_chunks_slots_and_workgroups(ops, kv, shape):
     run_both(ops, make_bulk_case(kv_cache_dtype=kv, seed=19, std=1.5, **shape))
 
 
+@pytest.mark.parametrize("L", [15, 16, 17, 64, 65])
+@pytest.mark.parametrize("heads_of", [dict(H=2, D=64), dict(H=3, D=80)])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+def test_layers_at_the_edges_of_the_pointer_tables(ops, L, heads_of, kv):
+    """Up to 16 layers travel in tables of 16, up to 64 in tables of 64, more in several launches."""
+    run_both(ops, make_bulk_case(T=6, L=L, bs=16, NB=2, kv_cache_dtype=kv, seed=23, std=1.5, pad_fraction=0.2, **heads_of))
+
+
 def test_all_padding_leaves_cache_untouched(ops):
     case = make_bulk_case(T=16, L=3, H=2, D=64, bs=16, NB=4, kv_cache_dtype="fp8", seed=7)
     case["slot_mapping"].fill_(-1)

@@ -89,6 +89,23 @@ def test_sum_lstm_beyond_four_gib(ops):
         assert bool(out.view(torch.int16).ne(0).any(dim=1).all())
 
 
+@pytest.mark.parametrize("pitch", [(1 << 32) - 8, 1 << 32])
+def test_sum_lstm_row_pitch_around_32_bits(ops, pitch):
+    """The vector kernels take pitches of 32 bits; the element-wise one takes what lies beyond."""
+    D = 512
+    memory = torch.empty(pitch + 4 * D, dtype=torch.bfloat16, device=DEV)
+    states = memory.as_strided((2, 4 * D), (pitch, 1))
+    g = torch.Generator().manual_seed(18)
+    s, z4, cell = (torch.randn(2, n, generator=g).to(torch.bfloat16) for n in (4 * D, 4 * D, D))
+    states.copy_(s)
+    w_cell, b_cell, w_state, b_state = ((m + 0.02 * torch.randn(D, generator=g)).to(torch.bfloat16) for m in (1.0, 0.0, 1.0, 0.0))
+    got_s, got_c = ops.sum_lstm(states, z4.to(DEV), cell.to(DEV), w_cell.to(DEV), b_cell.to(DEV), w_state.to(DEV),
+                                b_state.to(DEV), 0.35, 1e-6, 1e-6, False)
+    want_s, want_c = oracle.sum_lstm(s, z4, cell, w_cell, b_cell, w_state, b_state, 0.35, 1e-6, 1e-6, False)
+    assert_close(got_c.cpu(), want_c, RTOL, ATOL, "cell")
+    assert_close(got_s.cpu(), want_s, RTOL, ATOL, "state")
+
+
 def test_speculator_ln_beyond_four_gib(ops):
     rows, hidden = 270_000, 8192                       # 4.4 GB in, 4.4 GB out
     x = randn_bf16(rows, hidden, 18)
