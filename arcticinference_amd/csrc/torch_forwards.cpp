@@ -12,8 +12,11 @@
 //   sum_lstm_cuda                  csrc/custom_ops/sum_lstm.cu:293-473
 // allocates outputs as it does, and hands pointers, sizes and strides to the library on torch's current stream.
 // Checks that the reference leaves out (it would read or write out of bounds instead) are marked as such.
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/hip/HIPFunctions.h>
 #include <torch/all.h>
 
 #include <string>
@@ -26,9 +29,45 @@
 namespace arctic_host {
 namespace {
 
-using DeviceGuard = c10::hip::OptionalHIPGuardMasqueradingAsCUDA;
+// Makes a tensor's device the current one for a launch.  Asking which it is costs half of what the guard does, and nearly
+// always it is that one already.
+class OnDevice {
+ public:
+  explicit OnDevice(const at::Tensor &t) : index_(t.device().index()) {
+    if (c10::hip::current_device() != index_) guard_.set_device(t.device());
+  }
+  void *stream() const { return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(index_).stream(); }
 
-void *current_stream() { return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
+ private:
+  const c10::DeviceIndex index_;
+  c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard_;
+};
+
+// Outputs, without the dispatcher where nothing listens to it: 0.47 us a tensor instead of 0.73.  `like` must be an
+// ordinary tensor of the GPU, and no mode (a Python dispatch mode, a functorch transform, tracing) may be on.
+bool undispatched(const at::Tensor &like) {
+  using c10::DispatchKey;
+  constexpr c10::DispatchKeySet kOrdinary({DispatchKey::Dense, DispatchKey::CUDA, DispatchKey::ADInplaceOrView,
+                                           DispatchKey::AutogradCUDA, DispatchKey::AutocastCUDA});
+  constexpr c10::DispatchKeySet kAlwaysOn({DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView});
+  return (like.key_set() - kOrdinary).empty() && (c10::impl::tls_local_dispatch_key_set().included_ - kAlwaysOn).empty() &&
+         !at::globalContext().deterministicAlgorithms();   // under which new memory is filled
+}
+at::Tensor new_empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor &like) {
+  if (undispatched(like)) return at::detail::empty_cuda(sizes, dtype, like.device(), c10::nullopt);
+  return at::empty(sizes, like.options().dtype(dtype));
+}
+at::Tensor new_empty_strided(at::IntArrayRef sizes, at::IntArrayRef strides, const at::Tensor &like) {
+  if (undispatched(like)) return at::detail::empty_strided_cuda(sizes, strides, like.scalar_type(), like.device());
+  return at::empty_strided(sizes, strides, like.options());
+}
+// at::empty_like: of a matrix whose rows are `cols` or more apart that is a dense one.
+at::Tensor new_like(const at::Tensor &t) {
+  if (t.dim() == 2 && t.size(0) >= 1 && t.size(1) > 1 && t.stride(1) == 1 &&
+      (t.size(0) == 1 ? t.stride(0) == t.size(1) : t.stride(0) >= t.size(1)))
+    return new_empty(t.sizes(), t.scalar_type(), t);
+  return at::empty_like(t);
+}
 
 const void *optional_ptr(const OptTensor &t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
@@ -84,16 +123,18 @@ CheckedLayers check_layers(const LayerLists &layers) {
   c.cache_element_size = first.element_size();
   c.device = first.device();
   const auto dtype0 = first.scalar_type();
-  c.key_caches.resize(num_layers);
-  c.value_caches.resize(num_layers);
+  c.key_caches.assign(num_layers, nullptr);
+  c.value_caches.assign(num_layers, nullptr);
   c.k_scales.assign(num_layers, nullptr);
   c.v_scales.assign(num_layers, nullptr);
   for (int64_t l = 0; l < num_layers; ++l) {
     const at::Tensor &k = layers(0, l), &v = layers(1, l);
-    TORCH_CHECK(k.scalar_type() == dtype0 && v.scalar_type() == dtype0 && k.stride(0) == c.block_stride &&
-                    v.stride(0) == c.block_stride && k.size(0) == c.num_blocks && v.size(0) == c.num_blocks &&
-                    k.size(1) == c.block_size && v.size(1) == c.block_size && k.device() == c.device &&
-                    v.device() == c.device,
+    const auto like_first = [&](const at::Tensor &t) {
+      const at::IntArrayRef sizes = t.sizes();
+      return sizes.size() >= 2 && t.scalar_type() == dtype0 && t.strides()[0] == c.block_stride && sizes[0] == c.num_blocks &&
+             sizes[1] == c.block_size && t.device() == c.device;
+    };
+    TORCH_CHECK(like_first(k) && like_first(v),
                 "reshape_and_cache_flash_bulk: key and value caches of all layers must share dtype, block stride, "
                 "number of blocks, block size and device");
     c.key_caches[l] = k.data_ptr();
@@ -205,8 +246,8 @@ void bulk_write(const at::Tensor &keys, const at::Tensor &values, const CheckedL
 
   const int layer_count = to_int(num_layers, "num_layers"), heads = to_int(num_heads, "num_heads");
   const int head = to_int(head_size, "head_size"), block = to_int(layers.block_size, "block_size");
-  const DeviceGuard guard(keys.device());
-  void *stream = current_stream();
+  const OnDevice device(keys);
+  void *stream = device.stream();
   if (!select) {
     check_rc(arctic_reshape_and_cache_flash_bulk(
         keys.data_ptr(), values.data_ptr(), keys.stride(0), values.stride(0), layers.key_caches.data(),
@@ -219,7 +260,7 @@ void bulk_write(const at::Tensor &keys, const at::Tensor &values, const CheckedL
   // ARCTIC_SELECT_SCAN_MAX_INDICES entries every token's workgroup scans the list itself and nothing is allocated.
   at::Tensor row_map;
   if (n_sel > ARCTIC_SELECT_SCAN_MAX_INDICES) {
-    row_map = at::empty({num_tokens}, keys.options().dtype(at::kLong));
+    row_map = new_empty({num_tokens}, at::kLong, keys);
     check_rc(arctic_build_row_map((int64_t *)row_map.data_ptr(), num_tokens, idx.data_ptr(), (int)idx.element_size(), n_sel,
                                   stream));
   }
@@ -275,13 +316,13 @@ void cache_write_fp4(const at::Tensor &key, const at::Tensor &value, const at::T
   TORCH_CHECK(slot_mapping.dim() == 1 && (slot_mapping.size(0) <= 1 || slot_mapping.stride(0) == 1) &&
                   key.size(0) >= slot_mapping.size(0),
               "reshape_and_cache_flash_fp4: slot_mapping must be 1-D, contiguous and no longer than key has tokens");
-  const DeviceGuard guard(key.device());
+  const OnDevice device(key);
   check_rc(arctic_reshape_and_cache_flash_fp4(
       key.data_ptr(), value.data_ptr(), key.stride(0), value.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
       key_scale_cache.data_ptr(), value_scale_cache.data_ptr(), (const int64_t *)slot_mapping.data_ptr(),
       slot_mapping.size(0), to_int(num_heads, "num_heads"), to_int(head_size, "head_size"),
       to_int(block_size, "block_size"), block_stride, page_stride, head_stride, key_cache.size(0), half_code(key),
-      current_stream()));
+      device.stream()));
 }
 
 namespace {
@@ -344,25 +385,25 @@ at::Tensor add_ln_act(const char *fn, const at::Tensor &input, const OptTensor &
     TORCH_CHECK(z->stride(-1) == 1, fn, ": last dimension of z must be contiguous");
     z_2d = rows_of(*z, hidden);
   }
-  at::Tensor out = at::empty_like(input);
+  at::Tensor out = new_like(input);
   if (rows == 0) return out;
   const at::Tensor out_2d = rows_of(out, hidden);   // rows are written dense, `hidden` apart
   TORCH_CHECK(out_2d.stride(0) == hidden || rows == 1, fn, ": internal - output rows must be dense");
-  const DeviceGuard guard(input.device());
+  const OnDevice device(input);
   const int code = half_code(input);
   if (given(token_ids)) {
     check_rc(arctic_speculator_embed_add_ln_act(
         out_2d.data_ptr(), in_2d.data_ptr(), z->data_ptr(), (const int64_t *)token_ids->data_ptr(), optional_ptr(weight),
         optional_ptr(bias), rows, to_int(hidden, "hidden"), in_2d.stride(0), z->stride(0), z->size(0), (float)alpha,
-        (float)eps, act, (float)out_scale, code, current_stream()));
+        (float)eps, act, (float)out_scale, code, device.stream()));
   } else if (!z_2d.defined() && act == ARCTIC_ACT_NONE && out_scale == 1.0) {
     check_rc(arctic_speculator_ln(out_2d.data_ptr(), in_2d.data_ptr(), optional_ptr(weight), optional_ptr(bias), rows,
-                                  to_int(hidden, "hidden"), in_2d.stride(0), (float)eps, code, current_stream()));
+                                  to_int(hidden, "hidden"), in_2d.stride(0), (float)eps, code, device.stream()));
   } else {
     check_rc(arctic_speculator_add_ln_act(out_2d.data_ptr(), in_2d.data_ptr(), z_2d.defined() ? z_2d.data_ptr() : nullptr,
                                           optional_ptr(weight), optional_ptr(bias), rows, to_int(hidden, "hidden"),
                                           in_2d.stride(0), z_2d.defined() ? z_2d.stride(0) : 0, (float)alpha, (float)eps,
-                                          act, (float)out_scale, code, current_stream()));
+                                          act, (float)out_scale, code, device.stream()));
   }
   return out;
 }
@@ -418,8 +459,8 @@ std::tuple<at::Tensor, at::Tensor> sum_lstm(const at::Tensor &states_4d, const a
   at::Tensor out_cell, out_state, cell_shaped, state_shaped;
   if (zero_cell) {
     // dense outputs shaped like states_4d with its last dimension cut to D_gate
-    out_cell = at::empty({rows, d_gate}, states_4d.options());
-    out_state = at::empty({rows, d_gate}, states_4d.options());
+    out_cell = new_empty({rows, d_gate}, states_4d.scalar_type(), states_4d);
+    out_state = new_empty({rows, d_gate}, states_4d.scalar_type(), states_4d);
     if (states_4d.dim() == 2) {
       cell_shaped = out_cell;
       state_shaped = out_state;
@@ -431,8 +472,8 @@ std::tuple<at::Tensor, at::Tensor> sum_lstm(const at::Tensor &states_4d, const a
     }
   } else {
     // outputs inherit prev_cell's row pitch (reference :356-365)
-    out_cell = at::empty_strided(p2.sizes(), p2.strides(), p2.options());
-    out_state = at::empty_strided(p2.sizes(), p2.strides(), p2.options());
+    out_cell = new_empty_strided(p2.sizes(), p2.strides(), p2);
+    out_state = new_empty_strided(p2.sizes(), p2.strides(), p2);
     TORCH_CHECK(out_cell.stride(0) == out_state.stride(0), "sum_lstm: internal - output strides mismatch");
     const bool flat = prev_cell_d->dim() == 2;
     cell_shaped = flat ? out_cell : out_cell.view(prev_cell_d->sizes());
@@ -442,20 +483,20 @@ std::tuple<at::Tensor, at::Tensor> sum_lstm(const at::Tensor &states_4d, const a
 
   const void *pc = zero_cell ? nullptr : p2.data_ptr();
   const int64_t pc_stride = zero_cell ? 0 : p2.stride(0);
-  const DeviceGuard guard(states_4d.device());
+  const OnDevice device(states_4d);
   const int code = half_code(states_4d);
   if (given(token_ids)) {
     check_rc(arctic_sum_lstm_embedded(
         out_state.data_ptr(), out_cell.data_ptr(), s2.data_ptr(), z.data_ptr(), (const int64_t *)token_ids->data_ptr(), pc,
         optional_ptr(w_cell), optional_ptr(b_cell), optional_ptr(w_state), optional_ptr(b_state), rows,
         to_int(d_gate, "d_gate"), s2.stride(0), z.stride(0), pc_stride, out_cell.stride(0), z.size(0), (float)alpha,
-        (float)eps_cell, (float)eps_state, use_fast_gelu ? 1 : 0, code, current_stream()));
+        (float)eps_cell, (float)eps_state, use_fast_gelu ? 1 : 0, code, device.stream()));
   } else {
     const auto entry = shared_z ? arctic_sum_lstm_shared_z : arctic_sum_lstm;
     check_rc(entry(out_state.data_ptr(), out_cell.data_ptr(), s2.data_ptr(), z2.data_ptr(), pc, optional_ptr(w_cell),
                    optional_ptr(b_cell), optional_ptr(w_state), optional_ptr(b_state), rows, to_int(d_gate, "d_gate"),
                    s2.stride(0), z2.stride(0), pc_stride, out_cell.stride(0), (float)alpha, (float)eps_cell,
-                   (float)eps_state, use_fast_gelu ? 1 : 0, code, current_stream()));
+                   (float)eps_state, use_fast_gelu ? 1 : 0, code, device.stream()));
   }
   return std::make_tuple(state_shaped, cell_shaped);
 }
@@ -496,10 +537,10 @@ void move_rows(const char *fn, const TensorList &sources, const at::Tensor &indi
     src_ptr[k] = src.data_ptr();
     dst_ptr[k] = dst.data_ptr();
   }
-  const DeviceGuard guard(indices.device());
+  const OnDevice device(indices);
   check_rc(arctic_gather_rows(to_int(count, "count"), src_ptr.data(), dst_ptr.data(), row_bytes.data(),
                               src_stride.data(), dst_stride.data(), indices.data_ptr(), (int)indices.element_size(), n,
-                              indexed_rows, scatter ? 1 : 0, current_stream()));
+                              indexed_rows, scatter ? 1 : 0, device.stream()));
 }
 
 at::Tensor argmax_clamp(const at::Tensor &logits, int64_t max_index) {
@@ -519,15 +560,14 @@ at::Tensor argmax_clamp(const at::Tensor &logits, int64_t max_index) {
   const at::Tensor in_2d = rows_of(logits, cols);
   const int64_t rows = in_2d.size(0);
   const auto shape = logits.sizes().slice(0, logits.dim() - 1);
-  const auto options = logits.options().dtype(at::kLong);
-  if (rows == 0) return at::empty(shape, options);
+  if (rows == 0) return new_empty(shape, at::kLong, logits);
   // a few long rows are split over workgroups that exchange their winners in memory behind the answers: one allocation
   const int64_t workspace = arctic_argmax_workspace_bytes(rows, to_int(cols, "cols"), code);
-  at::Tensor out = workspace ? at::empty({rows + (workspace + 7) / 8}, options) : at::empty(shape, options);
-  const DeviceGuard guard(logits.device());
+  at::Tensor out = workspace ? new_empty({rows + (workspace + 7) / 8}, at::kLong, logits) : new_empty(shape, at::kLong, logits);
+  const OnDevice device(logits);
   check_rc(arctic_argmax_clamp_split((int64_t *)out.data_ptr(), in_2d.data_ptr(), rows, (int)cols, in_2d.stride(0), max_index,
                                      code, workspace ? (int64_t *)out.data_ptr() + rows : nullptr, workspace,
-                                     current_stream()));
+                                     device.stream()));
   if (workspace) {
     // the answers keep the block, but what a caller saves, shares or looks at is their own size
     out.resize_(shape);

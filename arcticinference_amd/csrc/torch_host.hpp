@@ -4,6 +4,7 @@
 // four functions of the reference's custom_ops.h (same file) and by the Python extension module in host_ext.cpp.
 #pragma once
 
+#include <c10/util/SmallVector.h>
 #include <torch/all.h>
 
 #include <string>
@@ -37,8 +38,8 @@ struct CheckedLayers {
   int64_t num_layers = 0, block_size = 0, block_stride = 0, num_blocks = 0, cache_element_size = 0;
   c10::Device device = c10::Device(c10::kCPU);
   const char *scales_problem = nullptr;   // why the scales cannot serve an fp8 write, or nullptr
-  std::vector<const void *> key_caches, value_caches;
-  std::vector<const float *> k_scales, v_scales;
+  c10::SmallVector<const void *, 64> key_caches, value_caches;   // of models of up to 64 layers on the caller's stack
+  c10::SmallVector<const float *, 64> k_scales, v_scales;
 };
 CheckedLayers check_layers(const LayerLists &layers);
 

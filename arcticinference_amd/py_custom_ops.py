@@ -78,6 +78,8 @@ _torch_lib: Optional[torch.library.Library] = None
 _registered = False
 # operator name -> its host-side implementation (the functions of the _host_ext extension module)
 _IMPLS: dict = {}
+# _host_ext.on_gpu once the operators are registered: whether a tensor, or the first one of a list, is on a GPU
+_on_gpu = lambda tensor: False
 
 
 def _load_host_layer() -> None:
@@ -145,7 +147,7 @@ _META_IMPLS = {
 def _register_ops() -> None:
     """Define the four schemas and bind the CUDA key (the only key the reference
     binds, torch_bindings.cpp:17,32,37,50)."""
-    global _torch_lib, _registered
+    global _torch_lib, _registered, _on_gpu
     if _registered:
         return
     _load_host_layer()
@@ -155,6 +157,8 @@ def _register_ops() -> None:
         lib.impl(name, _IMPLS[name], "CUDA")
         lib.impl(name, _META_IMPLS[name], "Meta")
     _torch_lib = lib  # keep alive: dropping the Library object unregisters the ops
+    from . import _host_ext
+    _on_gpu = _host_ext.on_gpu
     _registered = True
 
 
@@ -207,11 +211,9 @@ def _call(name: str, *args):
     tensors and handing them back to Python) costs more host time than the whole call.  Under
     ``torch.compile`` the registered operator is used, so that the call stays one opaque node of the
     traced graph."""
-    ops = _ops()
-    first = args[0][0] if isinstance(args[0], (list, tuple)) and args[0] else args[0]
-    if _is_compiling() or not (isinstance(first, torch.Tensor) and first.is_cuda):
-        return getattr(ops, name)(*args)   # also the path on which non-GPU tensors are turned away
-    return _IMPLS[name](*args)
+    if not _is_compiling() and _on_gpu(args[0]):
+        return _IMPLS[name](*args)
+    return getattr(_ops(), name)(*args)   # also the path on which non-GPU tensors are turned away
 
 
 def reshape_and_cache_flash_bulk(

@@ -3,6 +3,7 @@ import ctypes
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import oracle
 from arcticinference_amd import _native
@@ -278,3 +279,51 @@ def test_reference_schemas_through_the_dispatcher(ops):
     oracle.reshape_and_cache_flash_fp4(key, value, caches[0], caches[1], caches[2], caches[3], slots, "fp4", one, one)
     for a, b in zip(dcaches, caches):
         assert torch.equal(a.cpu(), b)
+
+
+class CountedEmpties(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen += "empty" in str(func)
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("form", ["dense", "pitched", "one row", "one pitched row", "one column", "same row", "rank 3", "no rows"])
+def test_outputs_are_made_as_the_dispatcher_makes_them(ops, form):
+    """Outputs are allocated past the dispatcher where nothing listens to it: sizes, strides and types as with it, and a
+    dispatch mode sees the allocations still."""
+    H = 1 if form == "one column" else 64
+    memory = torch.randn(6, H + 16, device=DEV).bfloat16()
+    x = {"dense": lambda: memory[:, :H].contiguous(), "pitched": lambda: memory[:, :H], "one row": lambda: memory[:1, :H].contiguous(),
+         "one pitched row": lambda: memory.as_strided((1, H), (999, 1)), "one column": lambda: memory[:, :1].contiguous(),
+         "same row": lambda: memory[:1, :H].expand(6, H), "rank 3": lambda: memory[:, :H].contiguous().view(2, 3, H),
+         "no rows": lambda: memory[:0, :H]}[form]()
+    ids = torch.zeros(x.shape[:-1], dtype=torch.int64, device=DEV)
+    s4 = torch.randn(*x.shape[:-1], 4 * H, device=DEV).bfloat16()
+    table = torch.randn(3, H, device=DEV).bfloat16()
+
+    def outputs():
+        return [ops.speculator_ln(x, None, None, 1e-6), ops.speculator_embed_add_ln_gelu(x, table, ids, None, None, 0.5, 1e-6),
+                ops.speculator_argmax(x, H), *ops.sum_lstm_embedded(s4, table, ids, None, None, None, None, None, 0.5, 1e-6, 1e-6, False),
+                *(ops.sum_lstm(s4, s4, x, None, None, None, None, 0.5, 1e-6, 1e-6, False) if form != "same row" else [])]
+
+    got = outputs()
+    with CountedEmpties() as mode:
+        want = outputs()
+    assert mode.seen >= len(want)
+    with torch.inference_mode():
+        inferred = outputs()
+    torch.use_deterministic_algorithms(True)
+    try:
+        filled = outputs()
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert got[0].stride() == torch.empty_like(x).stride()
+    for others in (want, inferred, filled):
+        for a, b in zip(got, others):
+            assert a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype and a.device == b.device
+            assert torch.equal(a, b) and not b.requires_grad
+    assert all(t.is_inference() for t in inferred) and not any(t.is_inference() for t in got)

@@ -1,6 +1,7 @@
 """Host side of the drop-in operator surface (runs without a GPU)."""
 import re
 
+import numpy as np
 import pytest
 import torch
 
@@ -143,6 +144,41 @@ def test_no_host_pointer_reaches_a_launch(loaded):
     # sizes that do not fit the library's ints are an error, not a wrapped value
     with pytest.raises(RuntimeError, match="num_heads and head_size must be positive"):
         f["reshape_and_cache_flash_bulk"](x, x, [cache[0]], [cache[1]], slots, "auto", [x], [x], 1 << 40, 64)
+
+
+def test_arguments_of_other_types_are_refused(loaded):
+    """The host layer's functions take positional arguments of their schema's types: what converts to one is accepted (here
+    it gets as far as the check of the device), anything else is a TypeError."""
+    x, slots = torch.randn(4, 64).bfloat16(), torch.zeros(4, dtype=torch.int64)
+    ln, lstm, argmax = (ops._IMPLS[n] for n in ("speculator_add_ln_act_cuda", "sum_lstm_zero_cell_cuda", "speculator_argmax_cuda"))
+    good = [x, None, x, None, 1.0, 1e-6, "gelu", 1.0]
+    for at, others in ((0, [torch.nn.Parameter(x)]), (4, [1, np.float32(1.0), True]), (6, [b"gelu"])):
+        for other in others:
+            with pytest.raises(RuntimeError, match="input must be CUDA"):
+                ln(*good[:at], other, *good[at + 1:])
+    for at, others in ((0, [None, 1.0, [x]]), (1, [1.0, "x"]), (4, ["1.0", None, x]), (6, [None, 1.0]), (7, [[]])):
+        for other in others:
+            with pytest.raises((TypeError, RuntimeError), match="incompatible function arguments"):
+                ln(*good[:at], other, *good[at + 1:])
+    with pytest.raises(TypeError, match="8 arguments are needed, 7 were given"):
+        ln(*good[:-1])
+    with pytest.raises(TypeError):
+        ln(*good[:-1], out_scale=1.0)
+    for accepted in (63, True, np.int64(63), torch.tensor(63)):
+        with pytest.raises(RuntimeError, match="logits must be CUDA"):
+            argmax(x, accepted)
+    for refused in (63.0, "63", None, 1 << 70):
+        with pytest.raises(TypeError, match="incompatible function arguments"):
+            argmax(x, refused)
+    s4 = torch.randn(4, 256).bfloat16()
+    for accepted in (False, None, 0, np.bool_(True)):
+        with pytest.raises(RuntimeError, match="inputs must be CUDA tensors"):
+            lstm(s4, s4, None, None, None, None, 1.0, 1e-6, 1e-6, accepted)
+    for refused in ("no", []):
+        with pytest.raises(TypeError, match="incompatible function arguments"):
+            lstm(s4, s4, None, None, None, None, 1.0, 1e-6, 1e-6, refused)
+    with pytest.raises(TypeError):
+        ops._IMPLS["gather_rows"](None, slots, [x])
 
 
 def test_missing_library_fails_loudly(monkeypatch):
