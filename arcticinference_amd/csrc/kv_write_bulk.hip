@@ -219,8 +219,9 @@ __device__ __forceinline__ void select_leftover_rows(const BulkSelectParams &p, 
 }
 
 // kBulkThreads x kUnroll 16-byte chunks form one batch of a workgroup.  Three shapes are built, all with batches
-// of 1024 chunks: 1024 x 1 (launches of more than 8192 tokens: a workgroup moves up to five batches), 512 x 2 (the
-// same launches when rows are selected as well) and 256 x 4 (everything smaller: one or two batches per workgroup).
+// of 1024 chunks: 1024 x 1 (launches of more than 8192 tokens, or 4096 of rows that are no power of two long: a workgroup
+// moves up to five batches), 512 x 2 (launches of more than 8192 tokens that select rows as well) and 256 x 4 (everything
+// smaller: at most two batches per workgroup).
 template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, typename Params, typename Tables>
 __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, unsigned block) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
@@ -520,7 +521,8 @@ static void launch_vec_shape(const BulkSelectParams &p, const LayerPointers &lay
     // The 256-lane shape is also that of the small launches, which cost what it takes to issue them: few layers leave
     // 1.5 KB of their arguments out.
     const bool few = p.num_layers <= kFewLayers;
-    if (p.chunk_shift < 0 && few) ARCTIC_BULK_LAUNCH(false, 256, 4, kFewLayers);
+    if (p.chunk_shift < 0 && wide) ARCTIC_BULK_LAUNCH(false, 1024, 1, kLayersPerLaunch);
+    else if (p.chunk_shift < 0 && few) ARCTIC_BULK_LAUNCH(false, 256, 4, kFewLayers);
     else if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch);
     else if (wide) ARCTIC_BULK_LAUNCH(true, 1024, 1, kLayersPerLaunch);   // 0.5-2 % faster than the same batch as 512 x 2
     else if (few) ARCTIC_BULK_LAUNCH(true, 256, 4, kFewLayers);
@@ -721,33 +723,51 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       if (vec && (p.chunks_per_row & (p.chunks_per_row - 1)) == 0) p.chunk_shift = __builtin_ctz(p.chunks_per_row);
 
       // A token's layers are split over `groups` workgroups.  Measured best on gfx950 (sweeps over the group count and
-      // both shapes at 64 to 16384 tokens, 16 and 40 layers):
-      //  - above 8192 tokens, the wide shape (batches of 1024 chunks by 1024 lanes, by 512 lanes when rows are
-      //    selected as well) with up to five batches per workgroup (20 layers of 8 x 128 bf16) and at least about
-      //    1024 workgroups; a workgroup that would get less than two batches takes the 256-lane shape instead;
-      //  - below that, the 256-lane shape with about two batches of 1024 chunks per workgroup (8 such layers), more
-      //    and smaller workgroups when fewer than about 2048 would exist otherwise, but never less than one batch each.
+      // the shapes at 5 to 16384 tokens, 16, 33 and 40 layers, rows of 240 to 1024 elements):
+      //  - as long as a batch (1024 chunks) per workgroup makes no more than about 2048 workgroups of 256 lanes, the eight
+      //    per CU that run side by side, a workgroup has one batch, the layers that fit it whole: a second one, mostly a
+      //    few chunks, costs a memory round trip and is what the last workgroups do (us in a graph, layers spread to at
+      //    least one batch each / to at most one: 100 x 33 of 3 x 80 6.12 / 4.71, 500 x 33 of 3 x 96 9.7 / 9.1, 1000 x
+      //    33 of 3 x 80 15.3 / 13.3);
+      //  - fewer than about 512 such workgroups leave CUs idle or with a wave or two per SIMD, whose instructions count
+      //    then: more and smaller ones, a chunk per lane at the least (5 x 16 of 8 x 128 3.61 / 3.19, 5 x 40 of 3 x 96
+      //    4.59 / 3.70, 30 x 16 of 8 x 128 3.80 / 3.49; from 800 workgroups on it is level, behind 2048 each one more
+      //    costs: 512 x 40 of 3 x 96 in 4 groups 9.95, in 5 11.7);
+      //  - more tokens, up to 8192: about two batches (8 layers of 8 x 128) per workgroup, never less than one each;
+      //  - above that, the wide shape (batches of 1024 chunks by 1024 lanes, by 512 lanes when rows are selected as well)
+      //    with up to five batches per workgroup (20 layers of 8 x 128 bf16) and at least about 1024 workgroups; a
+      //    workgroup that would get less than two batches takes the 256-lane shape instead.
+      // Rows that are no power of two long take the wide shape from 4097 tokens on where its batches come out filled: a
+      // lane's loads of a batch that is not full are idle slots of 1024-lane workgroups, of which only two run per CU (us,
+      // 256 lanes / 1024: 5003 x 33 of 3 x 96 72.1 / 69.0, three batches 77 % full; 16384 x 40 of it 305 / 285, 94 %; 8000
+      // x 33 of 3 x 80 117 / 111, 97 %; a single batch at 94 % 55.2 / 53.8, at 77 % 72 / 81; two batches at 56 % 56.6 / 59.4).
       int groups = 1;
       bool wide = false;
       if (vec) {
+        constexpr int64_t kBatch = 1024, kSideBySide = 2048, kFewWorkgroups = 512, kFewestChunks = 256;
         const int64_t chunks_per_layer = 2LL * p.chunks_per_row;
-        const int min_layers = (int)std::max<int64_t>(1, (1024 + chunks_per_layer - 1) / chunks_per_layer);
-        if (num_tokens > 8192) {
-          int64_t g = std::max<int64_t>((1024 + num_tokens - 1) / num_tokens, (chunks_per_layer * count + 5119) / 5120);
-          g = std::max<int64_t>(1, std::min<int64_t>(g, count));
-          const int64_t layers_per_group = (count + g - 1) / g;
-          if (layers_per_group * chunks_per_layer >= 2048) {
-            wide = true;
-            groups = (int)g;
-          } else {
-            const int64_t want = (2048 + num_tokens - 1) / num_tokens;
-            groups = (int)std::max<int64_t>(1, std::min<int64_t>(want, count / min_layers));
-          }
+        const auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+        const auto limit = [&](int64_t g) { return std::max<int64_t>(1, std::min<int64_t>(g, count)); };
+        const int64_t min_layers = std::max<int64_t>(1, ceil_div(kBatch, chunks_per_layer));
+        const bool ragged = p.chunk_shift < 0;
+        const int64_t one_batch_groups = ceil_div(count, std::max<int64_t>(1, kBatch / chunks_per_layer));
+        if (num_tokens > 8192 || (ragged && !select && num_tokens > 4096)) {
+          const int64_t g = limit(std::max(ceil_div(1024, num_tokens), ceil_div(chunks_per_layer * count, 5 * kBatch)));
+          const int64_t chunks = ceil_div(count, g) * chunks_per_layer, slots = ceil_div(chunks, kBatch) * kBatch;
+          wide = ragged && !select ? chunks * 8 >= slots * (slots == kBatch ? 7 : 6) : chunks >= 2 * kBatch;
+          if (wide) groups = (int)g;
+        }
+        if (wide) {
+          // as above
+        } else if (num_tokens > 8192) {
+          groups = (int)limit(std::min(ceil_div(kSideBySide, num_tokens), count / min_layers));
+        } else if (num_tokens * one_batch_groups <= kSideBySide) {
+          const int64_t fewest_layers = std::max<int64_t>(1, ceil_div(kFewestChunks, chunks_per_layer));
+          groups = (int)limit(std::max(one_batch_groups, std::min(kFewWorkgroups / num_tokens, ceil_div(count, fewest_layers))));
         } else {
-          const int64_t two_batches = std::max<int64_t>(1, (2048 + chunks_per_layer - 1) / chunks_per_layer);   // layers
-          const int64_t want =
-              std::max<int64_t>((count + two_batches - 1) / two_batches, (2048 + num_tokens - 1) / num_tokens);
-          groups = (int)std::max<int64_t>(1, std::min<int64_t>(want, count / min_layers));
+          const int64_t want = std::max(ceil_div(count, std::max<int64_t>(1, ceil_div(2 * kBatch, chunks_per_layer))),
+                                        ceil_div(kSideBySide, num_tokens));
+          groups = (int)limit(std::min(want, count / min_layers));
         }
       } else {
         groups = (int)std::max<int64_t>(1, std::min<int64_t>(count, (2048 + num_tokens - 1) / num_tokens));

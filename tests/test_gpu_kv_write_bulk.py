@@ -82,6 +82,18 @@ def test_layers_at_the_edges_of_the_pointer_tables(ops, L, heads_of, kv):
     run_both(ops, make_bulk_case(T=6, L=L, bs=16, NB=2, kv_cache_dtype=kv, seed=23, std=1.5, pad_fraction=0.2, **heads_of))
 
 
+@pytest.mark.parametrize("shape", [
+    dict(T=1, L=40, H=3, D=96), dict(T=31, L=40, H=1, D=128),      # a chunk per lane, groups with a ragged tail
+    dict(T=682, L=40, H=3, D=96), dict(T=683, L=40, H=3, D=96),    # 2046 workgroups of one batch; two batches each
+    dict(T=1024, L=17, H=3, D=80), dict(T=1025, L=18, H=3, D=80),  # one batch per token; nothing smaller than a batch
+    dict(T=4096, L=16, H=3, D=80), dict(T=4097, L=16, H=3, D=80),  # 256 lanes; 1024 lanes, a batch 94 % full
+    dict(T=4097, L=14, H=3, D=80), dict(T=4097, L=27, H=3, D=80),  # 82 % full: 256 lanes; two batches, 79 %: 1024
+])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+def test_layers_split_over_workgroups(ops, kv, shape):
+    run_both(ops, make_bulk_case(bs=16, NB=shape["T"] // 16 + 2, kv_cache_dtype=kv, seed=29, std=1.5, pad_fraction=0.05, **shape))
+
+
 def test_all_padding_leaves_cache_untouched(ops):
     case = make_bulk_case(T=16, L=3, H=2, D=64, bs=16, NB=4, kv_cache_dtype="fp8", seed=7)
     case["slot_mapping"].fill_(-1)
