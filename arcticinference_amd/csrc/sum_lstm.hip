@@ -3,7 +3,7 @@
 // Replaces sum_lstm_cuda and its kernels
 // (csrc/custom_ops/sum_lstm.cu:14-473 in the reference).
 //
-// One workgroup per row.  On the vector paths each lane owns 16-byte chunks
+// One workgroup per row (few long rows: several, which share its last phase).  On the vector paths each lane owns 16-byte chunks
 // (8 elements) at the same column of all four gates of `states` and `z4` and of
 // `prev_cell`: nine 16-byte loads per chunk.  The row then stays in registers
 // across both RMS reductions, so HBM sees 9*D elements read and 2*D written per
@@ -56,6 +56,12 @@ struct LstmSharedParams : LstmParams<Size> {
 template <bool kSharedZ>
 using LstmParamsOf = std::conditional_t<kSharedZ, LstmSharedParams<uint32_t>, LstmParams<uint32_t>>;
 using LstmCall = LstmSharedParams<int64_t>;   // what an entry point was given
+template <bool kSharedZ>
+struct LstmPartsParams : LstmParamsOf<kSharedZ> {
+  int rows;   // the grid's first dimension is rounded up
+};
+template <bool kSharedZ, bool kParts>
+using LstmStagedParams = std::conditional_t<kParts, LstmPartsParams<kSharedZ>, LstmParamsOf<kSharedZ>>;
 
 // The row of z4 that a row adds.
 template <bool kSharedZ, typename Params>
@@ -259,16 +265,26 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
 // leave earlier).
 //
 // kZeroCell: the previous cell is all zeros (the first step of a proposal round) and is not read.
-template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, RowKind kKind>
-__global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParamsOf<kSharedZ> p) {
+// kParts: few rows leave most CUs idle while a row's waves share the four SIMDs of one, and there the instructions count
+// (about 590 a wave: one row of 2048 / 4096 / 8192 elements takes 3.1 / 4.1 / 6.3 us).  The new cell's norm needs the whole
+// row, so each of a row's workgroups (blockIdx.y) does the cell update of all of it; the state behind that norm, two fifths
+// of the arithmetic, and the stores it does for four waves' chunks alone, one wave per SIMD.  The workgroups of a row read
+// the same bytes, so they belong on one XCD: the hardware deals workgroups round robin over the eight, and blockIdx.x counts
+// to a multiple of eight.
+template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, RowKind kKind, bool kParts>
+__global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedParams<kSharedZ, kParts> p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
   constexpr int E = Chunk::kElems;
   using C = Chunk;
   using std::integral_constant;
   const int64_t row = blockIdx.x;
+  if constexpr (kParts)
+    if ((int)blockIdx.x >= p.rows) return;   // all of the workgroup
   constexpr bool kAny = kKind == kAnyRow;
   const int waves = ((p.D + 7) / 8 + 63) / 64;   // of the workgroup, as launched
+  // whether this wave's chunks are this workgroup's to store
+  const bool mine = !kParts || __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) == (int)blockIdx.y;
   // the barriers need every wave, so the lanes behind the last chunk run along on it
   const Place at(threadIdx.x, kKind == kFullWaves ? INT32_MAX : p.D);
   const uint32_t off = at.off;
@@ -319,7 +335,11 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParamsO
 #pragma unroll
     for (int j = 0; j < E; ++j) cact[j] = gelu<kFastGelu>(fmaf(cact[j] * inv_cpre, w[j], sh[j]));
   }
-  const C ws = load_scale<T, kAny>(p.w_state, off), bs = load_shift<kAny>(p.b_state, off);
+  C ws = C::zero(), bs = C::zero();
+  if (mine) {
+    ws = load_scale<T, kAny>(p.w_state, off);
+    bs = load_shift<kAny>(p.b_state, off);
+  }
   request(integral_constant<int, 3>(), integral_constant<int, 7>());
   __builtin_amdgcn_s_barrier();   // waits for no memory: only keeps the row's waves in step at their largest group of requests
   __builtin_amdgcn_sched_barrier(0);
@@ -343,11 +363,12 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmParamsO
   }
   {
     const C packed = C::template pack<T>(cell);
-    if (kKind == kFullWaves || at.live()) packed.template store_stream<kAny>(oc_row + off);
+    if (mine && (kKind == kFullWaves || at.live())) packed.template store_stream<kAny>(oc_row + off);
     packed.template unpack<T>(cell);   // the state phase sees the rounded cell (:163,174)
   }
-  request(integral_constant<int, 7>(), integral_constant<int, 9>());
+  if (mine) request(integral_constant<int, 7>(), integral_constant<int, 9>());
   const float inv_cnew = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cnew, waves) * p.inv_D + p.eps_state);
+  if (!mine) return;   // behind the last barrier
 
   // phase 3: state = gelu(rmsnorm(rounded cell)) * sigmoid(pre_o) (reference :160-190)
   float st[E];
@@ -447,7 +468,7 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
                        aligned16(p.b_cell) && aligned16(p.w_state) && aligned16(p.b_state);
   const int chunks = (p.D + 7) / 8;
   const int lanes = (chunks + 63) & ~63;
-  const dim3 grid((unsigned)rows);
+  dim3 grid((unsigned)rows);
   // One chunk per lane up to 1024 lanes (512 rows of 5120 / 6144 / 8192 elements: 12.0 / 13.9 / 17.5 us against 17.6 /
   // 19.9 / 22.5 us with two chunks per lane in the other kernel; without scale and shift 512 rows of 4096 / 8192: 9.6 /
   // 17.3 us against 11.0 / 24.1 us).  Rows that are not 16-byte aligned take the same kernels with accesses at any
@@ -458,12 +479,14 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   // 3.30, 512 x 128 3.01 / 3.87, 64 x 256 2.77 / 3.27, 4096 x 256 8.7 / 9.5; with all of them 512 x 128 3.31 / 3.88, 64 x
   // 256 3.07 / 3.24); with all vectors and more than 256 rows it is chunks from 129 on (300 x 136 level, 512 x 160 7 % and
   // 2048 x 256 8 % faster).  From 257 on chunks are faster at every row count (64 x 257 by 10 to 23 %, 64 x 513 by 21 to 35).
-#define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND) \
-  launch(sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND>, grid, lanes, s, compact)
-#define ARCTIC_LSTM_STAGED(KIND)                                    \
-  do {                                                              \
-    if (p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND);        \
-    else ARCTIC_LSTM_STAGED_LAUNCH(true, KIND);                     \
+#define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, PARTS, PARAMS) \
+  launch(sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND, PARTS>, grid, lanes, s, PARAMS)
+#define ARCTIC_LSTM_STAGED(KIND)                                                         \
+  do {                                                                                   \
+    if (in_parts && p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND, true, of_parts); \
+    else if (in_parts) ARCTIC_LSTM_STAGED_LAUNCH(true, KIND, true, of_parts);            \
+    else if (p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND, false, compact);        \
+    else ARCTIC_LSTM_STAGED_LAUNCH(true, KIND, false, compact);                          \
   } while (0)
   const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
   const bool narrow = !aligned && p.D <= (all_vectors && rows > 256 ? 128 : 256);
@@ -503,6 +526,20 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   } else if (aliased && aligned) {
     ARCTIC_LSTM_VEC(2, false);
   } else if (chunks <= 1024) {
+    // Few rows of more than 2048 elements: a workgroup per four waves of a row, as long as every workgroup has a CU of its
+    // own.  Us per call in a graph, one workgroup per row / in parts: 7 x 4096 4.14 / 3.87, 3 x 8192 6.30 / 5.50, 45 x 5120
+    // 6.16 / 5.40, 64 x 8192 7.71 / 7.11, 128 x 4096 5.41 / 5.18; with two workgroups on a CU 85 x 5120 6.39 / 8.01, and
+    // with a last part of less than four waves it is level from 200 workgroups on (128 x 2880 5.16 / 5.23).  A call that
+    // updates a tensor in place would read in one workgroup what another one has written.
+    const int parts = (lanes + 255) / 256;
+    const int64_t rows_up = (rows + 7) & ~(int64_t)7;
+    const bool in_parts = parts > 1 && rows_up * parts <= (lanes % 256 ? 224 : 256) && !in_place(p, rows, kSharedZ);
+    LstmPartsParams<kSharedZ> of_parts;
+    if (in_parts) {
+      static_cast<LstmParamsOf<kSharedZ> &>(of_parts) = compact;
+      of_parts.rows = (int)rows;
+      grid = dim3((unsigned)rows_up, (unsigned)parts);
+    }
     if (!aligned || !all_vectors) ARCTIC_LSTM_STAGED(kAnyRow);
     else if (lanes != chunks) ARCTIC_LSTM_STAGED(kRagged);
     else ARCTIC_LSTM_STAGED(kFullWaves);

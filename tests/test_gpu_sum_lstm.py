@@ -374,7 +374,7 @@ def test_absent_vectors_equal_ones_and_zeros(ops, D, rows, dtype):
 @pytest.mark.parametrize("D,rows,vectors,into", [
     (513, 300, True, "cell"), (1537, 300, False, "cell"), (8193, 40, True, "cell"), (300, 20, False, "cell"),   # widths of no multiple of 8
     (1024, 600, False, "output gate"), (4096, 64, False, "output gate"), (8192, 3, False, "output gate"),        # no vectors
-    (4096, 64, True, "cell")])
+    (4096, 64, True, "cell"), (4104, 3, True, "cell")])
 def test_updates_in_place(ops, D, rows, vectors, into):
     """Through the C entry point the new cell may be stored over the previous one, and, without vectors, over the output
     gate: the results are the oracle's."""
@@ -393,3 +393,27 @@ def test_updates_in_place(ops, D, rows, vectors, into):
         torch.cuda.current_stream().cuda_stream))
     assert_close(cell, want_c, RTOL, ATOL, "cell")
     assert_close(state, want_s, RTOL, ATOL, "state")
+
+
+@pytest.mark.parametrize("D,pad4,padD,vectors", [(2049, 3, 3, True), (2056, 0, 0, True), (2880, 0, 0, False), (4096, 0, 0, True),
+                                                 (4104, 8, 0, True), (5120, 0, 8, True), (6145, 0, 0, False), (8185, 1, 0, True),
+                                                 (8192, 0, 0, True)])
+@pytest.mark.parametrize("rows", [1, 8, 9, 63, 64, 65, 112, 113, 128, 129])
+def test_few_rows_shared_by_several_workgroups(ops, D, pad4, padD, vectors, rows):
+    """Up to where a workgroup per row takes over: the bits of the same rows among 300, which a workgroup each computes; with
+    and without a previous cell, z given and looked up."""
+    dtype = torch.bfloat16 if D % 16 else torch.float16
+    c = make_lstm_case(rows=300, D=D, dtype=dtype, seed=D, pad4=pad4, padD=padD, wb_cell=vectors, wb_state=vectors)
+    d = {k: dev(v) for k, v in c.items()}
+    vec = [d[k] for k in ("w_cell", "b_cell", "w_state", "b_state")]
+    ids = torch.randint(0, 300, (300,), generator=torch.Generator().manual_seed(rows)).to(DEV)
+    table = d["z4"][:, :D].contiguous()
+    for prev in (d["prev_cell"], None):
+        head = None if prev is None else prev[:rows]
+        for got, want in ((ops.sum_lstm(d["states"][:rows], d["z4"][:rows], head, *vec, 0.35, 1e-6, 1e-6, False),
+                           ops.sum_lstm(d["states"], d["z4"], prev, *vec, 0.35, 1e-6, 1e-6, False)),
+                          (ops.sum_lstm_embedded(d["states"][:rows], table, ids[:rows], head, *vec, 0.35, 1e-6, 1e-6, True),
+                           ops.sum_lstm_embedded(d["states"], table, ids, prev, *vec, 0.35, 1e-6, 1e-6, True))):
+            for few, many in zip(got, want):
+                assert torch.equal(few, many[:rows])
+    run(ops, {k: v[:2] if v is not None and v.dim() == 2 else v for k, v in c.items()}, 0.35)
