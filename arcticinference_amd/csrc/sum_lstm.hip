@@ -97,7 +97,7 @@ __device__ __forceinline__ Chunk load_shift(const char *b, uint32_t off) {
   return Chunk::load<true>((b ? b : (const char *)kChunkOfZeros) + (b ? off : 0u));
 }
 
-// Rows beyond one chunk per lane of 1024 lanes, with two of them, and aligned rows of up to 2048 elements that lack a
+// Rows beyond one chunk per lane of 1024 lanes, with two of them, and rows of up to 2048 elements that lack a
 // scale or shift vector, with one (launch_lstm has the rule).  Loads are issued in the order in which the arithmetic needs them -
 // cell gate, forget gate, previous cell, input gate, output gate - and memory returns them in that order, so the first
 // row sum, the candidate GELU and the early sigmoids run while the later gates are still on their way, and only one
@@ -506,23 +506,29 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
       (uint32_t)p.z_stride, (uint32_t)p.pc_stride, (uint32_t)p.out_stride, (uint32_t)p.z_rows, p.D, p.inv_D, p.alpha,
       p.eps_cell, p.eps_state};
   if constexpr (kSharedZ) compact.z_index = p.z_index;
-  // Aligned rows of up to 2048 elements that lack a vector: at most four waves per row, whose loads are few enough to be
-  // requested together.  Us per call in a graph, in stages (ones and zeros read in place of an absent vector) / together:
+  // Rows of up to 2048 elements that lack a vector: at most four waves per row, whose loads are few enough to be
+  // requested together.  Aligned ones, us per call in a graph, in stages (ones and zeros read in place of an absent vector) / together:
   // 64 x 256 without vectors 4.0 / 3.2, 512 x 512 4.2 / 3.3, 300 x 2048 5.6 / 4.8, 512 x 512 with the scales alone 4.1 / 3.4;
   // from 513 elements and 513 rows on the stages are faster (2048 x 1024 8.8 / 9.4), but for one z for all gates (8.4 / 7.7).
-  const bool together = aligned && !all_vectors && chunks <= 256 && (chunks <= 64 || rows <= 512 || kSharedZ);
+  // Rows at any alignment do it without any vector, or with one wave per row: 300 x 1537 without 5.89 / 5.34, 64 x 513 3.57 /
+  // 3.26, 1500 x 257 5.58 / 4.88, with one z for all gates 1500 x 1537 11.1 / 10.0; with the scales alone 300 x 300 3.41 /
+  // 3.33, but 300 x 769 4.62 / 4.84 (without any vector 4.70 / 4.59, and without a previous cell either 4.54 / 4.63).
+  const bool no_vector = !p.w_cell && !p.b_cell && !p.w_state && !p.b_state;
+  const bool together = !all_vectors && chunks <= 256 && (chunks <= 64 || ((aligned || no_vector) && (rows <= 512 || kSharedZ)));
 #define ARCTIC_LSTM_VEC_LAUNCH(K, ANY, BARE) \
   launch(sum_lstm_vec_kernel<T, K, kFastGelu, kSharedZ, ANY, BARE>, grid, threads, s, compact)
 #define ARCTIC_LSTM_VEC(K, ANY)                                       \
   do {                                                                \
     const int threads = ((chunks + (K) - 1) / (K) + 63) & ~63;        \
-    if (p.w_cell || p.b_cell || p.w_state || p.b_state) ARCTIC_LSTM_VEC_LAUNCH(K, ANY, false); \
-    else ARCTIC_LSTM_VEC_LAUNCH(K, ANY, true);                        \
+    if (no_vector) ARCTIC_LSTM_VEC_LAUNCH(K, ANY, true);              \
+    else ARCTIC_LSTM_VEC_LAUNCH(K, ANY, false);                       \
   } while (0)
   if (element_wise) {
     launch(sum_lstm_scalar_kernel<T, kFastGelu>, grid, kScalarLanes, s, LstmScalarParams{p, kSharedZ ? 0 : p.D});
-  } else if (together) {
+  } else if (together && aligned) {
     ARCTIC_LSTM_VEC(1, false);
+  } else if (together) {
+    ARCTIC_LSTM_VEC(1, true);
   } else if (aliased && aligned) {
     ARCTIC_LSTM_VEC(2, false);
   } else if (chunks <= 1024) {

@@ -350,7 +350,8 @@ def test_rows_that_are_not_16_byte_aligned(ops, D, pad4, padD, rows):
 
 
 @pytest.mark.parametrize("D,rows", [(8, 513), (504, 1), (512, 600), (520, 512), (520, 513), (2040, 3), (2048, 512), (2048, 513),
-                                    (2056, 2), (8192, 2), (8200, 3), (16384, 2), (16383, 2)])
+                                    (2056, 2), (8192, 2), (8200, 3), (16384, 2), (16383, 2), (257, 600), (511, 513), (513, 512),
+                                    (513, 513), (2047, 512), (2047, 513), (2049, 2)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_absent_vectors_equal_ones_and_zeros(ops, D, rows, dtype):
     """None of the four vectors, or the shifts alone missing: bit for bit what ones and zeros in their place give, on both
