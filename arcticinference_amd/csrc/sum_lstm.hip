@@ -10,7 +10,7 @@
 // row (the reference re-reads the cell gate and reads out_cell back: 12*D).
 // Sums are DPP wave reductions plus an LDS combine.  Three kernels:
 // sum_lstm_staged_kernel (rows of up to 8192 elements: the nine loads are
-// requested in stages, between the stages of the arithmetic, one chunk per lane),
+// requested in stages, between the stages of the arithmetic, or, for few short rows, ahead of it; one chunk per lane),
 // sum_lstm_vec_kernel (the loads requested together: rows of up to 16384 elements
 // with two chunks per lane, and short ones without all vectors) and sum_lstm_scalar_kernel (what is left: short rows
 // that are not 16-byte aligned and more than 16384 elements, element by element).
@@ -69,6 +69,14 @@ __device__ __forceinline__ int64_t z_row_of(const Params &p, int64_t row) {
   if constexpr (kSharedZ)
     if (p.z_index) return min(max(p.z_index[row], (int64_t)0), (int64_t)p.z_rows - 1);
   return row;
+}
+
+// The index of that row as it was given, by a load that nothing waits for yet (without indices of the arguments themselves).
+template <typename Params>
+__device__ __forceinline__ int64_t z_id_of(const Params &p, int64_t row) {
+  typedef const __attribute__((address_space(4))) int64_t *Constant;
+  const uintptr_t none = (uintptr_t)(const void *)__builtin_amdgcn_kernarg_segment_ptr();
+  return *(Constant)(p.z_index ? (uintptr_t)(p.z_index + row) : none);
 }
 
 // kFullWaves: rows 16-byte aligned, all four scale / shift vectors given, every lane of every wave owns a chunk of 8
@@ -265,22 +273,27 @@ __global__ __launch_bounds__(K == 1 ? 256 : 1024) void sum_lstm_vec_kernel(const
 // leave earlier).
 //
 // kZeroCell: the previous cell is all zeros (the first step of a proposal round) and is not read.
+// kAhead: few rows of few waves, where nothing else fills the CU while a stage waits for its round trip: all of the row is
+// requested at the start, in the same order (launch_lstm has the rule).  With one z for all gates the chunks of `states`
+// go first, so that they are on their way while the index of the embedding arrives.
 // kParts: few rows leave most CUs idle while a row's waves share the four SIMDs of one, and there the instructions count
 // (about 590 a wave: one row of 2048 / 4096 / 8192 elements takes 3.1 / 4.1 / 6.3 us).  The new cell's norm needs the whole
 // row, so each of a row's workgroups (blockIdx.y) does the cell update of all of it; the state behind that norm, two fifths
 // of the arithmetic, and the stores it does for four waves' chunks alone, one wave per SIMD.  The workgroups of a row read
 // the same bytes, so they belong on one XCD: the hardware deals workgroups round robin over the eight, and blockIdx.x counts
 // to a multiple of eight.
-template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, RowKind kKind, bool kParts>
+template <typename T, bool kFastGelu, bool kSharedZ, bool kZeroCell, RowKind kKind, bool kParts, bool kAhead>
 __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedParams<kSharedZ, kParts> p) {
   __shared__ float slots_cpre[16];
   __shared__ float slots_cnew[16];
   constexpr int E = Chunk::kElems;
   using C = Chunk;
   using std::integral_constant;
-  const int64_t row = blockIdx.x;
-  if constexpr (kParts)
-    if ((int)blockIdx.x >= p.rows) return;   // all of the workgroup
+  int64_t row = blockIdx.x, z_id = 0;
+  if constexpr (kParts) row = min((int)blockIdx.x, p.rows - 1);
+  if constexpr (kAhead && kSharedZ) z_id = z_id_of(p, row);
+  if constexpr (kParts)   // all of the workgroup
+    if ((int)blockIdx.x >= p.rows) return;
   constexpr bool kAny = kKind == kAnyRow;
   const int waves = ((p.D + 7) / 8 + 63) / 64;   // of the workgroup, as launched
   // whether this wave's chunks are this workgroup's to store
@@ -291,7 +304,8 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedP
   auto load = [off](const char *q) { return C::load_stream<kAny>(q + off); };
   const int64_t gate_bytes = (int64_t)p.D * 2;
   const char *s_row = p.states + row * p.s_stride * 2;
-  const char *z_row = p.z4 + z_row_of<kSharedZ>(p, row) * p.z_stride * 2;
+  const char *z_row = nullptr;
+  if constexpr (!(kAhead && kSharedZ)) z_row = p.z4 + z_row_of<kSharedZ>(p, row) * p.z_stride * 2;
   const char *pc_row = kZeroCell ? s_row : p.prev_cell + row * p.pc_stride * 2;
   char *oc_row = p.out_cell + row * p.out_stride * 2;
   char *os_row = p.out_state + row * p.out_stride * 2;
@@ -312,9 +326,29 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedP
     if constexpr (kFrom <= 8 && 8 < kTo && !kSharedZ) in[8] = load(z_row + 2 * gate_bytes);
     __builtin_amdgcn_sched_barrier(0);
   };
-  request(integral_constant<int, 0>(), integral_constant<int, 2>());
+  C ws = C::zero(), bs = C::zero();
+  auto request_state_vectors = [&] {
+    if (mine) {
+      ws = load_scale<T, kAny>(p.w_state, off);
+      bs = load_shift<kAny>(p.b_state, off);
+    }
+  };
+  if constexpr (kAhead && kSharedZ) {
+    request(integral_constant<int, 1>(), integral_constant<int, 3>());
+    asm volatile("" : "+s"(z_id));   // the wait for the index is here
+    z_row = p.z4 + (p.z_index ? min(max(z_id, (int64_t)0), (int64_t)p.z_rows - 1) : row) * p.z_stride * 2;
+    request(integral_constant<int, 0>(), integral_constant<int, 1>());
+  } else {
+    request(integral_constant<int, 0>(), integral_constant<int, 2>());
+  }
   const C wc = load_scale<T, kAny>(p.w_cell, off), bc = load_shift<kAny>(p.b_cell, off);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (kAhead) {
+    request(integral_constant<int, kSharedZ ? 3 : 2>(), integral_constant<int, 7>());
+    request_state_vectors();
+    if (mine) request(integral_constant<int, 7>(), integral_constant<int, 9>());
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // phase 1: pre_c and its sum of squares (reference :65-82)
   float cact[E], a[E], b[E], c[E];
@@ -326,7 +360,7 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedP
     cact[j] = fmaf(p.alpha, b[j], a[j]);
     if (!kAny || j >= at.repeated) ss = fmaf(cact[j], cact[j], ss);
   }
-  request(integral_constant<int, 2>(), integral_constant<int, 3>());
+  if constexpr (!kAhead) request(integral_constant<int, 2>(), integral_constant<int, 3>());
   const float inv_cpre = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cpre, waves) * p.inv_D + p.eps_cell);
   {
     float w[E], sh[E];
@@ -335,13 +369,11 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedP
 #pragma unroll
     for (int j = 0; j < E; ++j) cact[j] = gelu<kFastGelu>(fmaf(cact[j] * inv_cpre, w[j], sh[j]));
   }
-  C ws = C::zero(), bs = C::zero();
-  if (mine) {
-    ws = load_scale<T, kAny>(p.w_state, off);
-    bs = load_shift<kAny>(p.b_state, off);
+  if constexpr (!kAhead) {
+    request_state_vectors();
+    request(integral_constant<int, 3>(), integral_constant<int, 7>());
+    __builtin_amdgcn_s_barrier();   // waits for no memory: only keeps the row's waves in step at their largest group of requests
   }
-  request(integral_constant<int, 3>(), integral_constant<int, 7>());
-  __builtin_amdgcn_s_barrier();   // waits for no memory: only keeps the row's waves in step at their largest group of requests
   __builtin_amdgcn_sched_barrier(0);
 
   // phase 2: cell update; write out_cell (reference :104-140)
@@ -366,7 +398,8 @@ __global__ __launch_bounds__(1024) void sum_lstm_staged_kernel(const LstmStagedP
     if (mine && (kKind == kFullWaves || at.live())) packed.template store_stream<kAny>(oc_row + off);
     packed.template unpack<T>(cell);   // the state phase sees the rounded cell (:163,174)
   }
-  if (mine) request(integral_constant<int, 7>(), integral_constant<int, 9>());
+  if constexpr (!kAhead)
+    if (mine) request(integral_constant<int, 7>(), integral_constant<int, 9>());
   const float inv_cnew = rsqrtf(block_sum(kKind != kRagged || at.live() ? ss : 0.f, slots_cnew, waves) * p.inv_D + p.eps_state);
   if (!mine) return;   // behind the last barrier
 
@@ -479,14 +512,19 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   // 3.30, 512 x 128 3.01 / 3.87, 64 x 256 2.77 / 3.27, 4096 x 256 8.7 / 9.5; with all of them 512 x 128 3.31 / 3.88, 64 x
   // 256 3.07 / 3.24); with all vectors and more than 256 rows it is chunks from 129 on (300 x 136 level, 512 x 160 7 % and
   // 2048 x 256 8 % faster).  From 257 on chunks are faster at every row count (64 x 257 by 10 to 23 %, 64 x 513 by 21 to 35).
-#define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, PARTS, PARAMS) \
-  launch(sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND, PARTS>, grid, lanes, s, PARAMS)
-#define ARCTIC_LSTM_STAGED(KIND)                                                         \
-  do {                                                                                   \
-    if (in_parts && p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND, true, of_parts); \
-    else if (in_parts) ARCTIC_LSTM_STAGED_LAUNCH(true, KIND, true, of_parts);            \
-    else if (p.prev_cell) ARCTIC_LSTM_STAGED_LAUNCH(false, KIND, false, compact);        \
-    else ARCTIC_LSTM_STAGED_LAUNCH(true, KIND, false, compact);                          \
+#define ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, PARTS, AHEAD, PARAMS) \
+  launch(sum_lstm_staged_kernel<T, kFastGelu, kSharedZ, ZERO, KIND, PARTS, AHEAD>, grid, lanes, s, PARAMS)
+#define ARCTIC_LSTM_STAGED_AS(ZERO, KIND)                                                                     \
+  do {                                                                                                        \
+    if (in_parts && kSharedZ && parts_ahead) ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, true, kSharedZ, of_parts); \
+    else if (in_parts) ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, true, false, of_parts);                          \
+    else if (ahead) ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, false, true, compact);                              \
+    else ARCTIC_LSTM_STAGED_LAUNCH(ZERO, KIND, false, false, compact);                                        \
+  } while (0)
+#define ARCTIC_LSTM_STAGED(KIND)                          \
+  do {                                                    \
+    if (p.prev_cell) ARCTIC_LSTM_STAGED_AS(false, KIND);  \
+    else ARCTIC_LSTM_STAGED_AS(true, KIND);               \
   } while (0)
   const bool all_vectors = p.w_cell && p.b_cell && p.w_state && p.b_state;
   const bool narrow = !aligned && p.D <= (all_vectors && rows > 256 ? 128 : 256);
@@ -506,6 +544,13 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
       (uint32_t)p.z_stride, (uint32_t)p.pc_stride, (uint32_t)p.out_stride, (uint32_t)p.z_rows, p.D, p.inv_D, p.alpha,
       p.eps_cell, p.eps_state};
   if constexpr (kSharedZ) compact.z_index = p.z_index;
+  // At most four waves per row and few rows: everything is requested ahead, since a CU with a row or two of one to four waves
+  // takes the requests as they come, and a stage that waits for its round trip has nobody to leave the CU to.  Us per call in a
+  // graph, in stages / ahead: 7 x 1024 3.25 / 2.93, 64 x 2048 4.15 / 3.58, 256 x 1537 5.48 / 4.53, 512 x 512 4.14 / 3.48,
+  // 1000 x 512 4.57 / 4.29, 512 x 1500 6.29 / 6.00, embedded 256 x 2048 4.55 / 4.01; behind the lines below 2000 x 512 5.27 /
+  // 5.41, 700 x 1024 5.46 / 5.77, one z for all gates 400 x 2048 5.38 / 5.56, and with more waves per row 512 x 4096 9.09 / 9.99.
+  const int64_t ahead_rows = chunks <= 64 ? 1024 : chunks > 256 ? 0 : kSharedZ && aligned && chunks > 192 ? 256 : 512;
+  const bool ahead = rows <= ahead_rows;
   // Rows of up to 2048 elements that lack a vector: at most four waves per row, whose loads are few enough to be
   // requested together.  Aligned ones, us per call in a graph, in stages (ones and zeros read in place of an absent vector) / together:
   // 64 x 256 without vectors 4.0 / 3.2, 512 x 512 4.2 / 3.3, 300 x 2048 5.6 / 4.8, 512 x 512 with the scales alone 4.1 / 3.4;
@@ -513,8 +558,11 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   // Rows at any alignment do it without any vector, or with one wave per row: 300 x 1537 without 5.89 / 5.34, 64 x 513 3.57 /
   // 3.26, 1500 x 257 5.58 / 4.88, with one z for all gates 1500 x 1537 11.1 / 10.0; with the scales alone 300 x 300 3.41 /
   // 3.33, but 300 x 769 4.62 / 4.84 (without any vector 4.70 / 4.59, and without a previous cell either 4.54 / 4.63).
+  // Where rows are requested ahead (above) that is as good for the ones with some vectors: 64 x 1024 3.47 / 3.36, 256 x 512 3.49
+  // / 3.42; calls that update a tensor in place stay here.
   const bool no_vector = !p.w_cell && !p.b_cell && !p.w_state && !p.b_state;
-  const bool together = !all_vectors && chunks <= 256 && (chunks <= 64 || ((aligned || no_vector) && (rows <= 512 || kSharedZ)));
+  const bool together = !all_vectors && chunks <= 256 && (chunks <= 64 || ((aligned || no_vector) && (rows <= 512 || kSharedZ))) &&
+                        (no_vector || aliased || !ahead);
 #define ARCTIC_LSTM_VEC_LAUNCH(K, ANY, BARE) \
   launch(sum_lstm_vec_kernel<T, K, kFastGelu, kSharedZ, ANY, BARE>, grid, threads, s, compact)
 #define ARCTIC_LSTM_VEC(K, ANY)                                       \
@@ -540,6 +588,9 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
     const int parts = (lanes + 255) / 256;
     const int64_t rows_up = (rows + 7) & ~(int64_t)7;
     const bool in_parts = parts > 1 && rows_up * parts <= (lanes % 256 ? 224 : 256) && !in_place(p, rows, kSharedZ);
+    // One z for all gates leaves few enough requests to make them ahead (embedded, in stages / ahead: 7 x 2880 3.90 / 3.71, 64 x
+    // 2880 4.89 / 4.55, 7 x 4096 3.98 / 3.82; 32 x 4096 without a previous cell 4.39 / 4.44, 32 x 6144 5.38 / 5.67).
+    const bool parts_ahead = lanes <= 384 || (lanes <= 512 && rows <= 16);
     LstmPartsParams<kSharedZ> of_parts;
     if (in_parts) {
       static_cast<LstmParamsOf<kSharedZ> &>(of_parts) = compact;
@@ -557,6 +608,7 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
 #undef ARCTIC_LSTM_VEC
 #undef ARCTIC_LSTM_VEC_LAUNCH
 #undef ARCTIC_LSTM_STAGED
+#undef ARCTIC_LSTM_STAGED_AS
 #undef ARCTIC_LSTM_STAGED_LAUNCH
 }
 

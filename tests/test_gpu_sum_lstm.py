@@ -418,3 +418,31 @@ def test_few_rows_shared_by_several_workgroups(ops, D, pad4, padD, vectors, rows
             for few, many in zip(got, want):
                 assert torch.equal(few, many[:rows])
     run(ops, {k: v[:2] if v is not None and v.dim() == 2 else v for k, v in c.items()}, 0.35)
+
+
+@pytest.mark.parametrize("D,pad4,padD", [(264, 0, 0), (512, 0, 0), (513, 3, 3), (520, 8, 0), (1537, 0, 0), (1544, 0, 0), (2000, 0, 8), (2048, 0, 0)])
+@pytest.mark.parametrize("rows", [1, 256, 257, 512, 513, 1024, 1025])
+@pytest.mark.parametrize("shifts", [True, False])
+def test_few_rows_requested_ahead(ops, D, pad4, padD, rows, shifts):
+    """On both sides of the row counts up to which a row is requested at once: the bits of the same rows among 1100; z given,
+    shared and looked up, by indices outside the table too, which are clamped into it; with and without the shift vectors and
+    a previous cell; the first rows against the oracle."""
+    dtype = torch.bfloat16 if D % 16 else torch.float16
+    c = make_lstm_case(rows=1100, D=D, dtype=dtype, seed=D, pad4=pad4, padD=padD)
+    if not shifts:
+        c["b_cell"] = c["b_state"] = None
+    d = {k: None if v is None else dev(v) for k, v in c.items()}
+    tail = [d[k] for k in ("w_cell", "b_cell", "w_state", "b_state")] + [0.35, 1e-6, 1e-6, False]
+    table = d["z4"][:, :D].contiguous()
+    ids = torch.randint(-40, 1140, (1100,), generator=torch.Generator().manual_seed(rows)).to(DEV)
+    for prev in (d["prev_cell"], None):
+        def results(n):
+            head, s = None if prev is None else prev[:n], d["states"][:n]
+            return (*ops.sum_lstm(s, d["z4"][:n], head, *tail), *ops.sum_lstm_shared_z(s, table[:n], head, *tail),
+                    *ops.sum_lstm_embedded(s, table, ids[:n], head, *tail),
+                    *ops.sum_lstm_shared_z(s, table[ids[:n].clamp(0, 1099)], head, *tail))
+        few, many = results(rows), results(1100)
+        for a, b in zip(few, many):
+            assert torch.equal(a, b[:rows])
+        assert torch.equal(few[4], few[6]) and torch.equal(few[5], few[7])
+    run(ops, {k: v[:3] if v is not None and v.dim() == 2 else v for k, v in c.items()}, 0.35)
