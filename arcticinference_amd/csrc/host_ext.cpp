@@ -58,8 +58,15 @@ struct From<double> {
 template <>
 struct From<int64_t> {
   static int64_t get(PyObject *o) {
-    const long long v = PyFloat_Check(o) ? -1 : PyLong_AsLongLong(o);
-    if (v == -1 && (PyFloat_Check(o) || PyErr_Occurred())) throw Refused{"an int"};
+    if (PyFloat_Check(o)) throw Refused{"an int"};
+    long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) {
+      // neither an int nor an index, but a number that int() takes (numpy's float32, a tensor of one float, a Decimal)
+      PyErr_Clear();
+      const py::object number = py::reinterpret_steal<py::object>(PyNumber_Check(o) ? PyNumber_Long(o) : nullptr);
+      if (number) v = PyLong_AsLongLong(number.ptr());
+      if (!number || (v == -1 && PyErr_Occurred())) throw Refused{"an int"};
+    }
     return v;
   }
 };
@@ -80,6 +87,7 @@ struct From<const std::string &> {
     Py_ssize_t n = 0;
     const char *text = PyUnicode_Check(o) ? PyUnicode_AsUTF8AndSize(o, &n) : nullptr;
     if (!text && PyBytes_Check(o)) text = PyBytes_AS_STRING(o), n = PyBytes_GET_SIZE(o);
+    if (!text && PyByteArray_Check(o)) text = PyByteArray_AS_STRING(o), n = PyByteArray_GET_SIZE(o);
     if (!text) throw Refused{"a str"};
     return std::string(text, (size_t)n);
   }

@@ -1,5 +1,7 @@
 """Host side of the drop-in operator surface (runs without a GPU)."""
 import re
+from decimal import Decimal
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -152,7 +154,7 @@ def test_arguments_of_other_types_are_refused(loaded):
     x, slots = torch.randn(4, 64).bfloat16(), torch.zeros(4, dtype=torch.int64)
     ln, lstm, argmax = (ops._IMPLS[n] for n in ("speculator_add_ln_act_cuda", "sum_lstm_zero_cell_cuda", "speculator_argmax_cuda"))
     good = [x, None, x, None, 1.0, 1e-6, "gelu", 1.0]
-    for at, others in ((0, [torch.nn.Parameter(x)]), (4, [1, np.float32(1.0), True]), (6, [b"gelu"])):
+    for at, others in ((0, [torch.nn.Parameter(x)]), (4, [1, np.float32(1.0), True]), (6, [b"gelu", bytearray(b"gelu")])):
         for other in others:
             with pytest.raises(RuntimeError, match="input must be CUDA"):
                 ln(*good[:at], other, *good[at + 1:])
@@ -164,10 +166,10 @@ def test_arguments_of_other_types_are_refused(loaded):
         ln(*good[:-1])
     with pytest.raises(TypeError):
         ln(*good[:-1], out_scale=1.0)
-    for accepted in (63, True, np.int64(63), torch.tensor(63)):
+    for accepted in (63, True, np.int64(63), torch.tensor(63), np.float32(63), torch.tensor(63.0), Decimal(63), Fraction(63)):   # the last four by int()
         with pytest.raises(RuntimeError, match="logits must be CUDA"):
             argmax(x, accepted)
-    for refused in (63.0, "63", None, 1 << 70):
+    for refused in (63.0, np.float64(63), "63", None, 1 << 70, Decimal(1 << 70), Decimal("inf"), 63j, np.ones(2)):
         with pytest.raises(TypeError, match="incompatible function arguments"):
             argmax(x, refused)
     s4 = torch.randn(4, 256).bfloat16()
