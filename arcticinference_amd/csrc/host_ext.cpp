@@ -20,7 +20,8 @@ namespace {
 namespace py = pybind11;
 using arctic_host::OptTensor;
 
-bool is_tensor(PyObject *o) { return (PyObject *)Py_TYPE(o) == THPVariableClass || THPVariable_Check(o); }
+// By the object's own type: a proxy or a mock that calls itself a Tensor holds none, and the question must not raise.
+bool is_tensor(PyObject *o) { return PyType_IsSubtype(Py_TYPE(o), (PyTypeObject *)THPVariableClass); }
 
 // ---- functions of positional arguments, called by Python's vector call -----------------------------------------
 // A call of an operator costs as much in the conversion of its arguments as in its checks, so these take what Python
@@ -145,11 +146,13 @@ void def(py::module_ &m, const char *name) {
 }
 
 // Whether `o`, or the first element of the list or tuple `o`, is a tensor on a GPU: what decides whether a call goes
-// straight to the functions below.
+// straight to the functions below.  A tensor subclass may answer for its device in Python, and raise there.
 PyObject *on_gpu(PyObject *, PyObject *o) {
+  HANDLE_TH_ERRORS
   if (PyList_Check(o) && PyList_GET_SIZE(o)) o = PyList_GET_ITEM(o, 0);
   else if (PyTuple_Check(o) && PyTuple_GET_SIZE(o)) o = PyTuple_GET_ITEM(o, 0);
   return PyBool_FromLong(is_tensor(o) && THPVariable_Unpack(o).is_cuda());
+  END_HANDLE_TH_ERRORS
 }
 
 // A Python list or tuple of tensors, read in place.

@@ -1,5 +1,6 @@
 """Host side of the drop-in operator surface (runs without a GPU)."""
 import re
+import weakref
 from decimal import Decimal
 from fractions import Fraction
 
@@ -181,6 +182,35 @@ def test_arguments_of_other_types_are_refused(loaded):
             lstm(s4, s4, None, None, None, None, 1.0, 1e-6, 1e-6, refused)
     with pytest.raises(TypeError):
         ops._IMPLS["gather_rows"](None, slots, [x])
+
+
+class NoDevice(torch.Tensor):
+    """A tensor that answers for its device in Python, with an error."""
+    @staticmethod
+    def __new__(cls):
+        return torch.Tensor._make_wrapper_subclass(cls, (4, 64), dispatch_device=True, device="meta")
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        raise LookupError("this tensor has no device")
+
+
+def test_the_question_for_the_device_raises_and_does_not_abort(loaded):
+    """What decides whether a call goes past the dispatcher is asked of whatever the caller hands over: an error of the
+    object's own reaches the caller as one."""
+    with pytest.raises(LookupError, match="no device"):
+        ops.speculator_argmax(NoDevice(), 3)
+    tensor = torch.zeros(2, 64)
+    proxy = weakref.proxy(tensor)
+    with pytest.raises(TypeError):
+        ops.speculator_argmax(proxy, 3)
+    with pytest.raises(TypeError, match="incompatible function arguments"):
+        ops._IMPLS["speculator_argmax_cuda"](proxy, 3)
+    del tensor
+    with pytest.raises((ReferenceError, TypeError)):
+        ops.speculator_argmax(proxy, 3)
+    with pytest.raises((ReferenceError, TypeError)):
+        ops.gather_rows([proxy], torch.zeros(1, dtype=torch.int64), [proxy])
 
 
 def test_missing_library_fails_loudly(monkeypatch):
