@@ -61,10 +61,11 @@ at::Tensor new_empty_strided(at::IntArrayRef sizes, at::IntArrayRef strides, con
   if (undispatched(like)) return at::detail::empty_strided_cuda(sizes, strides, like.scalar_type(), like.device());
   return at::empty_strided(sizes, strides, like.options());
 }
-// at::empty_like: of a matrix whose rows are `cols` or more apart that is a dense one.
+// at::empty_like: of a matrix whose rows are `cols` or more apart that is a dense one.  Who listens is asked for an empty_like:
+// a subclass makes one of its own kind, and names stay.
 at::Tensor new_like(const at::Tensor &t) {
   if (t.dim() == 2 && t.size(0) >= 1 && t.size(1) > 1 && t.stride(1) == 1 &&
-      (t.size(0) == 1 ? t.stride(0) == t.size(1) : t.stride(0) >= t.size(1)))
+      (t.size(0) == 1 ? t.stride(0) == t.size(1) : t.stride(0) >= t.size(1)) && undispatched(t))
     return new_empty(t.sizes(), t.scalar_type(), t);
   return at::empty_like(t);
 }

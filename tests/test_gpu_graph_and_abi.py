@@ -327,3 +327,49 @@ def test_outputs_are_made_as_the_dispatcher_makes_them(ops, form):
             assert a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype and a.device == b.device
             assert torch.equal(a, b) and not b.requires_grad
     assert all(t.is_inference() for t in inferred) and not any(t.is_inference() for t in got)
+
+
+class Marked(torch.Tensor):
+    """A tensor subclass that sees the operators called with it and makes its own kind of their results."""
+    asked = []
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        cls.asked.append(str(func))
+        guard = torch._C._DisableTorchDispatch()
+        out = func(*args, **(kwargs or {}))
+        del guard
+        return torch.Tensor._make_subclass(cls, out) if isinstance(out, torch.Tensor) else out
+
+
+class Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("form", ["dense", "pitched", "one row"])
+def test_the_norm_asks_a_listener_for_an_empty_like(ops, form):
+    """The norm's output is an `empty_like` of its input for whoever looks at the operators: a tensor subclass is asked for
+    it and makes one of its own kind, a dispatch mode sees that operator and no other, names are kept."""
+    memory = torch.randn(5, 96, device=DEV).bfloat16()
+    x = {"dense": lambda: memory[:, :64].contiguous(), "pitched": lambda: memory[:, :64], "one row": lambda: memory[:1]}[form]()
+    table, ids = torch.randn(3, x.size(1), device=DEV).bfloat16(), torch.zeros(x.size(0), dtype=torch.int64, device=DEV)
+    calls = [lambda x: ops.speculator_ln(x, None, None, 1e-6),
+             lambda x: ops.speculator_embed_add_ln_gelu(x, table, ids, None, None, 0.5, 1e-6)]
+    for call in calls:
+        want = call(x)
+        Marked.asked.clear()
+        got = call(torch.Tensor._make_subclass(Marked, x))
+        assert type(got) is Marked and "aten.empty_like.default" in Marked.asked
+        assert got.stride() == want.stride() and torch.equal(got.as_subclass(torch.Tensor), want)
+        with Seen() as mode:
+            got = call(x)
+        assert mode.names.count("aten.empty_like.default") == 1 and torch.equal(got, want)
+        if form != "one row":   # those are viewed as rows first, which names do not allow
+            got = call(x.rename("row", "column"))
+            assert got.names == ("row", "column") and torch.equal(got.rename(None), want)
