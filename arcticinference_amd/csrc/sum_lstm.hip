@@ -492,6 +492,22 @@ static bool in_place(const LstmCall &p, int64_t rows, bool shared_z) {
 template <typename T, bool kFastGelu, bool kSharedZ>
 static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   const bool multi = rows > 1;
+  // The vector kernels' arguments are 32 bits wide.  Rows 2^32 elements and more apart (8 GiB, so there are few) are launched
+  // one by one, where no pitch counts; a table of embeddings with such rows is the element-wise kernel's.
+  const auto fits = [](int64_t v) { return v <= (int64_t)UINT32_MAX; };
+  if (multi && !(fits(p.s_stride) && fits(p.pc_stride) && fits(p.out_stride) && (p.z_index || fits(p.z_stride)))) {
+    for (int64_t r = 0; r < rows; ++r) {
+      LstmCall one = p;
+      one.out_state += r * p.out_stride * 2;
+      one.out_cell += r * p.out_stride * 2;
+      one.states += r * p.s_stride * 2;
+      if (p.prev_cell) one.prev_cell += r * p.pc_stride * 2;
+      if (p.z_index) one.z_index += r;
+      else one.z4 += r * p.z_stride * 2;
+      launch_lstm<T, kFastGelu, kSharedZ>(one, 1, s);
+    }
+    return;
+  }
   const bool aligned = p.D % 8 == 0 &&
                        (!multi || (p.s_stride % 8 == 0 && p.z_stride % 8 == 0 && p.pc_stride % 8 == 0 &&
                                    p.out_stride % 8 == 0)) &&
@@ -533,11 +549,7 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
   // and nothing orders the one's load before the other's store: such a call goes element by element.  Aligned rows that
   // lack a vector are requested together, since the stages read the output gate behind the first store.
   const bool aliased = (p.D % 8 || !all_vectors) && in_place(p, rows, kSharedZ);
-  // (strides and rows of 2^32 elements and more are the element-wise kernel's: the others' arguments are 32 bits wide)
-  const auto fits = [](int64_t v) { return v <= (int64_t)UINT32_MAX; };
-  const bool wide = (multi && !(fits(p.s_stride) && fits(p.pc_stride) && fits(p.out_stride))) ||
-                    ((multi || p.z_index) && !fits(p.z_stride)) || !fits(p.z_rows);
-  const bool element_wise = narrow || (aliased && p.D % 8) || wide || chunks > 2 * 1024;
+  const bool element_wise = narrow || (aliased && p.D % 8) || !fits(p.z_rows) || (p.z_index && !fits(p.z_stride)) || chunks > 2 * 1024;
   LstmParamsOf<kSharedZ> compact;
   static_cast<LstmParams<uint32_t> &>(compact) = {
       p.out_state, p.out_cell, p.states, p.z4, p.prev_cell, p.w_cell, p.b_cell, p.w_state, p.b_state, (uint32_t)p.s_stride,

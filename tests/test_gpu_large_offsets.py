@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import oracle
+from arcticinference_amd import _native
 from helpers import assert_close, speculator_alpha
 
 pytestmark = pytest.mark.gpu
@@ -91,7 +92,7 @@ def test_sum_lstm_beyond_four_gib(ops):
 
 @pytest.mark.parametrize("pitch", [(1 << 32) - 8, 1 << 32])
 def test_sum_lstm_row_pitch_around_32_bits(ops, pitch):
-    """The vector kernels take pitches of 32 bits; the element-wise one takes what lies beyond."""
+    """The vector kernels take pitches of 32 bits; rows that lie further apart are launched one by one."""
     D = 512
     memory = torch.empty(pitch + 4 * D, dtype=torch.bfloat16, device=DEV)
     states = memory.as_strided((2, 4 * D), (pitch, 1))
@@ -104,6 +105,24 @@ def test_sum_lstm_row_pitch_around_32_bits(ops, pitch):
     want_s, want_c = oracle.sum_lstm(s, z4, cell, w_cell, b_cell, w_state, b_state, 0.35, 1e-6, 1e-6, False)
     assert_close(got_c.cpu(), want_c, RTOL, ATOL, "cell")
     assert_close(got_s.cpu(), want_s, RTOL, ATOL, "state")
+    # the same bits as rows that lie close together, with four z, one z and one looked up
+    close_by = s.to(DEV)
+    vec = [v.to(DEV) for v in (w_cell, b_cell, w_state, b_state)]
+    z, table, ids = z4.to(DEV), torch.randn(5, D, generator=g).to(torch.bfloat16).to(DEV), torch.tensor([4, 1], device=DEV)
+    for op in (lambda x: ops.sum_lstm(x, z, cell.to(DEV), *vec, 0.35, 1e-6, 1e-6, False),
+               lambda x: ops.sum_lstm_shared_z(x, z[:, :D], None, *vec, 0.35, 1e-6, 1e-6, True),
+               lambda x: ops.sum_lstm_embedded(x, table, ids, cell.to(DEV), None, None, None, None, 0.35, 1e-6, 1e-6, False)):
+        for got, want in zip(op(states), op(close_by)):
+            assert torch.equal(got, want)
+    # without vectors the new cell may be stored over the output gate (test_updates_in_place) at any pitch
+    want_s, want_c = oracle.sum_lstm(s, z4, cell, None, None, None, None, 0.35, 1e-6, 1e-6, False)
+    state = torch.empty(pitch + D, dtype=torch.bfloat16, device=DEV).as_strided((2, D), (pitch, 1))
+    new_cell, dcell = states[:, 2 * D:3 * D], cell.to(DEV)
+    _native.check(_native.load().arctic_sum_lstm(
+        state.data_ptr(), new_cell.data_ptr(), states.data_ptr(), z.data_ptr(), dcell.data_ptr(), None, None, None, None, 2, D,
+        pitch, 4 * D, D, pitch, 0.35, 1e-6, 1e-6, 0, _native.DTYPE_BF16, torch.cuda.current_stream().cuda_stream))
+    assert_close(new_cell.cpu(), want_c, RTOL, ATOL, "cell over the output gate")
+    assert_close(state.cpu(), want_s, RTOL, ATOL, "state")
 
 
 def test_speculator_ln_beyond_four_gib(ops):
