@@ -221,7 +221,7 @@ __device__ __forceinline__ void select_leftover_rows(const BulkSelectParams &p, 
 // kBulkThreads x kUnroll 16-byte chunks form one batch of a workgroup.  Three shapes are built, all with batches
 // of 1024 chunks: 1024 x 1 (launches of more than 8192 tokens, or 4096 of rows that are no power of two long: a workgroup
 // moves up to five batches), 512 x 2 (launches of more than 8192 tokens that select rows as well) and 256 x 4 (everything
-// smaller: at most two batches per workgroup).
+// else: about two batches per workgroup, up to five where more than 8192 tokens of rows that are no power of two long select).
 template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, typename Params, typename Tables>
 __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, unsigned block) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
@@ -737,10 +737,14 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       //  - above that, the wide shape (batches of 1024 chunks by 1024 lanes, by 512 lanes when rows are selected as well)
       //    with up to five batches per workgroup (20 layers of 8 x 128 bf16) and at least about 1024 workgroups; a
       //    workgroup that would get less than two batches takes the 256-lane shape instead.
-      // Rows that are no power of two long take the wide shape from 4097 tokens on where its batches come out filled: a
-      // lane's loads of a batch that is not full are idle slots of 1024-lane workgroups, of which only two run per CU (us,
-      // 256 lanes / 1024: 5003 x 33 of 3 x 96 72.1 / 69.0, three batches 77 % full; 16384 x 40 of it 305 / 285, 94 %; 8000
-      // x 33 of 3 x 80 117 / 111, 97 %; a single batch at 94 % 55.2 / 53.8, at 77 % 72 / 81; two batches at 56 % 56.6 / 59.4).
+      // Rows that are no power of two long take the wide shape from 4097 tokens on where a workgroup has three batches or
+      // more, however full the last one (us, 256 lanes / 1024, fp8: 5003 x 33 of 3 x 96 73.1 / 71.3, 16384 x 40 of 3 x 80
+      // 295 / 276, 8193 x 61 of 5 x 80 346 / 306, three batches 70 % full 8193 x 36 of 3 x 80 129 / 122; of 300 drawn calls up
+      // to 8192 tokens the middle one is 1 % faster and the slowest 2.7 % slower, of 540 above 3 % faster and 1.4 % slower).
+      // With one or two batches a lane has too few loads in flight to pay for a CU that holds two workgroups only: 5437 x 12
+      // of 5 x 64 28.4 / 33.8, 4097 x 32 of 3 x 64 31.9 / 36.3, 5101 x 40 of 3 x 64 49.3 / 52.3, 9066 x 4 of 1 x 832 23 %
+      // slower; only copies, which store twice as much, gain there as well where a single batch comes out 7/8 and two 3/4
+      // full (two at 75 %, 8000 x 32 of 3 x 64 75.8 / 73.3; one at 94 %, 6572 x 20 of it 39.3 / 38.5).
       int groups = 1;
       bool wide = false;
       if (vec) {
@@ -754,7 +758,8 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
         if (num_tokens > 8192 || (ragged && !select && num_tokens > 4096)) {
           const int64_t g = limit(std::max(ceil_div(1024, num_tokens), ceil_div(chunks_per_layer * count, 5 * kBatch)));
           const int64_t chunks = ceil_div(count, g) * chunks_per_layer, slots = ceil_div(chunks, kBatch) * kBatch;
-          wide = ragged && !select ? chunks * 8 >= slots * (slots == kBatch ? 7 : 6) : chunks >= 2 * kBatch;
+          if (!ragged || select) wide = chunks >= 2 * kBatch;
+          else wide = chunks > 2 * kBatch || (!quant && chunks * 8 >= slots * (slots == kBatch ? 7 : 6));
           if (wide) groups = (int)g;
         }
         if (wide) {
