@@ -600,9 +600,11 @@ static void launch_lstm(const LstmCall &p, int64_t rows, hipStream_t s) {
     const int parts = (lanes + 255) / 256;
     const int64_t rows_up = (rows + 7) & ~(int64_t)7;
     const bool in_parts = parts > 1 && rows_up * parts <= (lanes % 256 ? 224 : 256) && !in_place(p, rows, kSharedZ);
-    // One z for all gates leaves few enough requests to make them ahead (embedded, in stages / ahead: 7 x 2880 3.90 / 3.71, 64 x
-    // 2880 4.89 / 4.55, 7 x 4096 3.98 / 3.82; 32 x 4096 without a previous cell 4.39 / 4.44, 32 x 6144 5.38 / 5.67).
-    const bool parts_ahead = lanes <= 384 || (lanes <= 512 && rows <= 16);
+    // One z for all gates leaves few enough requests to make them ahead (embedded, in stages / ahead: 7 x 2880 4.07 / 3.90, 64 x
+    // 2880 4.19 / 4.11, 7, 10, 16, 24, 32 and 64 x 4096 4.17 / 4.00, 4.17 / 3.97, 4.13 / 4.00, 4.21 / 4.02, 4.16 / 4.06 and 4.68 /
+    // 4.63, where it is level).  Rows at any alignment are not faster for it: pitched by 1, 8 x 3600 3.9 to 8 % slower, 8 x 4096 7 to
+    // 8 %, 8 x 2880 1 to 6 %, odd widths between 5 % faster and 4 % slower.
+    const bool parts_ahead = aligned && (lanes <= 384 || (lanes <= 512 && rows <= 16));
     LstmPartsParams<kSharedZ> of_parts;
     if (in_parts) {
       static_cast<LstmParamsOf<kSharedZ> &>(of_parts) = compact;
