@@ -731,7 +731,9 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       //    33 of 3 x 80 15.3 / 13.3).  Copies, which store twice as much, do so up to seven per
       //    CU: of 230 drawn ones with 1792 to 2048 workgroups, plain and selecting, the middle one is 4 % faster and the slowest
       //    are 5 to 6 % slower (316 x 31 of 10 x 64 11.5 / 12.1, 1002 x 14 of 6 x 96 12.5 / 13.0; selecting 993 x 7 of 16 x
-      //    64 18.1 / 19.3); fp8 there, 420 drawn, is 9 % faster, the slowest 3 % slower (244 x 57 of 8 x 64 10.5 / 10.9);
+      //    64 18.1 / 19.3), and so do plain fp8 rows of a power of two, whose second batch is a full layer or two (80 drawn, the
+      //    middle one 3 % faster, 245 x 58 of 4 x 128 11.0 / 11.7, 493 x 14 of 8 x 128 10.8 / 11.3); other fp8 rows there
+      //    gain 9 %, selecting ones of any length 11 %;
       //  - fewer than about 512 such workgroups leave CUs idle or with a wave or two per SIMD, whose instructions count
       //    then: more and smaller ones, a chunk per lane at the least (5 x 16 of 8 x 128 3.61 / 3.19, 5 x 40 of 3 x 96
       //    4.59 / 3.70, 30 x 16 of 8 x 128 3.80 / 3.49; from 800 workgroups on it is level, behind 2048 each one more
@@ -769,7 +771,7 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
           // as above
         } else if (num_tokens > 8192) {
           groups = (int)limit(std::min(ceil_div(kSideBySide, num_tokens), count / min_layers));
-        } else if (num_tokens * one_batch_groups <= (quant ? kSideBySide : kSideBySide * 7 / 8)) {
+        } else if (num_tokens * one_batch_groups <= (quant && (ragged || select) ? kSideBySide : kSideBySide * 7 / 8)) {
           const int64_t fewest_layers = std::max<int64_t>(1, ceil_div(kFewestChunks, chunks_per_layer));
           groups = (int)limit(std::max(one_batch_groups, std::min(kFewWorkgroups / num_tokens, ceil_div(count, fewest_layers))));
         } else {

@@ -86,6 +86,7 @@ def test_layers_at_the_edges_of_the_pointer_tables(ops, L, heads_of, kv):
     dict(T=1, L=40, H=3, D=96), dict(T=31, L=40, H=1, D=128),      # a chunk per lane, groups with a ragged tail
     dict(T=682, L=40, H=3, D=96), dict(T=683, L=40, H=3, D=96),    # 2046 workgroups of one batch; two batches each
     dict(T=597, L=40, H=3, D=96), dict(T=598, L=40, H=3, D=96),    # 1791 workgroups; 1794: two batches each for copies
+    dict(T=128, L=14, H=32, D=128), dict(T=129, L=14, H=32, D=128),  # the same with rows of a power of two, fp8 too
     dict(T=1024, L=17, H=3, D=80), dict(T=1025, L=18, H=3, D=80),  # one batch per token; nothing smaller than a batch
     dict(T=4096, L=16, H=3, D=80), dict(T=4097, L=16, H=3, D=80),  # 256 lanes; 1024 lanes for copies, a batch 94 % full
     dict(T=4097, L=14, H=3, D=80), dict(T=4097, L=27, H=3, D=80),  # 82 % full: 256 lanes; two batches, 79 %: 1024 for copies
