@@ -73,6 +73,19 @@ def test_layer_groups_more_than_one_launch_and_tiny_batches(ops, T, L):
     run_select(ops, case, idx, T)
 
 
+@pytest.mark.parametrize("T,L,H,D", [
+    (1, 16, 8, 128), (5, 40, 3, 96), (31, 40, 1, 128), (85, 12, 8, 128), (86, 12, 8, 128),   # a chunk per lane; 512 workgroups
+    (597, 40, 3, 96), (598, 40, 3, 96), (682, 40, 3, 96), (683, 40, 3, 96),   # 1791, 1794, 2046 workgroups of one batch; two batches
+    (128, 14, 32, 128), (129, 14, 32, 128), (146, 14, 32, 128), (147, 14, 32, 128),   # the same lines, rows of a power of two
+    (2049, 4, 3, 80), (4097, 35, 3, 80), (8193, 6, 3, 80), (8193, 35, 3, 80), (8193, 16, 1, 128)])   # by row map; the wide shapes' lines
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+def test_layers_split_over_workgroups(ops, kv, T, L, H, D):
+    """Every workgroup of a token stores and copies its own layers, whether it scans the list or looks into the row map: all
+    tokens selected, the last one first."""
+    case = make_bulk_case(T=T, L=L, H=H, D=D, bs=16, NB=T // 16 + 2, kv_cache_dtype=kv, seed=T + L, std=1.5, pad_fraction=0.05)
+    run_select(ops, case, torch.arange(T - 1, -1, -1), T)
+
+
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 def test_rows_that_force_the_element_wise_kernel(ops, kv):
     # 3 heads x 20 = 60 elements per row and an odd output pitch: no 16-byte access possible
