@@ -21,7 +21,7 @@ namespace py = pybind11;
 using arctic_host::OptTensor;
 
 // By the object's own type: a proxy or a mock that calls itself a Tensor holds none, and the question must not raise.
-bool is_tensor(PyObject *o) { return PyType_IsSubtype(Py_TYPE(o), (PyTypeObject *)THPVariableClass); }
+bool is_tensor(PyObject *o) { return PyObject_TypeCheck(o, (PyTypeObject *)THPVariableClass); }
 
 // ---- functions of positional arguments, called by Python's vector call -----------------------------------------
 // A call of an operator costs as much in the conversion of its arguments as in its checks, so these take what Python
