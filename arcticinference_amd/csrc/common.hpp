@@ -42,9 +42,11 @@ struct Divisor {
 // A launch.  The host writes a launch's arguments into the GPU's memory, and what that costs is the processor's stores over
 // the bus: an empty kernel with one structure of up to 112 bytes is issued in 2.4 to 2.8 us (two levels, by where the process
 // runs), with one of 256 to 768 bytes in 2.5 to 3.5 us, with 2288 bytes in 2.6 to 3.8 us, and with ten scalars in place of a
-// structure of 64 bytes in 2.5 to 3.3 us.  The kernels that small calls take therefore have one structure or two, as small as
-// their contents allow, and none of them asks for blockDim or gridDim: for those the runtime appends 256 bytes.  The structures
-// go to the runtime from where they are, without the copy that passing them by value to the kernel's host-side function makes.
+// structure of 64 bytes in 2.5 to 3.3 us.  The kernels launched here (the cache writes in 16-byte accesses, the norm, the gate
+// update, the argmax) therefore have one structure or two, as small as their contents allow, but for the tables of 64 layers
+// that every selecting write carries, and none of them asks for blockDim or gridDim: for those the runtime appends 256 bytes.
+// The structures go to the runtime from where they are, without the copy that passing them by value to the kernel's host-side
+// function makes.  (The row gather, the row map and the element-wise cache write are launched the usual way.)
 template <typename... Args>
 inline void launch(void (*kernel)(Args...), dim3 grid, int lanes, hipStream_t s, const Args &...args) {
   void *list[] = {const_cast<Args *>(&args)...};
@@ -171,7 +173,8 @@ __device__ __forceinline__ void store16_stream(void *p, const uint4 &v) {
 }
 
 // A lane's unit of work on the speculator paths: eight consecutive 16-bit elements
-// moved with one 16-byte access (narrower units measured slower).
+// moved with one 16-byte access.  (8-byte units with twice the lanes took 512 rows of 4096 of the gate update in 10.7 us where
+// these took 10.0, all requests at once; that is the only size they were timed at, few rows were not.)
 struct Chunk {
   static constexpr int kElems = 8;
   static constexpr int kBytes = 16;

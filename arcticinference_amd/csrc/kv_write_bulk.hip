@@ -221,7 +221,8 @@ __device__ __forceinline__ void select_leftover_rows(const BulkSelectParams &p, 
 // kBulkThreads x kUnroll 16-byte chunks form one batch of a workgroup.  Three shapes are built, all with batches
 // of 1024 chunks: 1024 x 1 (launches of more than 8192 tokens, or 4096 of rows that are no power of two long: a workgroup
 // moves up to five batches), 512 x 2 (launches of more than 8192 tokens that select rows as well) and 256 x 4 (everything
-// else: about two batches per workgroup, up to five where more than 8192 tokens of rows that are no power of two long select).
+// else: up to two batches per workgroup, rounded up to whole layers, and up to five where more than 8192 tokens of rows
+// that are no power of two long select).
 template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, typename Params, typename Tables>
 __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, unsigned block) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
@@ -737,7 +738,10 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       //  - fewer than about 512 such workgroups leave CUs idle or with a wave or two per SIMD, whose instructions count
       //    then: more and smaller ones, a chunk per lane at the least (5 x 16 of 8 x 128 3.61 / 3.19, 5 x 40 of 3 x 96
       //    4.59 / 3.70, 30 x 16 of 8 x 128 3.80 / 3.49; from 800 workgroups on it is level, behind 2048 each one more
-      //    costs: 512 x 40 of 3 x 96 in 4 groups 9.95, in 5 11.7);
+      //    costs: 512 x 40 of 3 x 96 in 4 groups 9.95, in 5 11.7).  Writes that select rows gain more, although each
+      //    of their workgroups looks through the whole index list (fp8, all rows selected, in two to ten groups / in three to
+      //    25: 1, 5, 20 and 64 x 16 of 8 x 128 4.42 / 3.25, 4.54 / 3.33, 4.72 / 3.70 and 5.23 / 4.45, 20 x 40 5.17 / 4.63, 20
+      //    and 512 x 33 of 3 x 96 5.71 / 4.13 and 14.3 / 11.9; the row map serves lists too long for these launches);
       //  - more tokens, up to 8192: about two batches (8 layers of 8 x 128) per workgroup, never less than one each;
       //  - above that, the wide shape (batches of 1024 chunks by 1024 lanes, by 512 lanes when rows are selected as well)
       //    with up to five batches per workgroup (20 layers of 8 x 128 bf16) and at least about 1024 workgroups; a
