@@ -256,10 +256,13 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
       col = c - r * cpr;
     }
   };
-  // kUnroll independent 16-byte loads per lane; lanes past the end load nothing
-  auto load_batch = [&](int c, uint4 (&v)[kUnroll]) {
+  constexpr std::integral_constant<int, 0> kNone;
+  constexpr std::integral_constant<int, kUnroll / 2> kHalf;
+  constexpr std::integral_constant<int, kUnroll> kAll;
+  // independent 16-byte loads `from` ... `to` - 1 of a lane's kUnroll; lanes past the end load nothing
+  auto load_part = [&](int c, uint4 (&v)[kUnroll], auto from, auto to) {
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = decltype(from)::value; u < decltype(to)::value; ++u) {
       const int cu = c + u * kBulkThreads;
       if (cu < total) {
         int r, col;
@@ -270,10 +273,16 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
     }
   };
 
-  // The slot lookup and the first batch of source loads are issued together:
-  // source addresses do not depend on the slot, so HBM is already streaming
-  // while the row descriptors below are being built.  (A padding token throws
-  // its first batch away.)
+  // The first half of the first batch is requested together with the slot (source addresses do not depend on it), the
+  // rest behind it: a padding token then throws half a batch away, or nothing in the shape of one chunk per lane.  With one
+  // batch per workgroup and 30 % padding what the padding's whole first batches read was 22 % of a launch's traffic; with
+  // nothing requested ahead CUs that hold a few short-lived workgroups wait for their slots.  Us per call in a graph, bf16 to
+  // fp8, all / none / two of a lane's four chunks ahead: 8192 x 16 of 8 x 128 156.4 / 157.0 / 155.7 without padding, 145.8 /
+  // 143.1 / 144.3 with 10 %, 124.9 / 110.9 / 117.3 with 30 %; without padding 512 x 40 23.7 / 24.2 / 23.8, 1024 x 16 18.7 /
+  // 19.0 / 18.7, 512 x 16 10.2 / 10.0 / 9.9, 64 x 16 3.71 / 3.73 / 3.49; in the 1024-lane shape, all / none, 16384 x 40 762.7 /
+  // 763.1 without padding, 695.9 / 687.3 with 10 %, 575 / 548 with 30 %.  Where the index list is scanned
+  // the scan stands between the slot and the stores already, and batches are requested whole (half ahead, 448 x 16 of 3 x 96,
+  // copied, 112 selected: 6.5 / 7.0).
   const int64_t slot = p.slot_mapping[token];
   int64_t out_row = -1;
   if constexpr (kSelect == kSelectByRowMap) out_row = p.row_map[token];
@@ -293,9 +302,20 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
     }
     if (threadIdx.x == 0) num_hits = 0;
   }
+  // padding (or a slot outside the cache) writes no cache row; this and to_out below are uniform over the workgroup
+  const bool to_cache = slot >= 0 && slot < p.num_slots;
+  bool to_out = false;
+  if constexpr (kSelect == kSelectByRowMap) to_out = out_row >= 0 && out_row < p.num_out_rows;
   int c = threadIdx.x;
   uint4 cur[kUnroll];
-  load_batch(c, cur);
+  if constexpr (kSelect == kSelectByScan) {
+    load_part(c, cur, kNone, kAll);
+  } else {
+    load_part(c, cur, kNone, kHalf);
+    __builtin_amdgcn_sched_barrier(0);   // ahead of the wait for the slot
+    if (!to_cache && !to_out) return;
+    load_part(c, cur, kHalf, kAll);
+  }
   int nhits = 0;
   if constexpr (kSelect == kSelectByScan) {
     __syncthreads();
@@ -304,12 +324,9 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
       if (mine[k] == token) hits[atomicAdd(&num_hits, 1)] = threadIdx.x + k * kBulkThreads;
     __syncthreads();
     nhits = num_hits;
+    to_out = nhits > 0;
+    if (!to_cache && !to_out) return;   // uniform, and behind the scan's barriers
   }
-  // padding (or a slot outside the cache) writes no cache row; both tests are uniform over the workgroup
-  const bool to_cache = slot >= 0 && slot < p.num_slots;
-  bool to_out = nhits > 0;
-  if constexpr (kSelect == kSelectByRowMap) to_out = out_row >= 0 && out_row < p.num_out_rows;
-  if (!to_cache && !to_out) return;  // uniform, and behind the scan's barriers
 
   if (to_cache) {
     int64_t blk, off;
@@ -377,7 +394,7 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
         }
       }
     }
-    load_batch(cn, nxt);
+    load_part(cn, nxt, kNone, kAll);
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) cur[u] = nxt[u];
     c = cn;

@@ -86,6 +86,18 @@ def test_layers_split_over_workgroups(ops, kv, T, L, H, D):
     run_select(ops, case, torch.arange(T - 1, -1, -1), T)
 
 
+@pytest.mark.parametrize("T,L,H,D", [
+    (512, 16, 8, 128), (2100, 33, 1, 80), (8193, 16, 4, 128)])   # 256 lanes, rows of a power of two and others; 512 lanes
+@pytest.mark.parametrize("selected", [60, 2050])
+def test_padding_that_is_selected_in_every_shape(ops, T, L, H, D, selected):
+    """Half of the tokens are padding, and half of the selected ones: by scan (up to 2048 indices) and by row map."""
+    case = make_bulk_case(T=T, L=L, H=H, D=D, bs=16, NB=T // 16 + 2, kv_cache_dtype="fp8", seed=T, std=1.5, pad_fraction=0.5)
+    g = torch.Generator().manual_seed(selected)
+    pads, valid = ((case["slot_mapping"] < 0) == b for b in (True, False))
+    some = [torch.nonzero(m).flatten()[torch.randint(0, int(m.sum()), (selected // 2,), generator=g)] for m in (pads, valid)]
+    run_select(ops, case, torch.cat(some)[torch.randperm(selected // 2 * 2, generator=g)], selected + 1)
+
+
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 def test_rows_that_force_the_element_wise_kernel(ops, kv):
     # 3 heads x 20 = 60 elements per row and an odd output pitch: no 16-byte access possible
