@@ -329,19 +329,33 @@ __global__ __launch_bounds__(kSplitLanes) void row_argmax_split_kernel(const Arg
 using namespace arctic;
 
 // How many workgroups share a row (1: not split), and the elements of each one's segment.  The exchange costs about
-// a microsecond (store, acknowledgement, read), so a row is split when it is long and the rows are few enough that each
-// gets six workgroups or more out of about 512 (two per CU): us per call inside a graph, not split / split,
-//   rows x 128256 bf16:   1 row 6.2 / 3.9,  7 rows 6.7 / 4.4,  32 rows 7.6 / 5.3,  64 rows 7.9 / 6.5,  128 rows 8.6 / 8.7
-//   rows x 50257 bf16:    1 row 3.6 / 3.7,  7 rows 3.9 / 4.2,  64 rows 5.2 / 5.1;    7 rows x 262144: 11.6 / 4.8
-// which cross at about 8000 chunks of 16 bytes per row.  Segments shorter than 1024 chunks and more than 16 of them gain
-// nothing (7 rows x 128256: 32 parts 4.7 us); workgroups of 256 and 1024 lanes are 0.1-0.2 us slower.
+// a microsecond (store, acknowledgement, read), so a row is split where that buys more (us per call in a graph, not split /
+// split, rows x bf16 columns):
+//  - up to 128 rows, which leave CUs idle: the more rows the longer they have to be (1 x 65536 4.21 / 3.95, 20 x 65536 5.16 /
+//    4.65, 41 x 65536 5.23 / 5.06, 64 x 65536 5.45 / 5.56; 64 x 80000 6.26 / 5.76, 70 x 80000 6.34 / 5.86; 86 x 128256 8.23 /
+//    7.48, 112 x 128256 8.62 / 8.45, 128 x 128256 2 % slower; 96 x 151936 9.48 / 8.74, 128 x 262144 9 % faster; 32000 and
+//    50257 columns between 8 % slower and 3 % faster; fp32, whose chunks are half as much work, 1 x 32768 3.74 / 4.22, 7 x 40000
+//    4.02 / 4.43);
+//  - up to a fifth more than one or two rows for every CU, where some CUs would do twice or half as much again as the others
+//    (264 x 128256 16.3 / 14.2, 304 x 128256 17.1 / 15.7, 288 x 151936 19.1 / 18.0, 257 x 80000 10.2 / 10.4, 320 x 100000 6 %
+//    faster to 320 x 80000 1 % slower; 513 x 128256 30.1 / 23.2, 704 x 128256 35.8 / 30.9, 640 x 80000 15 % faster, 640 x 65536
+//    6 %).  Only where every row starts on a 16-byte boundary: 264 x 128257 gains 1 %, 320 loses 4 %.
+// Up to sixteen segments of 1024 chunks or more while they make no more than two workgroups per CU (7 x 128256: 32 segments 4.7
+// us, 16 4.4), and not fewer than eight, of very long rows six (85 x 128256 six 7.93, eight 7.47, sixteen 8.08; 78 x 262144 six
+// 10.3, eight 10.8).  Workgroups of 256 and 1024 lanes are 0.1-0.2 us slower.
 static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
-  constexpr int64_t kMinChunksPerRow = 10240, kMinChunksPerPart = 1024, kMostParts = 16, kFewestParts = 6, kWorkgroups = 512;
+  constexpr int64_t kMostParts = 16, kParts = 8, kWorkgroups = 512, kMinChunksPerPart = 1024;
   *segment = cols;
   const int64_t chunks = dtype == ARCTIC_DTYPE_F32 ? cols / 4 : cols / 8;
-  if (rows <= 0 || chunks < kMinChunksPerRow) return 1;
-  const int64_t parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
-  if (parts < kFewestParts) return 1;
+  int64_t parts = 1;
+  const int64_t shortest = dtype == ARCTIC_DTYPE_F32 ? 10240 : rows <= 48 ? 8192 : 10000;
+  if (rows > 0 && rows <= 128 && chunks >= std::max(shortest, 140 * rows)) {
+    parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
+    if (parts < (chunks < 18000 ? kParts : 6)) parts = kParts;
+  } else if ((rows > 256 && rows <= 304 && chunks >= 12288) || (rows > 512 && rows <= 704 && chunks >= 10000)) {
+    parts = kParts;
+  }
+  if (parts == 1) return 1;
   *segment = (int)((cols + parts - 1) / parts + 63) & ~63;   // whole 128-byte lines of an aligned row
   return (cols + *segment - 1) / *segment;
 }
@@ -384,7 +398,7 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
   hipStream_t s = (hipStream_t)stream;
   int segment;
   const int parts = argmax_parts(rows, cols, dtype, &segment);
-  if (vec && parts > 1 && workspace) {
+  if (vec && parts > 1 && workspace && (aligned_rows || rows <= 256)) {
     if ((uintptr_t)workspace % 8 || workspace_bytes < rows * parts * (int64_t)sizeof(Segment))
       return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: the workspace must be 8-byte aligned and hold %lld bytes", fn,
                   (long long)(rows * parts * (int64_t)sizeof(Segment)));

@@ -193,6 +193,25 @@ def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
         assert torch.equal(got.cpu(), reference(x[:, :cols], cols - 1))
 
 
+@pytest.mark.parametrize("rows,cols,dtype,pad", [
+    (48, 65536, torch.bfloat16, 0), (48, 65535, torch.bfloat16, 0), (49, 65536, torch.float16, 0),   # 8192 chunks, and fewer
+    (71, 80000, torch.bfloat16, 0), (72, 80000, torch.bfloat16, 0), (85, 144000, torch.float16, 0),   # 140 chunks for each row; six segments
+    (128, 72000, torch.float32, 1), (129, 144512, torch.bfloat16, 0), (9, 40959, torch.float32, 0),   # the most rows that leave CUs idle; fp32
+    (256, 98304, torch.bfloat16, 0), (257, 98304, torch.bfloat16, 0), (304, 98304, torch.float16, 0), (305, 98304, torch.float16, 0),
+    (257, 98304, torch.bfloat16, 3),   # not aligned: not split
+    (512, 80000, torch.bfloat16, 0), (513, 80000, torch.bfloat16, 0), (704, 80000, torch.bfloat16, 0), (705, 80000, torch.float16, 0)])
+def test_row_counts_where_the_split_begins_and_ends(ops, rows, cols, dtype, pad):
+    """The winner in every eighth of a row, the cuts and both ends, ties of the first and the last place."""
+    x = torch.randint(-3, 2, (rows, cols + pad), generator=torch.Generator().manual_seed(rows), dtype=torch.int8).to(dtype)
+    places = [0, cols - 1, *(min(cols - 1, -(-cols // 8) * k + d) for k in range(1, 8) for d in (-1, 0, 63, 64))]
+    for r in range(0, rows, 2):
+        x[r, places[r // 2 % len(places)]] = 4.0
+        if r % 3 == 0:
+            x[r, cols - 1] = 4.0
+    for _ in range(2):
+        assert torch.equal(ops.speculator_argmax(x.to(DEV)[:, :cols], cols).cpu(), reference(x[:, :cols], cols))
+
+
 def test_split_rows_on_two_streams_at_once(ops):
     """Each call exchanges winners in memory of its own: calls of two streams that run at the same time do not meet."""
     cols = 128256
