@@ -338,8 +338,10 @@ using namespace arctic;
 //    4.02 / 4.43);
 //  - up to a fifth more than one or two rows for every CU, where some CUs would do twice or half as much again as the others
 //    (264 x 128256 16.3 / 14.2, 304 x 128256 17.1 / 15.7, 288 x 151936 19.1 / 18.0, 257 x 80000 10.2 / 10.4, 320 x 100000 6 %
-//    faster to 320 x 80000 1 % slower; 513 x 128256 30.1 / 23.2, 704 x 128256 35.8 / 30.9, 640 x 80000 15 % faster, 640 x 65536
-//    6 %).  Only where every row starts on a 16-byte boundary: 264 x 128257 gains 1 %, 320 loses 4 %.
+//    faster to 320 x 80000 1 % slower; 513 x 80000 16.1 / 15.9, 560 x 80000 17.4 / 16.7, 600 x 80000 17.5 / 17.7, 513 x 128256
+//    24.6 / 23.3, 600 x 128256 26.5 / 26.4, 640 x 128256 27.2 / 27.6, 704 x 128256 28.8 / 30.4, but 513 x 262144 51.0 / 44.6, 704 x 262144
+//    60.5 / 58.2).
+//    Only where every row starts on a 16-byte boundary: 264 x 128257 gains 1 %, 320 loses 4 %.
 // Up to sixteen segments of 1024 chunks or more while they make no more than two workgroups per CU (7 x 128256: 32 segments 4.7
 // us, 16 4.4), and not fewer than eight, of very long rows six (85 x 128256 six 7.93, eight 7.47, sixteen 8.08; 78 x 262144 six
 // 10.3, eight 10.8).  Workgroups of 256 and 1024 lanes are 0.1-0.2 us slower.
@@ -352,7 +354,7 @@ static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
   if (rows > 0 && rows <= 128 && chunks >= std::max(shortest, 140 * rows)) {
     parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
     if (parts < (chunks < 18000 ? kParts : 6)) parts = kParts;
-  } else if ((rows > 256 && rows <= 304 && chunks >= 12288) || (rows > 512 && rows <= 704 && chunks >= 10000)) {
+  } else if ((rows > 256 && rows <= 304 && chunks >= 12288) || (rows > 512 && rows <= (chunks >= 28672 ? 704 : 600) && chunks >= 10000)) {
     parts = kParts;
   }
   if (parts == 1) return 1;
@@ -421,11 +423,16 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
   }
   int threads = (int)std::min<int64_t>(1024, std::max<int64_t>(64, ((cols / per_chunk / 4 + 63) / 64) * 64));
   const dim3 grid((unsigned)rows);
-  // Launches of about one and a half to three workgroups per CU (the 256 CUs of this GPU; a decode batch of a few
-  // hundred rows) keep their waves in step, a chunk at a time: the two workgroups of a CU then finish together with
-  // little left to do, 5 % faster at 384 and 512 rows.  With fewer rows a wave needs four chunks in flight to cover
-  // the latency, with more the generations of workgroups overlap by themselves (measured 16 to 4096 rows).
-  const bool lockstep = rows > 256 && rows <= 768;
+  // Two workgroups on a CU (its 2048 lanes hold no third) keep their waves in step, a chunk at a time: they then finish
+  // together with little left to do.  A row of one batch (four chunks for each of 1024 lanes) only loses by asking for one chunk
+  // at a time, so do rows of about two batches when nearly every CU has two workgroups, and beyond 512 rows a workgroup that
+  // ends early lets the next one begin, which steps prevent.  Us per call in a graph, in step / not, rows x bf16 columns: 257 x
+  // 16000 4.0 / 3.4, 512 x 16000 5.1 / 4.4, 512 x 32000 7.0 / 6.7; 400 x 40000 7.3 / 7.5, 384 x 57344 9.0 / 9.2, 304 x 65536 9.3 /
+  // 9.6, 304 x 80000 10.8 / 11.6, 400 x 98304 13.9 / 14.5, 400 x 128256 17.7 / 18.2, 512 x 262144 41.0 / 45.4; 450 x 65536 11.1 /
+  // 10.9, 512 x 65536 12.5 / 12.0; 600 x 32000 9.7 / 8.3, 600 x 65536 17.9 / 14.6, 704 x 128256 32.5 / 28.8, 768 x 151936 39.5 /
+  // 36.8, of 768 x 262144 alone 64.6 / 66.1; fp32 400 x 16000 5.9 / 5.8, 400 x 24000 7.7 / 8.0, 768 x 128256 62.8 / 59.9.
+  const int chunks = cols / per_chunk;
+  const bool lockstep = rows > 256 && rows <= 512 && chunks > 4096 && !(rows > 420 && chunks >= 6000 && chunks <= 8192);
   const ArgmaxParams p = {out, (const char *)logits, stride_bytes, max_index, cols, threads, cols, 1, 0, nullptr};
 #define ARCTIC_ARGMAX_KERNEL(...) launch(row_argmax_kernel<__VA_ARGS__>, grid, threads, s, p)
 #define ARCTIC_ARGMAX_LAUNCH(ELEM)                                                       \

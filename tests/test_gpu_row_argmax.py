@@ -199,7 +199,8 @@ def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
     (128, 72000, torch.float32, 1), (129, 144512, torch.bfloat16, 0), (9, 40959, torch.float32, 0),   # the most rows that leave CUs idle; fp32
     (256, 98304, torch.bfloat16, 0), (257, 98304, torch.bfloat16, 0), (304, 98304, torch.float16, 0), (305, 98304, torch.float16, 0),
     (257, 98304, torch.bfloat16, 3),   # not aligned: not split
-    (512, 80000, torch.bfloat16, 0), (513, 80000, torch.bfloat16, 0), (704, 80000, torch.bfloat16, 0), (705, 80000, torch.float16, 0)])
+    (512, 80000, torch.bfloat16, 0), (513, 80000, torch.bfloat16, 0), (600, 80000, torch.bfloat16, 0), (601, 80000, torch.float16, 0),
+    (704, 80000, torch.bfloat16, 0), (705, 80000, torch.float16, 0)])
 def test_row_counts_where_the_split_begins_and_ends(ops, rows, cols, dtype, pad):
     """The winner in every eighth of a row, the cuts and both ends, ties of the first and the last place."""
     x = torch.randint(-3, 2, (rows, cols + pad), generator=torch.Generator().manual_seed(rows), dtype=torch.int8).to(dtype)
@@ -210,6 +211,23 @@ def test_row_counts_where_the_split_begins_and_ends(ops, rows, cols, dtype, pad)
             x[r, cols - 1] = 4.0
     for _ in range(2):
         assert torch.equal(ops.speculator_argmax(x.to(DEV)[:, :cols], cols).cpu(), reference(x[:, :cols], cols))
+
+
+@pytest.mark.parametrize("rows,cols,dtype,pad", [
+    (256, 40000, torch.bfloat16, 0), (257, 32775, torch.float16, 0), (257, 32776, torch.float16, 0), (300, 32783, torch.bfloat16, 2),
+    (420, 65536, torch.bfloat16, 0), (421, 65543, torch.bfloat16, 0), (421, 65544, torch.bfloat16, 3), (512, 48000, torch.float16, 0),
+    (512, 47999, torch.float16, 0), (513, 48000, torch.bfloat16, 1), (512, 16387, torch.float32, 0), (512, 16388, torch.float32, 0),
+    (300, 20483, torch.float32, 2)])
+def test_where_waves_keep_in_step_and_where_not(ops, rows, cols, dtype, pad):
+    """The winner at a row's ends and about the ends of its batches of one and of four chunks for each of 1024 lanes."""
+    x = torch.randint(-3, 2, (rows, cols + pad), generator=torch.Generator().manual_seed(cols), dtype=torch.int8).to(dtype)
+    batch = 1024 * (4 if dtype is torch.float32 else 8)
+    places = [0, cols - 1, *(min(cols - 1, batch * k + d) for k in range(1, 9) for d in (-1, 0, 7))]
+    for r in range(0, rows, 2):
+        x[r, places[r // 2 % len(places)]] = 4.0
+        if r % 3 == 0:
+            x[r, cols - 1] = 4.0
+    assert torch.equal(ops.speculator_argmax(x.to(DEV)[:, :cols], cols).cpu(), reference(x[:, :cols], cols))
 
 
 def test_split_rows_on_two_streams_at_once(ops):
