@@ -331,11 +331,14 @@ using namespace arctic;
 // How many workgroups share a row (1: not split), and the elements of each one's segment.  The exchange costs about
 // a microsecond (store, acknowledgement, read), so a row is split where that buys more (us per call in a graph, not split /
 // split, rows x bf16 columns):
-//  - up to 128 rows, which leave CUs idle: the more rows the longer they have to be (1 x 65536 4.21 / 3.95, 20 x 65536 5.16 /
-//    4.65, 41 x 65536 5.23 / 5.06, 64 x 65536 5.45 / 5.56; 64 x 80000 6.26 / 5.76, 70 x 80000 6.34 / 5.86; 86 x 128256 8.23 /
-//    7.48, 112 x 128256 8.62 / 8.45, 128 x 128256 2 % slower; 96 x 151936 9.48 / 8.74, 128 x 262144 9 % faster; 32000 and
-//    50257 columns between 8 % slower and 3 % faster; fp32, whose chunks are half as much work, 1 x 32768 3.74 / 4.22, 7 x 40000
-//    4.02 / 4.43);
+//  - up to 128 rows, which leave CUs idle: the more rows the longer they have to be, from 85 on 180 chunks of 16 bytes for each
+//    row but 5100.  Eight segments against one, in per cent, aligned rows / others: bf16 74 rows of 10240 chunks -9 / -4, 80 of
+//    11000 -5 / -4, 85 of 12000 -4 / -4, 96 of 12000 -3 / -1, of 11000 -2 / -1, 100 of 13500 -10 / -5, of 12000 +1 / +3, 112 of
+//    15500 -7 / -5, of 12500 -1 / +3, 128 of 17500 -4 / -2, of 18992 +1 / -3, of 12500 +2 / +4; fp32 74 of 10240 -5 / -2, 85 of
+//    12000 -1 / -3, 96 of 12500 -6 / -4, of 11000 +2 / 0, 112 of 15500 -5 / -4, of 18992 +2 / -5, 128 of 19500 -2 / -2, of 14000
+//    +3 / 0.  Up to 48 rows of 16-bit logits from 8192 chunks on (20 of 8192 -15 / -15, 41 -7 / +2, 48 -6 / +2, 64 -2 / +3); fp32
+//    rows, whose chunks are half as much work, from 10240 (1 of 8192 3.74 us / 4.22 where the L2 holds the inputs, from HBM 4.34
+//    / 3.88);
 //  - up to a fifth more than one or two rows for every CU, where some CUs would do twice or half as much again as the others
 //    (264 x 128256 16.3 / 14.2, 304 x 128256 17.1 / 15.7, 288 x 151936 19.1 / 18.0, 257 x 80000 10.2 / 10.4, 320 x 100000 6 %
 //    faster to 320 x 80000 1 % slower; 513 x 80000 16.1 / 15.9, 560 x 80000 17.4 / 16.7, 600 x 80000 17.5 / 17.7, 513 x 128256
@@ -351,7 +354,7 @@ static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
   const int64_t chunks = dtype == ARCTIC_DTYPE_F32 ? cols / 4 : cols / 8;
   int64_t parts = 1;
   const int64_t shortest = dtype == ARCTIC_DTYPE_F32 ? 10240 : rows <= 48 ? 8192 : 10000;
-  if (rows > 0 && rows <= 128 && chunks >= std::max(shortest, 140 * rows)) {
+  if (rows > 0 && rows <= 128 && chunks >= std::max(shortest, 180 * rows - 5100)) {
     parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
     if (parts < (chunks < 18000 ? kParts : 6)) parts = kParts;
   } else if ((rows > 256 && rows <= 304 && chunks >= 12288) || (rows > 512 && rows <= (chunks >= 28672 ? 704 : 600) && chunks >= 10000)) {

@@ -1,0 +1,21 @@
+"""Into how many segments a row of logits is cut: arctic_argmax_workspace_bytes holds 16 bytes for each, and makes no HIP
+call.  On both sides of every line the rule draws."""
+import pytest
+
+from arcticinference_amd import _native
+
+BF16, F32 = _native.DTYPE_BF16, _native.DTYPE_F32
+CHUNK = {BF16: 8, F32: 4}   # elements of 16 bytes
+
+
+def parts(rows, chunks, dtype):
+    return _native.load().arctic_argmax_workspace_bytes(rows, chunks * CHUNK[dtype], dtype) // (16 * rows)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("rows,chunks,segments", [
+    (1, 10240, 10), (1, 10239, {BF16: 9, F32: 0}), (48, 8192, {BF16: 8, F32: 0}), (49, 9999, 0), (49, 10000, {BF16: 9, F32: 0}),
+    (74, 10240, 8), (80, 11000, 8), (85, 11250, 8), (85, 10240, 8), (85, 18000, 6),   # 180 chunks for each row but 5100
+    (86, 10379, 0), (86, 10380, 8), (128, 17939, 0), (128, 17940, 8), (129, 40000, 0)])
+def test_rows_that_leave_cus_idle(rows, chunks, segments, dtype):
+    assert parts(rows, chunks, dtype) == (segments[dtype] if isinstance(segments, dict) else segments)
