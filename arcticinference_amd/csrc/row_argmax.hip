@@ -329,8 +329,8 @@ __global__ __launch_bounds__(kSplitLanes) void row_argmax_split_kernel(const Arg
 using namespace arctic;
 
 // How many workgroups share a row (1: not split), and the elements of each one's segment.  The exchange costs about
-// a microsecond (store, acknowledgement, read), so a row is split where that buys more (us per call in a graph, not split /
-// split, rows x bf16 columns):
+// a microsecond (store, acknowledgement, read), so a row is split where that buys more (calls in graphs, both sides in turn,
+// their inputs one after the other out of 800 MB and more, of the smallest 96 sets):
 //  - up to 128 rows, which leave CUs idle: the more rows the longer they have to be, from 85 on 180 chunks of 16 bytes for each
 //    row but 5100.  Eight segments against one, in per cent, aligned rows / others: bf16 74 rows of 10240 chunks -9 / -4, 80 of
 //    11000 -5 / -4, 85 of 12000 -4 / -4, 96 of 12000 -3 / -1, of 11000 -2 / -1, 100 of 13500 -10 / -5, of 12000 +1 / +3, 112 of
@@ -339,11 +339,13 @@ using namespace arctic;
 //    +3 / 0.  Up to 48 rows of 16-bit logits from 8192 chunks on (20 of 8192 -15 / -15, 41 -7 / +2, 48 -6 / +2, 64 -2 / +3); fp32
 //    rows, whose chunks are half as much work, from 10240 (1 of 8192 3.74 us / 4.22 where the L2 holds the inputs, from HBM 4.34
 //    / 3.88);
-//  - up to a fifth more than one or two rows for every CU, where some CUs would do twice or half as much again as the others
-//    (264 x 128256 16.3 / 14.2, 304 x 128256 17.1 / 15.7, 288 x 151936 19.1 / 18.0, 257 x 80000 10.2 / 10.4, 320 x 100000 6 %
-//    faster to 320 x 80000 1 % slower; 513 x 80000 16.1 / 15.9, 560 x 80000 17.4 / 16.7, 600 x 80000 17.5 / 17.7, 513 x 128256
-//    24.6 / 23.3, 600 x 128256 26.5 / 26.4, 640 x 128256 27.2 / 27.6, 704 x 128256 28.8 / 30.4, but 513 x 262144 51.0 / 44.6, 704 x 262144
-//    60.5 / 58.2).
+//  - a few more rows than one or two for every CU, where some CUs would do twice or half as much again as the others: up to 304
+//    from 12288 chunks on (bf16, per cent against one workgroup per row: 257 rows of 12288 -6, of 18992 -2, of 24576 -9, of 10000
+//    -1, 288 of 12288 -4, 304 of 12288 -2, of 18992 0, of 24576 -4, 320 of 12288 0, of 18992 +2), fp32 beyond 288 rows from 24576
+//    (257 of 12288 -1, 288 0, 296 +1, 304 +2, of 18992 +2, of 24576 -2, of 32768 -3); up to 600 from 10000 (bf16 513 of 10000 -6, 600
+//    of 10000 0, of 10500 -5, of 16032 -2, 616 of 10000 +1; fp32 513 of 10000 -3, 600 of 10000 -1, of 16032 0); up to 704 from 28672,
+//    of which the upper half is level (bf16 640 of 28672 -2, of 32768 -6, 704 of 28672 +2, of 32768 -2, of 40960 +2, of 65536 -2; fp32
+//    640 of 30720 -2, 704 of 28672 +1, of 32768 -1, of 40960 +4, of 65536 -3).
 //    Only where every row starts on a 16-byte boundary: 264 x 128257 gains 1 %, 320 loses 4 %.
 // Up to sixteen segments of 1024 chunks or more while they make no more than two workgroups per CU (7 x 128256: 32 segments 4.7
 // us, 16 4.4), and not fewer than eight, of very long rows six (85 x 128256 six 7.93, eight 7.47, sixteen 8.08; 78 x 262144 six
@@ -357,7 +359,8 @@ static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
   if (rows > 0 && rows <= 128 && chunks >= std::max(shortest, 180 * rows - 5100)) {
     parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
     if (parts < (chunks < 18000 ? kParts : 6)) parts = kParts;
-  } else if ((rows > 256 && rows <= 304 && chunks >= 12288) || (rows > 512 && rows <= (chunks >= 28672 ? 704 : 600) && chunks >= 10000)) {
+  } else if ((rows > 256 && rows <= 304 && chunks >= (dtype == ARCTIC_DTYPE_F32 && rows > 288 ? 24576 : 12288)) ||
+             (rows > 512 && rows <= (chunks >= 28672 ? 704 : 600) && chunks >= 10000)) {
     parts = kParts;
   }
   if (parts == 1) return 1;

@@ -19,3 +19,12 @@ def parts(rows, chunks, dtype):
     (86, 10379, 0), (86, 10380, 8), (128, 17939, 0), (128, 17940, 8), (129, 40000, 0)])
 def test_rows_that_leave_cus_idle(rows, chunks, segments, dtype):
     assert parts(rows, chunks, dtype) == (segments[dtype] if isinstance(segments, dict) else segments)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("rows,chunks,segments", [
+    (256, 40000, 0), (257, 12287, 0), (257, 12288, 8), (288, 12288, 8), (289, 12288, {BF16: 8, F32: 0}), (304, 24575, {BF16: 8, F32: 0}),
+    (304, 24576, 8), (305, 40000, 0), (512, 40000, 0), (513, 9999, 0), (513, 10000, 8), (600, 10000, 8), (601, 28671, 0), (601, 28672, 8),
+    (704, 28672, 8), (705, 40000, 0)])
+def test_a_few_more_rows_than_cus(rows, chunks, segments, dtype):
+    assert parts(rows, chunks, dtype) == (segments[dtype] if isinstance(segments, dict) else segments)
