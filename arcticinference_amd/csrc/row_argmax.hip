@@ -431,14 +431,12 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
   const dim3 grid((unsigned)rows);
   // Two workgroups on a CU (its 2048 lanes hold no third) keep their waves in step, a chunk at a time: they then finish
   // together with little left to do.  A row of one batch (four chunks for each of 1024 lanes) only loses by asking for one chunk
-  // at a time, so do rows of about two batches when nearly every CU has two workgroups, and beyond 512 rows a workgroup that
-  // ends early lets the next one begin, which steps prevent.  Us per call in a graph, in step / not, rows x bf16 columns: 257 x
-  // 16000 4.0 / 3.4, 512 x 16000 5.1 / 4.4, 512 x 32000 7.0 / 6.7; 400 x 40000 7.3 / 7.5, 384 x 57344 9.0 / 9.2, 304 x 65536 9.3 /
-  // 9.6, 304 x 80000 10.8 / 11.6, 400 x 98304 13.9 / 14.5, 400 x 128256 17.7 / 18.2, 512 x 262144 41.0 / 45.4; 450 x 65536 11.1 /
-  // 10.9, 512 x 65536 12.5 / 12.0; 600 x 32000 9.7 / 8.3, 600 x 65536 17.9 / 14.6, 704 x 128256 32.5 / 28.8, 768 x 151936 39.5 /
-  // 36.8, of 768 x 262144 alone 64.6 / 66.1; fp32 400 x 16000 5.9 / 5.8, 400 x 24000 7.7 / 8.0, 768 x 128256 62.8 / 59.9.
-  const int chunks = cols / per_chunk;
-  const bool lockstep = rows > 256 && rows <= 512 && chunks > 4096 && !(rows > 420 && chunks >= 6000 && chunks <= 8192);
+  // at a time, and beyond 512 rows a workgroup that ends early lets the next one begin, which steps prevent.  In step against
+  // not, per cent per call in a graph (inputs as above), lowest and highest of bf16 and fp32 rows, aligned and not: 257 to 512 rows
+  // of 2000 chunks of 16 bytes +7 and +20, of 4097 -5 and +3, of 4500 -7 and +1, of 5000 -11 and -3, of 6000 to 6500 -9 and +2, of
+  // 7000 to 8192 -10 and +2 (420 to 512 rows -3 and +2), of 9000 -12 and -2, of 16032 -12 and 0, of 32768 -18 and -6; 513 to 704
+  // rows of up to 28672 chunks +3 and +22; 768 rows +1 and +14, of 32768 chunks alone -5 and -2 (of 30720 and 36000 0 and +4).
+  const bool lockstep = rows > 256 && rows <= 512 && cols / per_chunk > 4096;
   const ArgmaxParams p = {out, (const char *)logits, stride_bytes, max_index, cols, threads, cols, 1, 0, nullptr};
 #define ARCTIC_ARGMAX_KERNEL(...) launch(row_argmax_kernel<__VA_ARGS__>, grid, threads, s, p)
 #define ARCTIC_ARGMAX_LAUNCH(ELEM)                                                       \
