@@ -39,6 +39,7 @@ EXPORTED_SYMBOLS = (
     "arctic_argmax_clamp",
     "arctic_argmax_clamp_split",
     "arctic_argmax_workspace_bytes",
+    "arctic_argmax_workspace_bytes_at",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -120,6 +121,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.arctic_argmax_clamp_split.restype = i32
     lib.arctic_argmax_workspace_bytes.argtypes = [i64, i32, i32]
     lib.arctic_argmax_workspace_bytes.restype = i64
+    lib.arctic_argmax_workspace_bytes_at.argtypes = [vp, i64, i32, i64, i32]
+    lib.arctic_argmax_workspace_bytes_at.restype = i64
 
 
 def load() -> ctypes.CDLL:

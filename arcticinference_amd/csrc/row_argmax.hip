@@ -346,11 +346,12 @@ using namespace arctic;
 //    of 10000 0, of 10500 -5, of 16032 -2, 616 of 10000 +1; fp32 513 of 10000 -3, 600 of 10000 -1, of 16032 0); up to 704 from 28672,
 //    of which the upper half is level (bf16 640 of 28672 -2, of 32768 -6, 704 of 28672 +2, of 32768 -2, of 40960 +2, of 65536 -2; fp32
 //    640 of 30720 -2, 704 of 28672 +1, of 32768 -1, of 40960 +4, of 65536 -3).
-//    Only where every row starts on a 16-byte boundary: 264 x 128257 gains 1 %, 320 loses 4 %.
+//    Only where every row starts on a 16-byte boundary: others lose up to a quarter below 14000 chunks (257 x 80001 +18, 272 x
+//    98305 +9, 513 x 80001 +19) and are level about 16032 (257 rows +4, 272 0, 304 +3, 513 0, 600 +1).
 // Up to sixteen segments of 1024 chunks or more while they make no more than two workgroups per CU (7 x 128256: 32 segments 4.7
 // us, 16 4.4), and not fewer than eight, of very long rows six (85 x 128256 six 7.93, eight 7.47, sixteen 8.08; 78 x 262144 six
 // 10.3, eight 10.8).  Workgroups of 256 and 1024 lanes are 0.1-0.2 us slower.
-static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
+static int argmax_parts(bool aligned_rows, int64_t rows, int cols, int dtype, int *segment) {
   constexpr int64_t kMostParts = 16, kParts = 8, kWorkgroups = 512, kMinChunksPerPart = 1024;
   *segment = cols;
   const int64_t chunks = dtype == ARCTIC_DTYPE_F32 ? cols / 4 : cols / 8;
@@ -359,8 +360,9 @@ static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
   if (rows > 0 && rows <= 128 && chunks >= std::max(shortest, 180 * rows - 5100)) {
     parts = std::min({kMostParts, chunks / kMinChunksPerPart, kWorkgroups / rows});
     if (parts < (chunks < 18000 ? kParts : 6)) parts = kParts;
-  } else if ((rows > 256 && rows <= 304 && chunks >= (dtype == ARCTIC_DTYPE_F32 && rows > 288 ? 24576 : 12288)) ||
-             (rows > 512 && rows <= (chunks >= 28672 ? 704 : 600) && chunks >= 10000)) {
+  } else if (aligned_rows &&
+             ((rows > 256 && rows <= 304 && chunks >= (dtype == ARCTIC_DTYPE_F32 && rows > 288 ? 24576 : 12288)) ||
+              (rows > 512 && rows <= (chunks >= 28672 ? 704 : 600) && chunks >= 10000))) {
     parts = kParts;
   }
   if (parts == 1) return 1;
@@ -368,10 +370,22 @@ static int argmax_parts(int64_t rows, int cols, int dtype, int *segment) {
   return (cols + *segment - 1) / *segment;
 }
 
-extern "C" int64_t arctic_argmax_workspace_bytes(int64_t rows, int cols, int dtype) {
+static bool rows_on_16_bytes(const void *logits, int64_t rows, int64_t row_stride, int dtype) {
+  const uint64_t pitch = (uint64_t)row_stride * (dtype == ARCTIC_DTYPE_F32 ? 4 : 2);
+  return (uintptr_t)logits % 16 == 0 && (pitch % 16 == 0 || rows == 1);
+}
+
+static int64_t argmax_workspace(bool aligned_rows, int64_t rows, int cols, int dtype) {
   int segment;
-  const int parts = argmax_parts(rows, cols, dtype, &segment);
+  const int parts = argmax_parts(aligned_rows, rows, cols, dtype, &segment);
   return parts > 1 ? rows * parts * (int64_t)sizeof(Segment) : 0;
+}
+extern "C" int64_t arctic_argmax_workspace_bytes(int64_t rows, int cols, int dtype) {
+  return argmax_workspace(true, rows, cols, dtype);   // what is split wherever its rows start is split the same aligned
+}
+extern "C" int64_t arctic_argmax_workspace_bytes_at(const void *logits, int64_t rows, int cols, int64_t row_stride, int dtype) {
+  if ((uintptr_t)logits % (dtype == ARCTIC_DTYPE_F32 ? 4 : 2)) return 0;   // element by element, one workgroup per row
+  return argmax_workspace(rows_on_16_bytes(logits, rows, row_stride, dtype), rows, cols, dtype);
 }
 
 // A number per call that no other call has: a 64-bit counter from a seed the system draws, spread by an odd factor.
@@ -401,12 +415,12 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
     return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: more than 2^30 columns, or a row pitch out of range", fn);
   const int64_t stride_bytes = row_stride * es;
   const bool vec = (uintptr_t)logits % es == 0;   // rows may start anywhere between two 16-byte boundaries
-  const bool aligned_rows = (uintptr_t)logits % 16 == 0 && (stride_bytes % 16 == 0 || rows == 1);
+  const bool aligned_rows = rows_on_16_bytes(logits, rows, row_stride, dtype);
   const int per_chunk = 16 / es;
   hipStream_t s = (hipStream_t)stream;
   int segment;
-  const int parts = argmax_parts(rows, cols, dtype, &segment);
-  if (vec && parts > 1 && workspace && (aligned_rows || rows <= 256)) {
+  const int parts = argmax_parts(aligned_rows, rows, cols, dtype, &segment);
+  if (vec && parts > 1 && workspace) {
     if ((uintptr_t)workspace % 8 || workspace_bytes < rows * parts * (int64_t)sizeof(Segment))
       return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: the workspace must be 8-byte aligned and hold %lld bytes", fn,
                   (long long)(rows * parts * (int64_t)sizeof(Segment)));

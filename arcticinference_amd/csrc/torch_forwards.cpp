@@ -566,8 +566,8 @@ at::Tensor argmax_clamp(const at::Tensor &logits, int64_t max_index) {
   const auto shape = logits.sizes().slice(0, logits.dim() - 1);
   const OnDevice device(logits);
   if (rows == 0) return new_empty(shape, at::kLong, logits);
-  // a few long rows are split over workgroups that exchange their winners in memory behind the answers: one allocation
-  const int64_t workspace = arctic_argmax_workspace_bytes(rows, to_int(cols, "cols"), code);
+  // rows that are split over workgroups exchange their winners in memory behind the answers: one allocation
+  const int64_t workspace = arctic_argmax_workspace_bytes_at(in_2d.data_ptr(), rows, to_int(cols, "cols"), in_2d.stride(0), code);
   at::Tensor out = workspace ? new_empty({rows + (workspace + 7) / 8}, at::kLong, logits) : new_empty(shape, at::kLong, logits);
   check_rc(arctic_argmax_clamp_split((int64_t *)out.data_ptr(), in_2d.data_ptr(), rows, (int)cols, in_2d.stride(0), max_index,
                                      code, workspace ? (int64_t *)out.data_ptr() + rows : nullptr, workspace,

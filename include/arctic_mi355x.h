@@ -400,16 +400,21 @@ int arctic_argmax_clamp(int64_t *out, const void *logits, int64_t rows, int cols
                         int64_t row_stride, int64_t max_index, int dtype, void *stream);
 
 /*
- * The same with a workspace of the caller's, which lets a few long rows be split over several workgroups each.
+ * The same with a workspace of the caller's, which lets rows be split over several workgroups each where one per row
+ * would leave part of the GPU idle: few long rows, and a few more rows than one or two for every CU.
  *
  *   workspace        device, 8-byte aligned, of at least arctic_argmax_workspace_bytes(rows, cols, dtype) bytes, which
  *                    this call alone uses until its kernel has run; its contents do not matter and need not be
  *                    cleared.  NULL: rows are not split (what arctic_argmax_clamp does).
  *
- * arctic_argmax_workspace_bytes returns 0 where splitting would not help; it makes no HIP call.
+ * arctic_argmax_workspace_bytes returns 0 where splitting would not help wherever the rows start; what it returns is enough
+ * for logits at any address and pitch.  arctic_argmax_workspace_bytes_at returns what the call for these logits uses, 0
+ * where it does not split them (more than 256 rows are split only where every row starts on a 16-byte boundary).  Neither
+ * makes a HIP call or reads the logits.
  */
 #define ARCTIC_ARGMAX_SEGMENT_BYTES 16
 int64_t arctic_argmax_workspace_bytes(int64_t rows, int cols, int dtype);
+int64_t arctic_argmax_workspace_bytes_at(const void *logits, int64_t rows, int cols, int64_t row_stride, int dtype);
 int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64_t rows, int cols,
                               int64_t row_stride, int64_t max_index, int dtype, void *workspace,
                               int64_t workspace_bytes, void *stream);

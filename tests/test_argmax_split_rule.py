@@ -28,3 +28,16 @@ def test_rows_that_leave_cus_idle(rows, chunks, segments, dtype):
     (704, 28672, 8), (705, 40000, 0)])
 def test_a_few_more_rows_than_cus(rows, chunks, segments, dtype):
     assert parts(rows, chunks, dtype) == (segments[dtype] if isinstance(segments, dict) else segments)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("rows,chunks,anywhere", [(1, 12000, True), (85, 12000, True), (128, 40000, True), (257, 30000, False),
+                                                  (304, 30000, False), (513, 12000, False), (704, 30000, False), (400, 30000, True)])
+def test_rows_that_start_between_16_byte_boundaries_ask_for_no_more_than_they_use(rows, chunks, anywhere, dtype):
+    lib, cols, size = _native.load(), chunks * CHUNK[dtype], 16 // CHUNK[dtype]
+    at = lambda address, pitch: lib.arctic_argmax_workspace_bytes_at(address, rows, cols, pitch, dtype)
+    most = lib.arctic_argmax_workspace_bytes(rows, cols, dtype)
+    assert at(4096, cols) == at(4096, cols + 8) == most
+    assert at(4096 + size, cols) == (most if anywhere else 0)
+    assert at(4096, cols + 1) == (most if anywhere or rows == 1 else 0)
+    assert at(4096 + 1, cols) == 0   # no element boundary: one workgroup per row, element by element

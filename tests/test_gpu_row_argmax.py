@@ -264,6 +264,16 @@ def test_the_result_is_the_answers_alone(ops, shape, tmp_path):
     assert torch.equal(got[:want.numel()].cpu(), want.flatten()) and torch.equal(grown[:want.numel()].cpu(), want.flatten())
 
 
+def test_rows_that_are_not_split_hold_no_memory_for_it(ops):
+    """300 rows that start between 16-byte boundaries get a workgroup each, and their answers a block of their own size."""
+    for pad, least, most in ((1, 0, 4096), (0, 300 * 8 * 16, 1 << 20)):
+        logits = torch.zeros(300, 98304 + pad, dtype=torch.bfloat16, device=DEV)
+        ops.speculator_argmax(logits[:, :98304], 98304)
+        before = torch.cuda.memory_allocated()
+        got = ops.speculator_argmax(logits[:, :98304], 98304)
+        assert least <= torch.cuda.memory_allocated() - before <= most and int(got.max()) == 0
+
+
 def test_no_rows_of_any_width(ops):
     got = ops.speculator_argmax(torch.empty(0, 2 ** 31 + 8, device=DEV, dtype=torch.bfloat16), 7)
     assert got.shape == (0,) and got.dtype == torch.int64
