@@ -223,7 +223,8 @@ __device__ __forceinline__ void select_leftover_rows(const BulkSelectParams &p, 
 // moves up to five batches), 512 x 2 (launches of more than 8192 tokens that select rows as well) and 256 x 4 (everything
 // else: up to two batches per workgroup, rounded up to whole layers, and up to five where more than 8192 tokens of rows
 // that are no power of two long select).
-template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, typename Params, typename Tables>
+template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, bool kWholeAhead, typename Params,
+          typename Tables>
 __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, unsigned block) {
   constexpr bool kCopy = std::is_same<Dst, Copy>::value;
   constexpr int kDstElemBytes = kCopy ? Src::kBytes : 1;
@@ -257,7 +258,7 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
     }
   };
   constexpr std::integral_constant<int, 0> kNone;
-  constexpr std::integral_constant<int, kUnroll / 2> kHalf;
+  constexpr std::integral_constant<int, kWholeAhead ? kUnroll : kUnroll / 2> kAhead;
   constexpr std::integral_constant<int, kUnroll> kAll;
   // independent 16-byte loads `from` ... `to` - 1 of a lane's kUnroll; lanes past the end load nothing
   auto load_part = [&](int c, uint4 (&v)[kUnroll], auto from, auto to) {
@@ -282,7 +283,13 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
   // 19.0 / 18.7, 512 x 16 10.2 / 10.0 / 9.9, 64 x 16 3.71 / 3.73 / 3.49; in the 1024-lane shape, all / none, 16384 x 40 762.7 /
   // 763.1 without padding, 695.9 / 687.3 with 10 %, 575 / 548 with 30 %.  Where the index list is scanned
   // the scan stands between the slot and the stores already, and batches are requested whole (half ahead, 448 x 16 of 3 x 96,
-  // copied, 112 selected: 6.5 / 7.0).
+  // copied, 112 selected: 6.5 / 7.0).  By row map half ahead is level (2049 to 16384 tokens, 1476 calls of bf16 and fp32: the
+  // middle one -0.2 %, with 30 % padding -0.4), fp32 sources gain as 16-bit ones do (with 30 % padding -2 %).
+  // kWholeAhead: copies of 10 to 26 MB, which have no scale to wait for and whose workgroups all run side by side.  Their time
+  // rises in steps (of 44 x 1 x 128 bf16 7 % at 18 MB and 28 % at 21), which come earlier with half of the batch ahead.  Us per call, whole / half: 512 x
+  // 40 of 1 x 128 fp32 7.74 / 8.43, 843 x 44 of 1 x 128 bf16 7.13 / 7.78, 506 x 36 of 3 x 96 8.35 / 9.11, 289 x 36 of it 5.53 /
+  // 5.75; of 391 drawn ones without padding half is 1.2 % slower in the mean and 10 % at the most, of 194 with 30 % padding 0.7 %
+  // faster in the mean.
   const int64_t slot = p.slot_mapping[token];
   int64_t out_row = -1;
   if constexpr (kSelect == kSelectByRowMap) out_row = p.row_map[token];
@@ -311,10 +318,10 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
   if constexpr (kSelect == kSelectByScan) {
     load_part(c, cur, kNone, kAll);
   } else {
-    load_part(c, cur, kNone, kHalf);
+    load_part(c, cur, kNone, kAhead);
     __builtin_amdgcn_sched_barrier(0);   // ahead of the wait for the slot
     if (!to_cache && !to_out) return;
-    load_part(c, cur, kHalf, kAll);
+    load_part(c, cur, kAhead, kAll);
   }
   int nhits = 0;
   if constexpr (kSelect == kSelectByScan) {
@@ -401,10 +408,10 @@ __device__ __forceinline__ void bulk_item(const Params &p, const Tables &tab, un
   }
 }
 
-template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, int kLayers>
+template <typename Src, typename Dst, bool kPow2, int kBulkThreads, int kUnroll, int kSelect, int kLayers, bool kWholeAhead>
 __global__ __launch_bounds__(kBulkThreads) void kv_write_bulk_kernel(const BulkParamsOf<kSelect> p,
                                                                          const LayerTables<kLayers> tab) {
-  bulk_item<Src, Dst, kPow2, kBulkThreads, kUnroll, kSelect>(p, tab, blockIdx.x);
+  bulk_item<Src, Dst, kPow2, kBulkThreads, kUnroll, kSelect, kWholeAhead>(p, tab, blockIdx.x);
 }
 
 // Fallback for shapes or addresses that do not allow 16-byte accesses: one
@@ -527,38 +534,53 @@ struct LayerPointers {
 
 template <typename Src, typename Dst, int kSelect>
 static void launch_vec_shape(const BulkSelectParams &p, const LayerPointers &layers, int64_t grid, bool wide,
-                             hipStream_t s) {
+                             bool whole_ahead, hipStream_t s) {
   const dim3 g((unsigned)grid);
-#define ARCTIC_BULK_LAUNCH(POW2, LANES, UNROLL, LAYERS)                                                             \
+#define ARCTIC_BULK_LAUNCH(POW2, LANES, UNROLL, LAYERS, WHOLE_AHEAD)                                                \
   do {                                                                                                             \
     LayerTables<LAYERS> tab;                                                                                       \
     layers.fill(tab, p.num_layers);                                                                                \
-    launch<BulkParamsOf<kSelect>>(kv_write_bulk_kernel<Src, Dst, POW2, LANES, UNROLL, kSelect, LAYERS>, g, LANES, s, p, tab); \
+    launch<BulkParamsOf<kSelect>>(kv_write_bulk_kernel<Src, Dst, POW2, LANES, UNROLL, kSelect, LAYERS, WHOLE_AHEAD>, g, LANES, \
+                                  s, p, tab);                                                                      \
   } while (0)
   if constexpr (kSelect == kSelectNone) {
     // The 256-lane shape is also that of the small launches, which cost what it takes to issue them: few layers leave
     // 1.5 KB of their arguments out.
     const bool few = p.num_layers <= kFewLayers;
-    if (p.chunk_shift < 0 && wide) ARCTIC_BULK_LAUNCH(false, 1024, 1, kLayersPerLaunch);
-    else if (p.chunk_shift < 0 && few) ARCTIC_BULK_LAUNCH(false, 256, 4, kFewLayers);
-    else if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch);
-    else if (wide) ARCTIC_BULK_LAUNCH(true, 1024, 1, kLayersPerLaunch);   // 0.5-2 % faster than the same batch as 512 x 2
-    else if (few) ARCTIC_BULK_LAUNCH(true, 256, 4, kFewLayers);
-    else ARCTIC_BULK_LAUNCH(true, 256, 4, kLayersPerLaunch);
+#define ARCTIC_BULK_LAUNCH_256(WHOLE_AHEAD)                                                               \
+  do {                                                                                                   \
+    if (p.chunk_shift < 0 && few) ARCTIC_BULK_LAUNCH(false, 256, 4, kFewLayers, WHOLE_AHEAD);             \
+    else if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch, WHOLE_AHEAD);         \
+    else if (few) ARCTIC_BULK_LAUNCH(true, 256, 4, kFewLayers, WHOLE_AHEAD);                              \
+    else ARCTIC_BULK_LAUNCH(true, 256, 4, kLayersPerLaunch, WHOLE_AHEAD);                                 \
+  } while (0)
+    if (wide) {
+      if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 1024, 1, kLayersPerLaunch, false);
+      else ARCTIC_BULK_LAUNCH(true, 1024, 1, kLayersPerLaunch, false);   // 0.5-2 % faster than the same batch as 512 x 2
+      return;
+    }
+    if constexpr (std::is_same<Dst, Copy>::value) {
+      if (whole_ahead) {
+        ARCTIC_BULK_LAUNCH_256(true);
+        return;
+      }
+    }
+    ARCTIC_BULK_LAUNCH_256(false);
+#undef ARCTIC_BULK_LAUNCH_256
   } else {
-    if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch);
-    else if (wide) ARCTIC_BULK_LAUNCH(true, 512, 2, kLayersPerLaunch);
-    else ARCTIC_BULK_LAUNCH(true, 256, 4, kLayersPerLaunch);
+    if (p.chunk_shift < 0) ARCTIC_BULK_LAUNCH(false, 256, 4, kLayersPerLaunch, false);
+    else if (wide) ARCTIC_BULK_LAUNCH(true, 512, 2, kLayersPerLaunch, false);
+    else ARCTIC_BULK_LAUNCH(true, 256, 4, kLayersPerLaunch, false);
   }
 #undef ARCTIC_BULK_LAUNCH
 }
 template <typename Src, typename Dst>
 static void launch_vec(const BulkSelectParams &p, const LayerPointers &layers, int64_t grid, bool wide,
-                       hipStream_t s) {
+                       bool whole_ahead, hipStream_t s) {
   switch (p.select_mode) {
-    case kSelectByScan: launch_vec_shape<Src, Dst, kSelectByScan>(p, layers, grid, wide, s); break;
-    case kSelectByRowMap: launch_vec_shape<Src, Dst, kSelectByRowMap>(p, layers, grid, wide, s); break;
-    default: launch_vec_shape<Src, Dst, kSelectNone>(p, layers, grid, wide, s); break;
+    case kSelectByScan: launch_vec_shape<Src, Dst, kSelectByScan>(p, layers, grid, wide, whole_ahead, s); break;
+    case kSelectByRowMap: launch_vec_shape<Src, Dst, kSelectByRowMap>(p, layers, grid, wide, whole_ahead, s); break;
+    default: launch_vec_shape<Src, Dst, kSelectNone>(p, layers, grid, wide, whole_ahead, s); break;
   }
 }
 template <typename SrcElem, typename Dst>
@@ -571,13 +593,13 @@ static void launch_scalar(const BulkSelectParams &p, const LayerPointers &layers
 }
 
 template <typename Dst>
-static void dispatch_src(bool vec, bool wide, int src_dtype, const BulkSelectParams &p,
+static void dispatch_src(bool vec, bool wide, bool whole_ahead, int src_dtype, const BulkSelectParams &p,
                          const LayerPointers &layers, int64_t grid, hipStream_t s) {
   if (vec) {
     switch (src_dtype) {
-      case ARCTIC_DTYPE_BF16: launch_vec<SrcBF16, Dst>(p, layers, grid, wide, s); break;
-      case ARCTIC_DTYPE_F16: launch_vec<SrcF16, Dst>(p, layers, grid, wide, s); break;
-      default: launch_vec<SrcF32, Dst>(p, layers, grid, wide, s); break;
+      case ARCTIC_DTYPE_BF16: launch_vec<SrcBF16, Dst>(p, layers, grid, wide, whole_ahead, s); break;
+      case ARCTIC_DTYPE_F16: launch_vec<SrcF16, Dst>(p, layers, grid, wide, whole_ahead, s); break;
+      default: launch_vec<SrcF32, Dst>(p, layers, grid, wide, whole_ahead, s); break;
     }
   } else {
     if (src_dtype == ARCTIC_DTYPE_F32)
@@ -816,11 +838,15 @@ static int bulk_entry(const char *fn, const void *keys, const void *values, int6
       if (grid > 0x7fffffffLL)
         return fail(ARCTIC_ERR_INVALID_ARGUMENT, "%s: too many tokens (%lld)", fn, (long long)num_tokens);
       if (pass == 0) continue;
+      // Copies of 10 to 26 MB request their whole first batch ahead of the slot (bulk_item has why).  Below, half ahead is level
+      // (padding 0 and 30 %: 8 to 9 MB -0.3 and -2 %), and so it is above (26 to 28 MB +0.4 and -3, 34 to 40 MB 0 and -4).
+      const double source_mb = 2e-6 * num_tokens * count * n * es;
+      const bool whole_ahead = !quant && !select && source_mb >= 10 && source_mb < 26;
 
       switch (kv_cache_dtype) {
-        case ARCTIC_KV_AUTO: dispatch_src<Copy>(vec, wide, src_dtype, p, layers, grid, s); break;
-        case ARCTIC_KV_FP8_E4M3: dispatch_src<E4M3>(vec, wide, src_dtype, p, layers, grid, s); break;
-        default: dispatch_src<E5M2>(vec, wide, src_dtype, p, layers, grid, s); break;
+        case ARCTIC_KV_AUTO: dispatch_src<Copy>(vec, wide, whole_ahead, src_dtype, p, layers, grid, s); break;
+        case ARCTIC_KV_FP8_E4M3: dispatch_src<E4M3>(vec, wide, whole_ahead, src_dtype, p, layers, grid, s); break;
+        default: dispatch_src<E5M2>(vec, wide, whole_ahead, src_dtype, p, layers, grid, s); break;
       }
       const int rc = check_launch(fn);
       if (rc) return rc;

@@ -97,6 +97,17 @@ def test_layers_split_over_workgroups(ops, kv, shape):
     run_both(ops, make_bulk_case(bs=16, NB=shape["T"] // 16 + 2, kv_cache_dtype=kv, seed=29, std=1.5, pad_fraction=0.05, **shape))
 
 
+@pytest.mark.parametrize("shape, megabytes", [
+    (dict(L=16, H=8, D=128), 10), (dict(L=17, H=1, D=128), 10), (dict(L=16, H=3, D=96), 26), (dict(L=40, H=3, D=96), 26)])
+@pytest.mark.parametrize("src_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("beyond", [0, 1])
+def test_copies_that_request_a_whole_batch_ahead(ops, src_dtype, shape, megabytes, beyond):
+    """On both sides of 10 and 26 MB; up to 16 layers and more, rows of a power of two and others."""
+    T = megabytes * 10 ** 6 // (2 * shape["L"] * shape["H"] * shape["D"] * src_dtype.itemsize) + beyond
+    run_both(ops, make_bulk_case(T=T, bs=16, NB=T // 16 + 2, src_dtype=src_dtype, kv_cache_dtype="auto", seed=31, pad_fraction=0.3,
+                                 **shape))
+
+
 def test_all_padding_leaves_cache_untouched(ops):
     case = make_bulk_case(T=16, L=3, H=2, D=64, bs=16, NB=4, kv_cache_dtype="fp8", seed=7)
     case["slot_mapping"].fill_(-1)
