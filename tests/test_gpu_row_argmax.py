@@ -3,6 +3,8 @@ arctic_speculator.py:846-848, 862) against torch itself: exact indices."""
 import pytest
 import torch
 
+from arcticinference_amd import _native
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
@@ -11,6 +13,13 @@ def reference(logits, vocab_size):
     # the reference's expression, on the CPU in fp32 (every 16-bit value is exact in fp32, so the order and
     # the ties are the same)
     return torch.argmax(logits.float().cpu(), dim=-1).clamp_(0, vocab_size - 1)
+
+
+def segments(rows, cols, dtype):
+    """How many segments a row is cut into (1: not split) and a segment's elements, as the library has them."""
+    code = {torch.float32: _native.DTYPE_F32, torch.float16: _native.DTYPE_F16, torch.bfloat16: _native.DTYPE_BF16}[dtype]
+    parts = max(1, _native.load().arctic_argmax_workspace_bytes(rows, cols, code) // (16 * rows))
+    return parts, cols if parts == 1 else -(-cols // parts) + 63 & ~63   # parts of whole 64 elements
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -124,12 +133,13 @@ def test_random_configurations(ops):
         assert torch.equal(got.cpu(), want), f"configuration {it}: {dtype}, {rows} x {cols}, pad {pad}, offset {off}"
 
 
-@pytest.mark.parametrize("rows", [257, 300, 768, 769])   # 257-768 rows take the kernel whose waves move in step
+@pytest.mark.parametrize("rows", [257, 300, 512, 513, 768, 769])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_row_counts_around_the_in_step_kernel(ops, rows, dtype):
-    """Launches of 257 to 768 rows keep the waves of a row in step, a 16-byte chunk at a time, behind a barrier whose
-    trip count has to be the same for every wave whatever the row length: rows shorter than one chunk per lane, rows
-    with a ragged last batch and an element-wise tail, ties everywhere, NaN and infinities, pitched rows."""
+    """Launches of 257 to 512 rows of more than 4096 16-byte chunks (here the longest rows) keep the waves of a row in step, a
+    chunk at a time, behind a barrier whose trip count has to be the same for every wave whatever the row length; shorter rows
+    and more of them do not.  Rows shorter than one chunk per lane, rows with a ragged last batch and an element-wise tail, ties
+    everywhere, NaN and infinities, pitched rows."""
     g = torch.Generator().manual_seed(900 + rows)
     for cols, pad in ((8, 0), (1000, 8), (4100, 0), (8200, 24), (33001, 7)):
         base = (torch.randint(0, 7, (rows, cols + pad), generator=g).float() - 3)
@@ -143,18 +153,19 @@ def test_row_counts_around_the_in_step_kernel(ops, rows, dtype):
         assert torch.equal(got.cpu(), want), f"{rows} x {cols} (+{pad}), {dtype}"
 
 
-@pytest.mark.parametrize("rows,cols,dtype,pad", [
-    (1, 81920, torch.bfloat16, 0), (1, 81919, torch.float16, 0),       # the shortest row that is split, and one below
-    (85, 128257, torch.float16, 0), (86, 128256, torch.bfloat16, 0),   # six workgroups per row, and no longer
-    (5, 131103, torch.bfloat16, 3), (3, 40960, torch.float32, 0), (2, 300001, torch.float32, 1)])
-def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
-    """Long rows of a small batch are cut into segments: single maxima, tied pairs, infinities and NaNs on both sides of
+@pytest.mark.parametrize("rows,cols,dtype,pad,cut", [
+    (1, 81920, torch.bfloat16, 0, 10), (1, 81919, torch.float16, 0, 9),
+    (85, 128257, torch.float16, 0, 8), (86, 128256, torch.bfloat16, 0, 8), (85, 144000, torch.bfloat16, 1, 6),
+    (5, 131103, torch.bfloat16, 3, 16), (3, 40960, torch.float32, 0, 10), (2, 300001, torch.float32, 1, 16),
+    (257, 98304, torch.bfloat16, 0, 8), (260, 49160, torch.float32, 0, 8), (513, 80008, torch.float16, 0, 8)])
+def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad, cut):
+    """Rows are cut into segments (some few, some a few more than one or two for every CU): single maxima, tied pairs, infinities and NaNs on both sides of
     the cuts, in the middle and at the ends, another answer every time, in eager calls whose outputs take the blocks of
     the ones before and in a captured graph whose inputs change between replays (the workspace keeps what the last replay
     left)."""
     g = torch.Generator().manual_seed(cols)
-    parts = min(16, cols * (2 if dtype == torch.float32 else 1) // 8192, 512 // rows)
-    segment = -(-cols // parts) + 63 & ~63
+    parts, segment = segments(rows, cols, dtype)
+    assert parts == cut
     places = [segment, 0, cols - 1, segment - 1, parts // 2 * segment + 17, cols - 2, (parts - 1) * segment]
     at = lambda r, k: places[(r + k) % len(places)]
     levels = torch.tensor([-float("inf"), -2.0, -0.0, 0.0, 1.5])
@@ -193,18 +204,29 @@ def test_rows_split_over_workgroups(ops, rows, cols, dtype, pad):
         assert torch.equal(got.cpu(), reference(x[:, :cols], cols - 1))
 
 
-@pytest.mark.parametrize("rows,cols,dtype,pad", [
-    (48, 65536, torch.bfloat16, 0), (48, 65535, torch.bfloat16, 0), (49, 65536, torch.float16, 0),   # 8192 chunks, and fewer
-    (71, 80000, torch.bfloat16, 0), (72, 80000, torch.bfloat16, 0), (85, 144000, torch.float16, 0),   # 140 chunks for each row; six segments
-    (128, 72000, torch.float32, 1), (129, 144512, torch.bfloat16, 0), (9, 40959, torch.float32, 0),   # the most rows that leave CUs idle; fp32
-    (256, 98304, torch.bfloat16, 0), (257, 98304, torch.bfloat16, 0), (304, 98304, torch.float16, 0), (305, 98304, torch.float16, 0),
-    (257, 98304, torch.bfloat16, 3),   # not aligned: not split
-    (512, 80000, torch.bfloat16, 0), (513, 80000, torch.bfloat16, 0), (600, 80000, torch.bfloat16, 0), (601, 80000, torch.float16, 0),
-    (704, 80000, torch.bfloat16, 0), (705, 80000, torch.float16, 0)])
-def test_row_counts_where_the_split_begins_and_ends(ops, rows, cols, dtype, pad):
-    """The winner in every eighth of a row, the cuts and both ends, ties of the first and the last place."""
+@pytest.mark.parametrize("rows,cols,dtype,pad,split", [
+    (48, 65536, torch.bfloat16, 0, True), (48, 65535, torch.bfloat16, 0, False), (49, 65536, torch.float16, 0, False),   # 8192 chunks
+    (71, 80000, torch.bfloat16, 0, True), (72, 80000, torch.bfloat16, 0, True), (72, 79999, torch.bfloat16, 0, False), (9, 40959, torch.float32, 0, False),    # 10000; fp32
+    (85, 81920, torch.bfloat16, 0, True), (85, 144000, torch.float16, 0, True),           # eight segments, six
+    (86, 83039, torch.bfloat16, 1, False), (86, 83040, torch.bfloat16, 1, True),          # 180 chunks for each row but 5100
+    (128, 71759, torch.float32, 0, False), (128, 72000, torch.float32, 1, True), (129, 144512, torch.bfloat16, 0, False),
+    (256, 98304, torch.bfloat16, 0, False), (257, 98304, torch.bfloat16, 0, True), (304, 98304, torch.float16, 0, True),
+    (305, 98304, torch.float16, 0, False), (288, 49152, torch.float32, 0, True), (289, 49152, torch.float32, 0, False),
+    (289, 98304, torch.float32, 0, True),
+    (257, 98304, torch.bfloat16, 3, True),   # not split where rows start anywhere (the segments are those of aligned ones)
+    (512, 80000, torch.bfloat16, 0, False), (513, 80000, torch.bfloat16, 0, True), (600, 80000, torch.bfloat16, 0, True),
+    (601, 80000, torch.float16, 0, False), (704, 80000, torch.bfloat16, 0, False), (705, 80000, torch.float16, 0, False),
+    (601, 229368, torch.bfloat16, 0, False), (601, 229376, torch.bfloat16, 0, True), (704, 229376, torch.bfloat16, 0, True),
+    (705, 229376, torch.float16, 0, False)])
+def test_row_counts_where_the_split_begins_and_ends(ops, rows, cols, dtype, pad, split):
+    """The winner in every segment of a row (where it is not split, in every eighth), on both sides of the cuts and at both ends,
+    ties of the first and the last place."""
     x = torch.randint(-3, 2, (rows, cols + pad), generator=torch.Generator().manual_seed(rows), dtype=torch.int8).to(dtype)
-    places = [0, cols - 1, *(min(cols - 1, -(-cols // 8) * k + d) for k in range(1, 8) for d in (-1, 0, 63, 64))]
+    parts, segment = segments(rows, cols, dtype)
+    assert (parts > 1) == split
+    if parts == 1:
+        parts, segment = 8, -(-cols // 8)
+    places = [0, cols - 1, *(min(cols - 1, segment * k + d) for k in range(1, parts) for d in (-1, 0, 63, 64))]
     for r in range(0, rows, 2):
         x[r, places[r // 2 % len(places)]] = 4.0
         if r % 3 == 0:
