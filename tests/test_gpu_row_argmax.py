@@ -136,7 +136,7 @@ def test_random_configurations(ops):
 @pytest.mark.parametrize("rows", [257, 300, 512, 513, 768, 769])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_row_counts_around_the_in_step_kernel(ops, rows, dtype):
-    """Launches of 257 to 512 rows of more than 4096 16-byte chunks (here the longest rows) keep the waves of a row in step, a
+    """Launches of 257 to 512 rows of more than 4096 16-byte chunks (here the longest) keep the waves of a row in step, a
     chunk at a time, behind a barrier whose trip count has to be the same for every wave whatever the row length; shorter rows
     and more of them do not.  Rows shorter than one chunk per lane, rows with a ragged last batch and an element-wise tail, ties
     everywhere, NaN and infinities, pitched rows."""
@@ -239,7 +239,8 @@ def test_row_counts_where_the_split_begins_and_ends(ops, rows, cols, dtype, pad,
     (256, 40000, torch.bfloat16, 0), (257, 32775, torch.float16, 0), (257, 32776, torch.float16, 0), (300, 32783, torch.bfloat16, 2),
     (420, 65536, torch.bfloat16, 0), (421, 65543, torch.bfloat16, 0), (421, 65544, torch.bfloat16, 3), (512, 48000, torch.float16, 0),
     (512, 47999, torch.float16, 0), (513, 48000, torch.bfloat16, 1), (512, 16387, torch.float32, 0), (512, 16388, torch.float32, 0),
-    (300, 20483, torch.float32, 2)])
+    (300, 20483, torch.float32, 2), (384, 14400, torch.float32, 0), (384, 14399, torch.float32, 1), (385, 14400, torch.float32, 1),
+    (421, 49592, torch.bfloat16, 0), (421, 49601, torch.float16, 0), (421, 56000, torch.bfloat16, 0), (421, 55992, torch.bfloat16, 0)])
 def test_where_waves_keep_in_step_and_where_not(ops, rows, cols, dtype, pad):
     """The winner at a row's ends and about the ends of its batches of one and of four chunks for each of 1024 lanes."""
     x = torch.randint(-3, 2, (rows, cols + pad), generator=torch.Generator().manual_seed(cols), dtype=torch.int8).to(dtype)
