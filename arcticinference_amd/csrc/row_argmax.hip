@@ -445,17 +445,17 @@ extern "C" int arctic_argmax_clamp_split(int64_t *out, const void *logits, int64
   const dim3 grid((unsigned)rows);
   // Two workgroups on a CU (its 2048 lanes hold no third) keep their waves in step, a chunk at a time: they then finish
   // together with little left to do.  A row of one batch (four chunks for each of 1024 lanes) only loses by asking for one chunk
-  // at a time, so does one of not quite two when nearly every CU has two workgroups, and beyond 512 rows a workgroup that ends
-  // early lets the next one begin, which steps prevent.  In step against not, per cent per call in a graph (inputs as above),
-  // lowest and highest of bf16 and fp32 rows, aligned and not: 257 to 512 rows of 2000 chunks of 16 bytes +7 and +22, of 3000 0 and
-  // +12, of 3600 to 4096 of bf16 and of more than 384 rows -4 and +4, of 270 to 350 fp32 rows of 3600 to 4096 -6 and +1 (mean -3),
-  // of 4097 -5 and +4, of 4500 -7 and +1, of 5000 -11 and -3, of 6000 -9 and 0, of 9000 -12 and -2, of 16032 -12 and 0, of 32768 -18 and -6;
-  // 257 to 420 rows of 7000 to 8192 -10 and +2; 421 to 512 rows, the mean of aligned ones / others, of 6000 -1.9 / -1.2, of 6200
-  // -2.6 / -0.1, of 6282 -0.8 / +1.8, of 6800 -2.1 / -1.3, of 7000 +1.3 / +0.8, of 7300 +1.0 / +3.4, of 7600 +0.3 / +1.2, of 7900 -0.9 /
-  // -0.6, of 8192 +0.6 / -0.6, of 8500 -0.4 / +1.1, of 9000 -3.5 / -3.5; 513 to 704 rows of up to 28672 chunks +3 and +22; 768 rows
-  // +1 and +14, of 32768 chunks alone -5 and -2 (of 30720 and 36000 0 and +4).
+  // at a time, and beyond 512 rows a workgroup that ends early lets the next one begin, which steps prevent.  In step against
+  // not, per cent per call in a graph (inputs as above), lowest and highest of bf16 and fp32 rows, aligned and not: 257 to 512 rows
+  // of 2000 chunks of 16 bytes +7 and +22, of 3000 0 and +12, of 3600 to 4096 of bf16 and of more than 384 rows -4 and +4, of 270 to
+  // 350 fp32 rows of 3600 to 4096 -6 and +1 (mean -3), of 4097 -5 and +4, of 5000 -11 and -3, of 9000 -12 and -2, of 16032 -12 and 0, of
+  // 32768 -18 and -6; 513 to 704 rows of up to 28672 chunks +3 and +22; 768 rows +1 and +14, of 32768 chunks alone -5 and -2 (of
+  // 30720 and 36000 0 and +4).  Where nearly every CU has two workgroups and rows are not quite two batches long it hangs on each
+  // length: of 2400 drawn launches of 421 to 512 rows the mean of aligned rows / others is +0.8 / +0.8 at 4097 to 4300 chunks, -0.4 /
+  // -0.9 to 4700, -3.8 / -2.3 to 6100, -1.9 / -0.6 to 6300, -1.5 / -0.2 to 7100, -0.4 / +0.9 to 7700, -1.2 / +0.2 to 8300, -0.6 / +1.0 to 8700,
+  // -2.8 / -1.9 to 9500, so that only others of 6200 to 8192, which include 50257 columns (+1.8), go without.
   const int chunks = cols / per_chunk;
-  const bool not_quite_two = rows > 420 && chunks >= (aligned_rows ? 7000 : 6200) && chunks <= 8192;
+  const bool not_quite_two = !aligned_rows && rows > 420 && chunks >= 6200 && chunks <= 8192;
   const int shortest = dtype == ARCTIC_DTYPE_F32 && rows <= 384 ? 3600 : 4097;
   const bool lockstep = rows > 256 && rows <= 512 && chunks >= shortest && !not_quite_two;
   const ArgmaxParams p = {out, (const char *)logits, stride_bytes, max_index, cols, threads, cols, 1, 0, nullptr};
